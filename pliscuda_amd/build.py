@@ -7,6 +7,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -26,9 +27,27 @@ def _run(cmd):
     subprocess.run(cmd, check=True)
 
 
+# (species, reactions) bounds the step kernels are instantiated for, smallest
+# fitting one is used: Schlogl-like, A-B-C, Brusselator, <= 8 x 16, general
+VARIANTS = [(1, 4), (3, 4), (5, 8), (8, 16), (64, 128)]
+
+
 def build_lib():
-    srcs = [os.path.join(CSRC, "plis_capi.hip")]
-    _run(["hipcc", *HIP_FLAGS, "-shared", "-o", LIB + ".tmp", *srcs])
+    obj = os.path.join(HERE, "_build")
+    os.makedirs(obj, exist_ok=True)
+    jobs = [("plis_capi", "plis_capi.hip", [])]
+    jobs += [(f"plis_variant_{s}_{r}", "plis_variant.hip", [f"-DPLIS_MS={s}", f"-DPLIS_MR={r}"]) for s, r in VARIANTS]
+
+    def compile_one(job):
+        name, src, defs = job
+        out = os.path.join(obj, name + ".o")
+        _run(["hipcc", *HIP_FLAGS, *defs, "-c", "-o", out, os.path.join(CSRC, src)])
+        return out
+
+    # the largest first: the build lasts as long as it does
+    with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as pool:
+        objs = list(pool.map(compile_one, reversed(jobs)))
+    _run(["hipcc", "--offload-arch=gfx950", "-shared", "-o", LIB + ".tmp", *objs])
     os.replace(LIB + ".tmp", LIB)
 
 

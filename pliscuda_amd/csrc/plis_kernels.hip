@@ -23,8 +23,10 @@
 // 256-byte access.  Blocks are dispatched round-robin over the 8 XCDs, so
 // each XCD walks a contiguous eighth of the tile list (its L2 holds the
 // neighbouring tiles it gathers from).
+#pragma once
 #include <type_traits>
 
+#include "plis_launch.h"
 #include "plis_numerics.h"
 #include "plis_types.h"
 
@@ -650,8 +652,6 @@ constexpr uint32_t decide_threads() { return 256u; }
 // scope: the blocks run on different XCDs); the last block clears the
 // counter for the next step (the next launch is ordered after this
 // kernel).  With one block per realization it decides directly.
-constexpr uint32_t kDecideChunks = 16;
-
 template <int MS>
 __device__ __forceinline__ void reduce_block_partA(double& tp, double& t2, uint32_t& v2, double* s_tp, double* s_t2,
                                                    uint32_t* s_v2) {
@@ -966,7 +966,6 @@ constexpr uint32_t kQueueDefer = kQueue + 1u;  // count bump that sends the tile
 // 10 (a deferred tile whose means are below 10 after all gets the same
 // values from the redo pass's complete sampler).
 constexpr float kPtrsMaybeF = 9.9999f;
-constexpr uint32_t kMaxTileEdges = 1u << 27;   // hop codes hold the entry offset in 27 bits
 
 // Queue append by the whole wavefront (every lane calls it at the same
 // point, qn is wave-uniform): the lanes whose draw is open take consecutive
@@ -1567,7 +1566,7 @@ void phase_b_finish_kernel(KernelArgs a) {
 
 // One block per realization: sum of firings / any negative over the tile
 // partials of phase B, then commit the step or leap back.
-__global__ __launch_bounds__(1024) void commit_kernel(KernelArgs a) {
+static __global__ __launch_bounds__(1024) void commit_kernel(KernelArgs a) {
     const uint32_t r = blockIdx.x;
     if (r >= a.nreal) return;
     const RealInfo ri = ld_ro(a.info + r);
@@ -1708,32 +1707,5 @@ __global__ __launch_bounds__(decide_threads<MS>()) void commit_decide_kernel(Ker
     }
     finalize_A<MS, MR>(a, net_view(a), ri, r, tp, t2, v2, c);
 }
-
-// Explicit instantiations, smallest fitting one is used: Schlogl-like
-// (1 species, <= 4 reactions), <= 3 x 4, <= 5 x 8 (Brusselator), <= 8 x 16
-// and the general case.
-#define PLIS_INST(MS, MR)                                                   \
-    template __global__ void phase_a_kernel<MS, MR, false>(KernelArgs);     \
-    template __global__ void phase_a_kernel<MS, MR, true>(KernelArgs);      \
-    template __global__ void decide_kernel<MS, MR>(KernelArgs);             \
-    template __global__ void commit_decide_kernel<MS, MR>(KernelArgs);      \
-    template __global__ void phase_b_kernel<MS, MR, false, false>(KernelArgs); \
-    template __global__ void phase_b_kernel<MS, MR, false, true>(KernelArgs);
-#define PLIS_INST_EP(MS, MR)                                                \
-    template __global__ void phase_b_kernel<MS, MR, true, false>(KernelArgs); \
-    template __global__ void phase_b_kernel<MS, MR, true, true>(KernelArgs);  \
-    template __global__ void phase_b_redo_kernel<MS, MR, false>(KernelArgs);  \
-    template __global__ void phase_b_redo_kernel<MS, MR, true>(KernelArgs);   \
-    template __global__ void phase_b_finish_kernel<MS, MR, false>(KernelArgs); \
-    template __global__ void phase_b_finish_kernel<MS, MR, true>(KernelArgs);
-PLIS_INST(1, 4)
-PLIS_INST(3, 4)
-PLIS_INST(5, 8)
-PLIS_INST(8, 16)
-PLIS_INST(64, 128)
-PLIS_INST_EP(1, 4)
-PLIS_INST_EP(3, 4)
-PLIS_INST_EP(5, 8)
-PLIS_INST_EP(8, 16)
 
 }  // namespace plis

@@ -343,19 +343,4 @@ __global__ __launch_bounds__(256) void records_kernel(KernelArgs a) {
     }
 }
 
-#define PLIS_INST_L(MS, MR)                                                          \
-    template __global__ void learned_tau_kernel<MS, MR, false, 0>(KernelArgs);      \
-    template __global__ void learned_tau_kernel<MS, MR, false, 1>(KernelArgs);      \
-    template __global__ void learned_tau_kernel<MS, MR, true, 0>(KernelArgs);       \
-    template __global__ void learned_tau_kernel<MS, MR, true, 1>(KernelArgs);       \
-    template __global__ void learned_finish_kernel<MS, MR, false, 0>(KernelArgs);   \
-    template __global__ void learned_finish_kernel<MS, MR, false, 1>(KernelArgs);   \
-    template __global__ void learned_finish_kernel<MS, MR, true, 0>(KernelArgs);    \
-    template __global__ void learned_finish_kernel<MS, MR, true, 1>(KernelArgs);    \
-    template __global__ void records_kernel<MS, MR>(KernelArgs);
-PLIS_INST_L(1, 4)
-PLIS_INST_L(3, 4)
-PLIS_INST_L(5, 8)
-PLIS_INST_L(8, 16)
-
 }  // namespace plis

@@ -355,7 +355,7 @@ struct AdamArgs {
 // (coalesced rows), then the four sums are combined in a fixed order, so the
 // gradient is deterministic.
 constexpr int kAdamParams = 64;
-__global__ __launch_bounds__(256) void mlp_adam_kernel(AdamArgs a) {
+static __global__ __launch_bounds__(256) void mlp_adam_kernel(AdamArgs a) {
     __shared__ float s_g[4][kAdamParams];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int p = blockIdx.x * kAdamParams + lane;
@@ -381,7 +381,7 @@ __global__ __launch_bounds__(256) void mlp_adam_kernel(AdamArgs a) {
 }
 
 // fp32 master -> packed bf16 copies
-__global__ __launch_bounds__(256) void mlp_pack_kernel(const float* w32, __bf16* q) {
+static __global__ __launch_bounds__(256) void mlp_pack_kernel(const float* w32, __bf16* q) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= kQTotal) return;
     float v = 0.f;

@@ -17,6 +17,8 @@ namespace plis {
 
 constexpr int kTile = 64;        // subvolumes per tile (one wavefront)
 constexpr uint32_t kFwdIdMask = (1u << 26) - 1u;  // neighbour id bits of a forward entry
+// forward entries of a tile: the leap pass's hop codes hold an entry's offset in 27 bits
+constexpr uint32_t kMaxTileEdges = 1u << 27;
 constexpr int kMaxS = 64;
 constexpr int kMaxR = 128;
 
