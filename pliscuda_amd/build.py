@@ -35,7 +35,7 @@ VARIANTS = [(1, 4), (3, 4), (5, 8), (8, 16), (64, 128)]
 def build_lib():
     obj = os.path.join(HERE, "_build")
     os.makedirs(obj, exist_ok=True)
-    jobs = [("plis_capi", "plis_capi.hip", [])]
+    jobs = [("plis_capi", "plis_capi.hip", []), ("plis_resident", "plis_resident.hip", [])]
     jobs += [(f"plis_variant_{s}_{r}", "plis_variant.hip", [f"-DPLIS_MS={s}", f"-DPLIS_MR={r}"]) for s, r in VARIANTS]
 
     def compile_one(job):

@@ -19,6 +19,7 @@
 #include "../../include/plis.h"
 #include "plis_launch.h"
 #include "plis_mlp.hip"
+#include "plis_resident.h"
 
 using namespace plis;
 
@@ -100,6 +101,11 @@ struct plis_ctx {
     uint64_t seed = 0;
     uint32_t wpb = 4, blocks = 8;
     int use_graph = 1;
+    // steps of small realizations inside one block each (resident_kernel)
+    bool resident_fits = false;
+    uint32_t res_waves = 0, res_lds = 0;
+    int res_mode = 0;
+    ResidentArgs res{};
     bool edge_parallel = false;  // every realization symmetric, tiles < 2^27 forward entries
     hipEvent_t* split_ev = nullptr;  // profiling: events between the leap pass's kernels
     // captured step sequences of 1, 2, 4, ..., 64 iterations (index log2 n)
@@ -306,6 +312,34 @@ static bool build_network(const plis_network& net, NetHeader& h, std::vector<int
     return true;
 }
 
+// The resident kernel's reaction tables (ResTables).
+struct ResLists {
+    std::vector<int4> rx;
+    std::vector<int2> sp, spe, jp, jpe, hm;
+};
+
+static ResLists res_lists(const NetHeader& h, const std::vector<int32_t>& I) {
+    ResLists l;
+    auto nu = [&](int s, int j) { return I[h.off_nu + s * h.R + j]; };
+    for (int s = 0; s < h.S; ++s) {
+        const int b = (int)l.spe.size();
+        for (int j = 0; j < h.R; ++j)
+            if (nu(s, j)) l.spe.push_back({j, nu(s, j)});
+        l.sp.push_back({b, (int)l.spe.size()});
+        l.hm.push_back({I[h.off_hor + s], I[h.off_mult + s]});
+    }
+    for (int j = 0; j < h.R; ++j) {
+        const int b = (int)l.jpe.size();
+        for (int s = 0; s < h.S; ++s)
+            if (nu(s, j)) l.jpe.push_back({s, nu(s, j)});
+        l.jp.push_back({b, (int)l.jpe.size()});
+        const int32_t *rs = &I[h.off_rs + j * 3], *rr = &I[h.off_rr + j * 3];
+        l.rx.push_back({I[h.off_nrs + j] | (I[h.off_order + j] > 0 ? 256 : 0), rs[0], rs[1], rs[2]});
+        l.rx.push_back({rr[0], rr[1], rr[2], 0});
+    }
+    return l;
+}
+
 static KernelArgs make_args(plis_ctx* c) {
     KernelArgs a{};
     a.net_i = c->d_net_i;
@@ -496,6 +530,59 @@ extern "C" void plis_destroy(plis_ctx* c) {
     delete c;
 }
 
+// Whether every realization of the context is small enough for
+// resident_kernel, and its launch shape.
+static bool resident_fit(plis_ctx* c, const NetHeader& h, const std::vector<double>& D, const ResLists& l,
+                         const std::vector<uint32_t>& frp, bool huge) {
+    uint64_t maxN = 0, nf = 0, ne = 0;
+    for (const auto& ri : c->info) {
+        maxN = std::max<uint64_t>(maxN, ri.N);
+        nf = std::max<uint64_t>(nf, frp[ri.rp_off + ri.N]);
+        ne = std::max<uint64_t>(ne, ri.n_in);
+    }
+    if (huge) return false;
+    // One CU makes a step of N subvolumes in about 5 us + N (2 + 0.84 S deg +
+    // 2.8 R) ns (measured: A-B-C 7.6 us at 64, 15 at 512, 26 at 1,000, 41 at
+    // 1,728; diffusion of one species 21 at 1,728; Brusselator mesh 25 at 512,
+    // 50 at 1,000).  The launch-per-pass step takes about 30 us (47 for the
+    // Brusselator) at these sizes, and 730 us or more in its general
+    // instantiation (cascade of 32 species, 62 reactions: 17 us here at 60
+    // subvolumes, 165 at 1,000).  The line lies where the two meet.
+    double est = 0.0;
+    for (const auto& ri : c->info)
+        est = std::max(est, 1e-3 * (ri.N * (2.0 + 2.8 * h.R) + 0.84 * h.S * (double)ri.n_in));
+    if (est > (c->variant > 3 ? 600.0 : 20.0 + 3.0 * h.S)) return false;
+    // wavefronts: one per item of the widest phase, 4 to 16
+    const uint64_t nt = (maxN + 63) / 64;
+    const uint64_t items = std::max<uint64_t>(nt * std::max(h.S + 1, h.R), (nf + 63) / 64 * ((h.S + 7) / 8) + nt * ((h.R + 3) / 4));
+    c->res_waves = (uint32_t)std::min<uint64_t>(16, std::max<uint64_t>(4, items));
+    const ResidentLds b = resident_lds(c->res_waves, h.S, h.R, h.C, l.spe.size(), maxN, nf, ne);
+    if (b.tables > 64 * 1024) return false;
+    c->res_mode = b.tables + b.arrays + b.topology <= kResidentLdsMax ? 0 : b.tables + b.arrays <= kResidentLdsMax ? 1 : 2;
+    c->res_lds = (uint32_t)(b.tables + (c->res_mode <= 1 ? b.arrays : 0) + (c->res_mode == 0 ? b.topology : 0));
+    c->res.ws_slice = c->res_mode == 2 ? (b.arrays + 255) & ~255ull : 0;
+    c->res.nspe = (uint32_t)l.spe.size();
+    for (int s = 0; s < h.S; ++s)
+        for (int q = 0; q < h.C; ++q)
+            if (D[h.off_d + q * h.S + s] > 0.0) c->res.diffusing |= 1ull << s;
+    return true;
+}
+
+// Plain stepping of a context whose realizations all fit.
+static bool resident(const plis_ctx* c) { return c->resident_fits && !c->learned_on && !(c->theta > 0.0); }
+
+static int resident_iters(plis_ctx* c, uint32_t n) {
+    ResidentArgs a = c->res;
+    a.k = make_args(c);
+    // (a launch makes at most 4,096 iterations, some tens of milliseconds)
+    while (n > 0) {
+        a.iters = std::min(n, 4096u);
+        HIPCHK(c, launch_resident(c->stream, c->nreal, c->res_waves, c->res_lds, c->res_mode, a));
+        n -= a.iters;
+    }
+    return 0;
+}
+
 extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_topology* topos,
                            const uint32_t* const* x0, const uint32_t* ids, const plis_params* params,
                            plis_ctx** out) {
@@ -536,6 +623,8 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
     std::vector<uint32_t> hx, hrp, hcol, hirp, hicol, hfrp;
     std::vector<float> hw, hiw;
     std::vector<uint64_t> hcw, hicw, hfcw;  // interleaved id + weight bits
+    std::vector<uint32_t> hfsrc;
+    std::vector<float> hfrw;
     auto idw = [](uint32_t u, float w) {
         uint32_t b;
         std::memcpy(&b, &w, 4);
@@ -574,12 +663,32 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         any_weighted = any_weighted || weighted;
         hrp.insert(hrp.end(), g.rp.begin(), g.rp.end());
         hcol.insert(hcol.end(), g.col.begin(), g.col.end());
-        // forward CSR: each undirected edge once, in the row of its lower end
+        Csr in;
+        if (!sym) transpose(g, N, in);
+        // forward CSR: each pair of linked subvolumes once, in the row of its
+        // lower end, with the weights of both hops (an asymmetric topology's
+        // may differ, or one of them be absent: weight 0)
         ri.fe_off = hfcw.size();
         for (uint32_t v = 0; v < N; ++v) {
             hfrp.push_back((uint32_t)(hfcw.size() - ri.fe_off));
-            for (uint32_t q = g.rp[v]; q < g.rp[v + 1]; ++q)
-                if (g.col[q] > v) hfcw.push_back(idw((g.col[q] & kFwdIdMask) | ((v % kTile) << 26), g.w[q]));
+            auto put = [&](uint32_t u, float wf, float wr) {
+                hfcw.push_back(idw((u & kFwdIdMask) | ((v % kTile) << 26), wf));
+                hfsrc.push_back(v);
+                hfrw.push_back(wr);
+            };
+            uint32_t q = g.rp[v], qe = g.rp[v + 1];
+            if (sym) {
+                for (; q < qe; ++q)
+                    if (g.col[q] > v) put(g.col[q], g.w[q], g.w[q]);
+                continue;
+            }
+            uint32_t p = in.rp[v], pe = in.rp[v + 1];
+            while (q < qe || p < pe) {  // merge the out-row and the in-row, both ascending
+                const uint32_t uo = q < qe ? g.col[q] : UINT32_MAX, ui = p < pe ? in.col[p] : UINT32_MAX;
+                const uint32_t u = std::min(uo, ui);
+                const float wf = uo == u ? g.w[q++] : 0.0f, wr = ui == u ? in.w[p++] : 0.0f;
+                if (u > v) put(u, wf, wr);
+            }
         }
         hfrp.push_back((uint32_t)(hfcw.size() - ri.fe_off));
         if (N > kFwdIdMask) huge_tile = true;  // ids take 26 bits of a forward entry
@@ -596,8 +705,6 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         hwsum.push_back(0.0);
         if (!sym) {
             any_asym = true;
-            Csr in;
-            transpose(g, N, in);
             ri.ie_off = ieoff;
             ri.irp_off = irpoff;
             hirp.insert(hirp.end(), in.rp.begin(), in.rp.end());
@@ -610,6 +717,7 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
             ri.ie_off = eoff;
             ri.irp_off = rpoff;
         }
+        ri.n_in = (uint32_t)g.col.size();
         if (nh.C > 1) {
             ri.comp_off = coff;
             for (uint32_t v = 0; v < N; ++v) {
@@ -693,11 +801,50 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
     }
     // the forward CSR and the zeroed balances serve the edge-parallel leap
     const bool ep = !any_asym && !huge_tile;
-    if (ep && ((rc = upload(c, &c->d_frp, hfrp)) || (rc = upload(c, &c->d_fcw, hfcw)) ||
-                      (rc = upload(c, &c->d_gdelta, std::vector<unsigned long long>(hx.size(), 0ull))))) {
+    const ResLists lists = res_lists(nh, I);
+    c->resident_fits = resident_fit(c, nh, D, lists, hfrp, huge_tile);
+    if ((ep || c->resident_fits) && ((rc = upload(c, &c->d_frp, hfrp)) || (rc = upload(c, &c->d_fcw, hfcw)))) {
         g_create_err = c->err;
         plis_destroy(c);
         return rc;
+    }
+    if (ep && (rc = upload(c, &c->d_gdelta, std::vector<unsigned long long>(hx.size(), 0ull)))) {
+        g_create_err = c->err;
+        plis_destroy(c);
+        return rc;
+    }
+    if (c->resident_fits) {
+        std::vector<uint4> fwd(hfcw.size());
+        for (size_t e = 0; e < fwd.size(); ++e) {
+            uint32_t back;
+            std::memcpy(&back, &hfrw[e], 4);
+            fwd[e] = {(uint32_t)hfcw[e] & kFwdIdMask, (uint32_t)(hfcw[e] >> 32), hfsrc[e], back};
+        }
+        int4* rx = nullptr;
+        int2 *sp = nullptr, *spe = nullptr, *jp = nullptr, *jpe = nullptr, *hm = nullptr;
+        uint4* fw = nullptr;
+        if ((rc = upload(c, &rx, lists.rx)) || (rc = upload(c, &sp, lists.sp)) || (rc = upload(c, &spe, lists.spe)) ||
+            (rc = upload(c, &jp, lists.jp)) || (rc = upload(c, &jpe, lists.jpe)) || (rc = upload(c, &hm, lists.hm)) ||
+            (rc = upload(c, &fw, fwd)) ||
+            (c->res.ws_slice && (rc = dev_alloc(c, &c->res.ws, c->res.ws_slice * c->nreal)))) {
+            g_create_err = c->err;
+            plis_destroy(c);
+            return rc;
+        }
+        // (one limit for every context: a smaller one set here would take it from another)
+        if (const hipError_t e = resident_reserve(kResidentLdsMax); e != hipSuccess) {
+            g_create_err = std::string("hipFuncSetAttribute(resident_kernel): ") + hipGetErrorString(e);
+            plis_destroy(c);
+            return PLIS_ERR_HIP;
+        }
+        c->res.rx = rx;
+        c->res.sp = sp;
+        c->res.spe = spe;
+        c->res.jp = jp;
+        c->res.jpe = jpe;
+        c->res.hm = hm;
+        c->res.fwd = fw;
+        c->res.count_redo = ep && c->variant <= 3 ? 1u : 0u;
     }
     c->edge_parallel = ep;
     if (hipHostMalloc((void**)&c->h_ndone, sizeof(uint32_t)) != hipSuccess) {
@@ -773,10 +920,11 @@ extern "C" int plis_run_until(plis_ctx* c, double t_end, double t_pause, uint64_
         return p;
     };
     last_progress = progress();
-    if (ndone < c->nreal)
+    const bool res = resident(c);
+    if (ndone < c->nreal && !res)
         if (int rc = prologue(c)) return rc;
     while (ndone < c->nreal) {
-        if (int rc = graph_iters(c, k)) return rc;
+        if (int rc = res ? resident_iters(c, 1024) : graph_iters(c, k)) return rc;
         HIPCHK(c, hipMemcpyAsync(c->h_ndone, d_ndone, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         ndone = *c->h_ndone;
@@ -809,6 +957,7 @@ extern "C" int plis_run(plis_ctx* c, double t_end, uint64_t step_limit) {
 
 extern "C" int plis_iterate(plis_ctx* c, uint32_t n) {
     if (!c) return PLIS_ERR_ARG;
+    if (resident(c)) return resident_iters(c, n);
     if (n > 0)
         if (int rc = prologue(c)) return rc;
     if (int rc = graph_iters(c, n)) return rc;

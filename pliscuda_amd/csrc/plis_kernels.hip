@@ -274,6 +274,33 @@ __device__ __forceinline__ void decide(RealCtl& c) {
     c.tau = tau;
 }
 
+// Destination of a critical hop from v: the edge of v's row at which the
+// weights, summed one edge at a time in CSR order, pass tw.  Run by a whole
+// wavefront, which loads up to 64 edges at once.
+__device__ __forceinline__ uint32_t choose_hop_edge(const KernelArgs& a, const RealInfo& ri, uint32_t v, double tw) {
+    const uint32_t rb = a.rp[ri.rp_off + v], re = a.rp[ri.rp_off + v + 1];
+    const bool weighted = (ri.flags & 2u) != 0;
+    const uint32_t lane = threadIdx.x & 63u;
+    double accw = 0.0;
+    uint32_t dst = v;
+    bool found = false;
+    for (uint32_t q0 = rb; q0 < re && !found; q0 += 64u) {
+        const uint32_t q = q0 + lane;
+        const float wl = q < re ? (weighted ? a.w[ri.e_off + q] : 1.0f) : 0.0f;
+        const uint32_t cl = q < re ? a.col[ri.e_off + q] : v;
+        const uint32_t cnt = min(64u, re - q0);
+        for (uint32_t i = 0; i < cnt; ++i) {
+            accw += (double)__shfl(wl, (int)i);
+            dst = (uint32_t)__shfl((int)cl, (int)i);
+            if (tw < accw) {
+                found = true;
+                break;
+            }
+        }
+    }
+    return dst;
+}
+
 // Critical event at v*: a critical reaction or a critical hop, chosen with
 // probability proportional to its propensity; a hop's edge is chosen in
 // proportion to its weight.  Run by a whole wavefront (every value is
@@ -291,8 +318,6 @@ __device__ void choose_event(const KernelArgs& a, const NetView& n, const RealIn
     double av[MR];
     uint32_t crit[(MR + 31) / 32];
     react_props<MR, MS>(n, x, cc, a.n_critical, av, crit);
-    const uint32_t rb = a.rp[ri.rp_off + v], re = a.rp[ri.rp_off + v + 1];
-    const bool weighted = (ri.flags & 2u) != 0;
     const double W = a.wsum[ri.rp_off + v];
     double a0c = 0.0;
 #pragma unroll
@@ -330,31 +355,7 @@ __device__ void choose_event(const KernelArgs& a, const NetView& n, const RealIn
     if (kind == 0) kind = lastkind;
     c.ev_kind = kind;
     c.ev_idx = idx;
-    c.ev_dst = v;
-    if (kind == 2) {
-        // the wave loads up to 64 edges of v's row at once; the weights are
-        // then summed one edge at a time in CSR order
-        const uint32_t lane = threadIdx.x & 63u;
-        const double tw = uniform01(o.y) * W;
-        double accw = 0.0;
-        uint32_t dst = v;
-        bool found = false;
-        for (uint32_t q0 = rb; q0 < re && !found; q0 += 64u) {
-            const uint32_t q = q0 + lane;
-            const float wl = q < re ? (weighted ? a.w[ri.e_off + q] : 1.0f) : 0.0f;
-            const uint32_t cl = q < re ? a.col[ri.e_off + q] : v;
-            const uint32_t cnt = min(64u, re - q0);
-            for (uint32_t i = 0; i < cnt; ++i) {
-                accw += (double)__shfl(wl, (int)i);
-                dst = (uint32_t)__shfl((int)cl, (int)i);
-                if (tw < accw) {
-                    found = true;
-                    break;
-                }
-            }
-        }
-        c.ev_dst = dst;
-    }
+    c.ev_dst = kind == 2 ? choose_hop_edge(a, ri, v, uniform01(o.y) * W) : v;
 }
 
 // ---------------------------------------------------------------------------
@@ -517,18 +518,65 @@ __device__ __forceinline__ void tau_subvolume(const KernelArgs& a, const NetView
     a0c_out = t.a0c;
 }
 
+// Wavefront reductions on DPP lane shifts (row_shr 1, 2, 4, 8, then the two
+// row broadcasts; lane 63 ends with all 64): an LDS permute per step and word
+// instead takes several times as long, and these sit at the end of every tile.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t identity, uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)identity, (int)x, CTRL, ROWS, 0xF, false);
+}
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned long long dpp_u64(unsigned long long identity, unsigned long long x) {
+    const uint32_t lo = dpp_u32<CTRL, ROWS>((uint32_t)identity, (uint32_t)x);
+    const uint32_t hi = dpp_u32<CTRL, ROWS>((uint32_t)(identity >> 32), (uint32_t)(x >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+template <class F>
+__device__ __forceinline__ unsigned long long wave_fold_u64(unsigned long long identity, unsigned long long x, F f) {
+    x = f(x, dpp_u64<0x111, 0xF>(identity, x));
+    x = f(x, dpp_u64<0x112, 0xF>(identity, x));
+    x = f(x, dpp_u64<0x114, 0xF>(identity, x));
+    x = f(x, dpp_u64<0x118, 0xF>(identity, x));
+    x = f(x, dpp_u64<0x142, 0xA>(identity, x));
+    x = f(x, dpp_u64<0x143, 0xC>(identity, x));
+    return ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), 63) << 32) |
+           (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
+template <class F>
+__device__ __forceinline__ uint32_t wave_fold_u32(uint32_t identity, uint32_t x, F f) {
+    x = f(x, dpp_u32<0x111, 0xF>(identity, x));
+    x = f(x, dpp_u32<0x112, 0xF>(identity, x));
+    x = f(x, dpp_u32<0x114, 0xF>(identity, x));
+    x = f(x, dpp_u32<0x118, 0xF>(identity, x));
+    x = f(x, dpp_u32<0x142, 0xA>(identity, x));
+    x = f(x, dpp_u32<0x143, 0xC>(identity, x));
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
+__device__ __forceinline__ double wave_min(double x) {
+    return __longlong_as_double((long long)wave_fold_u64(
+        (unsigned long long)__double_as_longlong(kInf), (unsigned long long)__double_as_longlong(x),
+        [](unsigned long long p, unsigned long long q) {
+            return (unsigned long long)__double_as_longlong(
+                fmin(__longlong_as_double((long long)p), __longlong_as_double((long long)q)));
+        }));
+}
+
+// (tp, t2, v2) <- min tau', argmin tau'' (lowest subvolume on ties) over the
+// wavefront, in every lane.  Every lane of the wavefront takes part.
 __device__ __forceinline__ void reduce_partA(double& tp, double& t2, uint32_t& v2) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const double otp = __shfl_xor(tp, off);
-        const double ot2 = __shfl_xor(t2, off);
-        const uint32_t ov = (uint32_t)__shfl_xor((int)v2, off);
-        tp = fmin(tp, otp);
-        if (ot2 < t2 || (ot2 == t2 && ov < v2)) {
-            t2 = ot2;
-            v2 = ov;
-        }
+    tp = wave_min(tp);
+    if (__ballot(t2 < kInf) == 0ull) {  // no critical channel: the usual case
+        v2 = wave_fold_u32(0xFFFFFFFFu, v2, [](uint32_t p, uint32_t q) { return min(p, q); });
+        t2 = kInf;
+        return;
     }
+    const double m = wave_min(t2);
+    v2 = wave_fold_u32(0xFFFFFFFFu, t2 == m ? v2 : 0xFFFFFFFFu, [](uint32_t p, uint32_t q) { return min(p, q); });
+    t2 = m;
 }
 
 template <int MS, int MR>
@@ -1364,12 +1412,10 @@ __device__ __forceinline__ void finish_tile(const KernelArgs& a, const NetView& 
 }
 
 __device__ __forceinline__ void reduce_partB(unsigned long long& fire, uint32_t& bad, uint32_t& viol) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        fire += __shfl_xor(fire, off);
-        bad |= (uint32_t)__shfl_xor((int)bad, off);
-        viol += (uint32_t)__shfl_xor((int)viol, off);
-    }
+    fire = wave_fold_u64(0ull, fire, [](unsigned long long p, unsigned long long q) { return p + q; });
+    bad = __ballot(bad != 0u) != 0ull ? 1u : 0u;
+    if (__ballot(viol != 0u) != 0ull)
+        viol = wave_fold_u32(0u, viol, [](uint32_t p, uint32_t q) { return p + q; });
 }
 
 // Commits the step or leaps back, on c: returns true when the step was

@@ -263,7 +263,7 @@ __device__ __attribute__((noinline)) long long poisson_slow(double lam, uint32_t
 // about 6e-5 per comparison) or k > kSqueezeK leaves it to the double search.
 constexpr float kSqueeze = 0x1p-15f;
 constexpr int kSqueezeK = 15;
-__constant__ float kRecipF[kSqueezeK + 1] = {
+constexpr float kRecipF[kSqueezeK + 1] = {
     0.0f,           0x1p+0f,        0x1p-1f,        0x1.555556p-2f, 0x1p-2f,        0x1.99999ap-3f,
     0x1.555556p-3f, 0x1.24924ap-3f, 0x1p-3f,        0x1.c71c72p-4f, 0x1.99999ap-4f, 0x1.745d18p-4f,
     0x1.555556p-4f, 0x1.3b13b2p-4f, 0x1.24924ap-4f, 0x1.111112p-4f};
@@ -291,13 +291,16 @@ __device__ __forceinline__ float fexp_neg(float l) {
 __device__ __forceinline__ int poisson_squeeze(float l, float u) {
     float p = fexp_neg(l);
     float G = p;
-#pragma unroll 1
-    for (int k = 0;; ++k) {
+    // (unrolled: the reciprocals are literals; from a table each trip waited
+    // on a scalar load)
+#pragma unroll
+    for (int k = 0; k <= kSqueezeK; ++k) {
         if (u <= G - kSqueeze) return k;
         if (!(u > G + kSqueeze) || k == kSqueezeK) return -1;
-        p = (p * l) * kRecipF[k + 1];
+        p = (p * l) * kRecipF[k < kSqueezeK ? k + 1 : 0];
         G = G + p;
     }
+    return -1;
 }
 
 // Poisson(lam) from the packed word u0 (inversion) or the draw's PTRS stream.

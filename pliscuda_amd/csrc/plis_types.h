@@ -48,7 +48,7 @@ struct RealInfo {
     uint32_t N, id;
     uint32_t tile_begin, ntiles;
     uint32_t flags;      // bit0: symmetric (in-CSR aliases out-CSR), bit1: weighted
-    uint32_t pad;
+    uint32_t n_in;       // in-edges
 };
 
 enum CtlStatus : int32_t { kRunning = 0, kDone = 1, kAbsorbed = 2, kErrLeapback = -3, kErrOverflow = -4 };
