@@ -135,11 +135,12 @@ int plis_iterate(plis_ctx *ctx, uint32_t n);
 int plis_profile(plis_ctx *ctx, uint32_t n, double *out);
 
 /* As plis_profile, with the leap pass split by kernel: out[0..4] as there,
- * out[5] = phase_b_kernel, out[6] = phase_b_redo_kernel, out[7] =
+ * out[5] = phase_b_kernel, out[6] = 0 (a pass that no longer exists), out[7] =
  * phase_b_finish_kernel (summed ms).  A context with the per-subvolume leap
- * kernel (some topology not symmetric) reports it in out[5] and 0 in
- * out[6..7].  Diagnostics of this implementation; no counterpart in the
- * reference. */
+ * kernel (more than 8 species or 16 reactions) reports it in out[5] and 0 in
+ * out[7].  Small realizations, whose steps run inside one kernel otherwise,
+ * are stepped with a launch per pass here.  Diagnostics of this
+ * implementation; no counterpart in the reference. */
 int plis_profile_kernels(plis_ctx *ctx, uint32_t n, double *out);
 
 int plis_set_state(plis_ctx *ctx, int32_t r, const uint32_t *x);
@@ -166,18 +167,17 @@ int plis_checkpoint_size(plis_ctx *ctx, uint64_t *bytes);
 int plis_checkpoint(plis_ctx *ctx, void *buf, uint64_t bytes);
 int plis_restore(plis_ctx *ctx, const void *buf, uint64_t bytes);
 
-/* Diagnostic (no counterpart in the reference): number of tiles the
- * edge-parallel leap passes of this context have handed to their redo pass
- * since plis_create, i.e. tiles holding a Poisson draw of mean >= 10 or more
- * undecided fast-path draws than the per-wavefront queue holds.  Results do
- * not depend on it. */
+/* Diagnostic (no counterpart in the reference): number of tiles, summed over
+ * the edge-parallel leap passes of this context on symmetric topologies since
+ * plis_create, that held a Poisson draw of mean >= 10 or more than 256 draws
+ * that their coarse byte left undecided.  Results do not depend on it. */
 int plis_redo_tiles(plis_ctx *ctx, uint64_t *total);
 
 /* Diagnostic standing in for the reference's cuda-memcheck initcheck job
  * (PLISCuda/test/run.sh:100-120): fill every device buffer that a step
  * writes before it reads -- each realization's non-current count buffer,
- * the tile partials of the tau and leap passes, the redo list -- with
- * sentinels that are harmless if read but change the trajectory, and forget
+ * the tile partials of the tau and leap passes -- with sentinels
+ * that are harmless if read but change the trajectory, and forget
  * any learned proposals.  A run after it must equal a run without it bit for
  * bit; a kernel that read an unwritten word would break that. */
 int plis_debug_poison(plis_ctx *ctx);

@@ -200,7 +200,7 @@ class Context:
         return list(out)
 
     def profile_kernels(self, n):
-        """profile() plus the leap pass by kernel: [..., phase_b, redo, finish]."""
+        """profile() plus the leap pass by kernel: [..., phase_b, 0, finish]."""
         out = (C.c_double * 8)()
         self._chk(lib().plis_profile_kernels(self.h, n, out), "plis_profile_kernels")
         return list(out)
@@ -234,8 +234,8 @@ class Context:
         self._chk(lib().plis_debug_poison(self.h), "plis_debug_poison")
 
     def redo_tiles(self):
-        """Tiles the edge-parallel leap passes have left to their redo pass
-        since the context was made."""
+        """Tiles with a draw of mean >= 10 or more than 256 undecided draws,
+        summed over the leap passes since the context was made."""
         n = C.c_uint64()
         self._chk(lib().plis_redo_tiles(self.h, C.byref(n)), "plis_redo_tiles")
         return n.value

@@ -81,8 +81,9 @@ struct plis_ctx {
     uint32_t *d_x0 = nullptr, *d_x1 = nullptr;
     uint32_t *d_rp = nullptr, *d_col = nullptr, *d_irp = nullptr, *d_icol = nullptr;
     double* d_wsum = nullptr;  // per subvolume, row_ptr layout
-    uint32_t* d_frp = nullptr;  // forward CSR (symmetric realizations): row pointers
+    uint32_t* d_frp = nullptr;  // forward CSR: row pointers
     uint64_t* d_fcw = nullptr;  // its entries: neighbour id, row's index in its tile, weight
+    float* d_frw = nullptr;     // weights of the hops back, if some topology is not symmetric
     unsigned long long* d_gdelta = nullptr;        // leap balances, counts layout
     float *d_w = nullptr, *d_iw = nullptr;
     uint64_t *d_cw = nullptr, *d_icw = nullptr;  // interleaved id + weight
@@ -93,8 +94,7 @@ struct plis_ctx {
     uint32_t decide_chunks = 1;   // decide_kernel's blocks per realization
     uint32_t* d_dcnt = nullptr;   // decide_kernel's per-realization chunk counters
     PartB* d_pb_t = nullptr;
-    uint32_t* d_cnt = nullptr;   // [0] realizations done, [1] redo-list length, [2..3] redone tiles (u64)
-    uint32_t* d_redo = nullptr;  // redo list of the leap pass (tile ids)
+    uint32_t* d_cnt = nullptr;   // [0] realizations done, [2..3] tiles beyond a wavefront's queue (u64)
     uint32_t* h_ndone = nullptr;  // pinned
     double eps = 0.03;
     int32_t nc = 10;
@@ -106,8 +106,8 @@ struct plis_ctx {
     uint32_t res_waves = 0, res_lds = 0;
     int res_mode = 0;
     ResidentArgs res{};
-    bool edge_parallel = false;  // every realization symmetric, tiles < 2^27 forward entries
-    hipEvent_t* split_ev = nullptr;  // profiling: events between the leap pass's kernels
+    bool edge_parallel = false;  // at most 8 species and 16 reactions, tiles < 2^19 forward entries
+    hipEvent_t* split_ev = nullptr;  // profiling: event between the leap pass's kernels
     // captured step sequences of 1, 2, 4, ..., 64 iterations (index log2 n)
     hipGraphExec_t graphs[kGraphSizes] = {};
     std::vector<void*> allocs;
@@ -370,12 +370,11 @@ static KernelArgs make_args(plis_ctx* c) {
     a.decide_chunks = c->decide_chunks;
     a.partB_tile = c->d_pb_t;
     a.ndone = c->d_cnt;
-    a.redo_count = c->d_cnt + 1;
-    a.redo_tiles = c->d_redo;
     a.frp = c->d_frp;
-
+    a.frw = c->d_frw;
     a.gdelta = c->d_gdelta;
     a.redo_total = reinterpret_cast<unsigned long long*>(c->d_cnt + 2);
+    a.count_redo = c->edge_parallel && !c->d_frw ? 1u : 0u;
     a.epsilon = c->eps;
     a.n_critical = c->nc;
     a.seed_lo = (uint32_t)c->seed;
@@ -400,7 +399,7 @@ static const int kVariantR[] = {4, 4, 8, 16, 128};
 static void launch_kernel(plis_ctx* c, int which, const KernelArgs& a) {
     const LaunchEnv e{c->stream,     c->split_ev,   c->blocks, c->wpb,        c->nreal,
                       c->decide_chunks, (uint32_t)c->cus, c->finish_bpc, c->learned_bpc, c->nh.C > 1,
-                      c->mlp_act == 1, c->learned_on != 0, c->edge_parallel};
+                      c->d_frw != nullptr, c->mlp_act == 1, c->learned_on != 0, c->edge_parallel};
     switch (c->variant) {
         case 0: launch_variant<1, 4>(e, which, a); break;
         case 1: launch_variant<3, 4>(e, which, a); break;
@@ -790,7 +789,6 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         (rc = upload(c, &c->d_iw, hiw)) || (rc = upload(c, &c->d_comp, hcomp)) ||
         (rc = upload(c, &c->d_cw, hcw)) || (rc = upload(c, &c->d_icw, hicw)) ||
         (rc = dev_alloc(c, &c->d_pa_t, c->ntiles)) || (rc = dev_alloc(c, &c->d_pb_t, c->ntiles)) ||
-        (rc = dev_alloc(c, &c->d_redo, c->ntiles)) ||
         (rc = dev_alloc(c, &c->d_pa_c, (size_t)c->nreal * kDecideChunks)) ||
         (rc = dev_alloc(c, &c->d_pb_c, (size_t)c->nreal * kDecideChunks)) ||
         (rc = upload(c, &c->d_dcnt, std::vector<uint32_t>(c->nreal, 0u))) ||
@@ -799,8 +797,9 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         plis_destroy(c);
         return rc;
     }
-    // the forward CSR and the zeroed balances serve the edge-parallel leap
-    const bool ep = !any_asym && !huge_tile;
+    // the forward CSR serves the edge-parallel leap and the resident kernel,
+    // the zeroed balances the former
+    const bool ep = !huge_tile && c->variant <= 3;
     const ResLists lists = res_lists(nh, I);
     c->resident_fits = resident_fit(c, nh, D, lists, hfrp, huge_tile);
     if ((ep || c->resident_fits) && ((rc = upload(c, &c->d_frp, hfrp)) || (rc = upload(c, &c->d_fcw, hfcw)))) {
@@ -808,7 +807,8 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         plis_destroy(c);
         return rc;
     }
-    if (ep && (rc = upload(c, &c->d_gdelta, std::vector<unsigned long long>(hx.size(), 0ull)))) {
+    if (ep && ((rc = upload(c, &c->d_gdelta, std::vector<unsigned long long>(hx.size(), 0ull))) ||
+               (any_asym && (rc = upload(c, &c->d_frw, hfrw))))) {
         g_create_err = c->err;
         plis_destroy(c);
         return rc;
@@ -844,7 +844,6 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         c->res.jpe = jpe;
         c->res.hm = hm;
         c->res.fwd = fw;
-        c->res.count_redo = ep && c->variant <= 3 ? 1u : 0u;
     }
     c->edge_parallel = ep;
     if (hipHostMalloc((void**)&c->h_ndone, sizeof(uint32_t)) != hipSuccess) {
@@ -852,8 +851,13 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         plis_destroy(c);
         return PLIS_ERR_HIP;
     }
+    // 16 blocks of 4 waves per CU unless told otherwise: about one tile per
+    // wave, so that tiles start as others end (Brusselator mesh of 1,048,576
+    // subvolumes 203 us a step with 4 blocks per CU, 193 with 8, 185 with 16;
+    // 2.6 M subvolumes of bistable grids 238, 228, 210; below one tile per
+    // wave the shapes are the same)
     set_shape(c, params->waves_per_block > 0 ? (uint32_t)params->waves_per_block : 4u,
-              params->blocks_per_cu > 0 ? (uint32_t)params->blocks_per_cu : 4u);
+              params->blocks_per_cu > 0 ? (uint32_t)params->blocks_per_cu : 16u);
     *out = c;
     return PLIS_OK;
 }
@@ -912,7 +916,6 @@ extern "C" int plis_run_until(plis_ctx* c, double t_end, double t_pause, uint64_
     uint32_t ndone = 0;
     if (int rc = arm(c, t_end, t_pause, step_limit, &ndone)) return rc;
     uint32_t* d_ndone = c->d_cnt;
-    uint32_t k = 2;
     uint64_t polls = 0, last_progress = 0;
     auto progress = [&]() {
         uint64_t p = 0;
@@ -920,14 +923,34 @@ extern "C" int plis_run_until(plis_ctx* c, double t_end, double t_pause, uint64_
         return p;
     };
     last_progress = progress();
+    // An iteration makes at most one step, so `left` -- the most steps that
+    // some realization has to its limit, less the iterations launched since
+    // the controls were read -- bounds how many more are of use.  With no end
+    // time or pause in sight they are launched up to 256 at once; a run to a
+    // time doubles its batches from 2, since any of them may be its last.
+    auto to_limit = [&]() {
+        uint64_t m = 0;
+        for (const auto& r : c->ctl_host)
+            if (!r.done && r.steps < step_limit) m = std::max(m, step_limit - r.steps);
+        return m;
+    };
+    uint64_t left = to_limit();
+    const bool timed = t_end < __builtin_huge_val() || t_pause < __builtin_huge_val();
+    uint32_t k = timed ? 2 : 256;
     const bool res = resident(c);
     if (ndone < c->nreal && !res)
         if (int rc = prologue(c)) return rc;
     while (ndone < c->nreal) {
-        if (int rc = res ? resident_iters(c, 1024) : graph_iters(c, k)) return rc;
+        if (left == 0) {  // leap-backs: some realization is behind
+            if (int rc = pull_ctl(c)) return rc;
+            left = std::max<uint64_t>(1, to_limit());
+        }
+        const uint32_t n = res ? 1024u : (uint32_t)std::min<uint64_t>(k, left);
+        if (int rc = res ? resident_iters(c, n) : graph_iters(c, n)) return rc;
         HIPCHK(c, hipMemcpyAsync(c->h_ndone, d_ndone, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         ndone = *c->h_ndone;
+        left -= std::min<uint64_t>(left, n);
         if (k < 64) k *= 2;
         // every iteration of an armed realization either accepts a step or
         // leaps back; a batch of iterations without either means the control
@@ -966,7 +989,7 @@ extern "C" int plis_iterate(plis_ctx* c, uint32_t n) {
 
 extern "C" int plis_profile_kernels(plis_ctx* c, uint32_t n, double* out) {
     if (!c || !out) return PLIS_ERR_ARG;
-    // per iteration: before/after each of the 4 phases, and 2 events
+    // per iteration: before/after each of the 4 phases, and one event
     // between the leap pass's kernels
     // (the folded order launches the leap pass, the tau pass and commit +
     // decide; its decide slot stays empty and its commit slot times the
@@ -985,7 +1008,7 @@ extern "C" int plis_profile_kernels(plis_ctx* c, uint32_t n, double* out) {
             const int which = fold ? (k == 0 ? 4 : k == 3 ? 6 : k) : k;
             hipEvent_t* e = &ev[1 + 10 * (size_t)i];
             HIPCHK(c, hipEventRecord(e[2 * k], c->stream));
-            c->split_ev = k == 2 ? &e[8] : nullptr;
+            c->split_ev = k == 2 ? &e[8] : nullptr;  // (after the draws)
             if (!(fold && k == 1)) launch_kernel(c, which, a);
             c->split_ev = nullptr;
             HIPCHK(c, hipEventRecord(e[2 * k + 1], c->stream));
@@ -1006,9 +1029,7 @@ extern "C" int plis_profile_kernels(plis_ctx* c, uint32_t n, double* out) {
         if (c->edge_parallel) {
             HIPCHK(c, hipEventElapsedTime(&x, e[4], e[8]));
             t[4] += x;
-            HIPCHK(c, hipEventElapsedTime(&x, e[8], e[9]));
-            t[5] += x;
-            HIPCHK(c, hipEventElapsedTime(&x, e[9], e[5]));
+            HIPCHK(c, hipEventElapsedTime(&x, e[8], e[5]));
             t[6] += x;
         }
     }
@@ -1223,17 +1244,15 @@ extern "C" int plis_launch_shape(plis_ctx* c, int32_t* out) {
 
 // Sentinels of plis_debug_poison: harmless if read (no index leaves its
 // range), but a read changes the trajectory -- a tiny tau in the tau
-// partials, firings and a negative flag in the leap partials, tile 0 in the
-// redo list (its open draws would be added twice), huge counts in the
-// non-current count buffers.
+// partials, firings and a negative flag in the leap partials, huge counts in
+// the non-current count buffers.
 constexpr uint32_t kPoisonCount = 0x7FFFFFF0u;
 
-__global__ __launch_bounds__(256) void poison_parts_kernel(PartA* pa, PartB* pb, uint32_t* redo, uint32_t ntiles,
+__global__ __launch_bounds__(256) void poison_parts_kernel(PartA* pa, PartB* pb, uint32_t ntiles,
                                                            PartA* pc, PartB* pbc, uint32_t nchunks) {
     for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < ntiles; t += gridDim.x * blockDim.x) {
         pa[t] = PartA{1e-300, 1e-300, 0u, 0xDEADu};
         pb[t] = PartB{1ull << 40, 1u, 7u};
-        redo[t] = 0u;
     }
     for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < nchunks; t += gridDim.x * blockDim.x) {
         pc[t] = PartA{1e-300, 1e-300, 0u, 0xDEADu};
@@ -1250,7 +1269,7 @@ extern "C" int plis_debug_poison(plis_ctx* c) {
         HIPCHK(c, hipMemsetD32Async(other + ri.x_off, (int)kPoisonCount, (size_t)c->S * ri.N, c->stream));
     }
     hipLaunchKernelGGL(poison_parts_kernel, dim3(std::min<uint32_t>((c->ntiles + 255) / 256, 1024u)), dim3(256), 0,
-                       c->stream, c->d_pa_t, c->d_pb_t, c->d_redo, c->ntiles, c->d_pa_c, c->d_pb_c,
+                       c->stream, c->d_pa_t, c->d_pb_t, c->ntiles, c->d_pa_c, c->d_pb_c,
                        c->nreal * kDecideChunks);
     HIPCHK(c, hipGetLastError());
     // the partials no longer hold any proposal

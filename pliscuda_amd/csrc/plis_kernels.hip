@@ -726,7 +726,6 @@ template <int MS, int MR>
 __global__ __launch_bounds__(decide_threads<MS>()) void decide_kernel(KernelArgs a) {
     const uint32_t nch = a.decide_chunks;
     const uint32_t r = blockIdx.x / nch, chunk = blockIdx.x % nch;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *a.redo_count = 0u;  // the coming leap pass's redo list
     if (r >= a.nreal) return;
     // the realization's control block and info in one round of loads
     const RealInfo ri = ld_ro(a.info + r);
@@ -973,60 +972,63 @@ __device__ __forceinline__ bool leap_subvolume(const KernelArgs& a, const NetVie
 }
 
 // ---------------------------------------------------------------------------
-// Edge-parallel leap of one tile (symmetric realizations).
+// Edge-parallel leap of one tile.
 //
-// Each undirected edge {v, u}, v < u, is drawn once, by the tile of its
-// lower end: the tile's forward-CSR entries are contiguous, lane l takes
+// Each pair of linked subvolumes {v, u}, v < u, is drawn once, by the tile of
+// its lower end: the tile's forward-CSR entries are contiguous, lane l takes
 // entries l, l+64, ... (coalesced loads, no divergence from uneven degrees),
 // each one 8-byte word that holds the neighbour, the owning subvolume's
-// index in the tile and the weight, and draws both hop directions of every species from the
-// edge's coarse Philox block; then lane i draws the reactions of subvolume
-// v0+i (one coarse block per 16 reactions).
+// index in the tile and the weight (an asymmetric topology's weight of the
+// hop back in a second array), and draws both hop directions of every species
+// from the pair's coarse Philox block; then lane i draws the reactions of
+// subvolume v0+i (one coarse block per 16 reactions).
 // Balances of the tile's own subvolumes collect in LDS, those of other
 // tiles' subvolumes go straight to the global balances (gdelta); integer
 // atomics keep every sum exact and order-free.  phase_b_finish_kernel adds
 // the balances to the counts once every draw of the pass is in.
 //
-// Compacted draws.  Almost every draw of a step is 0 (hop means are ~1e-3
-// on the headline mesh), so phase_b_kernel's walk only applies the zero
+// Compacted draws.  Almost every draw of a step is 0 where hop means are
+// small (~1e-3 on the headline mesh), so the walk only applies the zero
 // shortcut to the coarse byte of each draw's word: a draw it cannot settle
-// as 0 goes to the wavefront's LDS queue as its code and coarse byte, and
-// after the walk the whole wavefront draws the queued ones, one per lane --
-// the fine bits, the float squeeze, then the double search where the
-// squeeze cannot decide -- so the fine block and the search run once per 64
-// open draws instead of once per draw site.  A tile whose queue
-// overflows, or that holds a draw whose mean may be 10 or more (PTRS; see
-// kPtrsMaybeF), applies nothing
-// from its queue and goes on the redo list: phase_b_redo_kernel walks it
-// again and draws every draw the zero shortcut leaves open (the same test
-// on the same inputs) with the complete sampler.  Draws are functions of
-// their counters, so the two passes give the tile the values one pass
-// would.  No call and no PTRS in phase_b_kernel keeps its register
-// footprint, and so its occupancy, at that of the walk.
+// as 0 goes to the wavefront's LDS queue as its code and coarse byte, and the
+// whole wavefront draws the queued ones, one per lane -- the fine bits, the
+// float squeeze, then the double search where the squeeze cannot decide, PTRS
+// for a mean of 10 or more -- so the fine block and the search run once per 64
+// open draws instead of once per draw site.  The queue is drawn when the next
+// 64 entries' open draws might not fit and at the end of the walk; a drained
+// walk forms its loads again, so nothing of it is live across the sampler.
+// Every draw is inline: no call keeps the kernel at the walk's registers.
+// (A tile whose queue overflowed, or that held a mean of 10 or more, used to
+// go to a second kernel that drew one draw site at a time on two blocks per
+// CU: where means are ~0.5, as in the bistable model at equilibrium, every
+// tile did, 80 us of a 127 us step on the 64^3 grid; and where none did, its
+// empty launch took 4.4 us.)
 // ---------------------------------------------------------------------------
-constexpr uint32_t kQueue = 256;               // queued draws per wavefront
-constexpr uint32_t kQueueReact = 0x80000000u;  // reaction code: flag | lane << 8 | j
-constexpr uint32_t kQueueDefer = kQueue + 1u;  // count bump that sends the tile to the redo pass
-// A hop's float mean is within 8 * 2^-24 (relative) of its double mean, so a
-// float mean at or below kPtrsMaybeF is a double mean below 10 (at most
-// 9.99990 * (1 + 5e-7)): the walk defers a tile with a float mean above it,
-// and every queued draw of a tile it does not defer has a double mean below
-// 10 (a deferred tile whose means are below 10 after all gets the same
-// values from the redo pass's complete sampler).
+// A tile counts as beyond its queue (plis_redo_tiles) with more open draws
+// than kQueue or a mean that may be 10 or more: a hop's float mean is within
+// 8 * 2^-24 (relative) of its double mean, so one at or below kPtrsMaybeF is
+// a double mean below 10.
+constexpr uint32_t kQueue = 256;
 constexpr float kPtrsMaybeF = 9.9999f;
+constexpr uint32_t kQueueReact = 0x80000000u;  // reaction: flag | lane << 16 | j << 8 | byte
+                                               // hop: entry << 12 | w << 8 | byte (kMaxTileEdges)
+constexpr float kNoHop = -0x1p+100f;           // rate of a hop that is critical or absent: never open
 
-// Queue append by the whole wavefront (every lane calls it at the same
-// point, qn is wave-uniform): the lanes whose draw is open take consecutive
-// slots in lane order (a ballot and its prefix count, no LDS atomics).
-__device__ __forceinline__ void q_append(uint2* s_q, uint32_t& qn, bool open, uint32_t code, uint32_t word) {
-    const unsigned long long mq = __ballot(open);
-    if (mq == 0ull) return;
-    if (open) {
-        const uint32_t slot =
-            qn + __builtin_amdgcn_mbcnt_hi((uint32_t)(mq >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mq, 0u));
-        if (slot < kQueue) s_q[slot] = make_uint2(code, word);
-    }
-    qn += (uint32_t)__popcll(mq);
+// One wavefront's staging.  The queue takes all draws of 64 entries.
+template <int MS, bool GEN>
+struct LeapLds {
+    static constexpr uint32_t kCap = MS > 2 ? 128u * MS : 256u;
+    uint32_t x[MS][kTile];   // the tile's counts
+    float rate[MS][kTile];   // their hops' coarse rates (kCoarseScale tau d x; kNoHop)
+    int32_t del[MS][kTile];  // the tile's balances
+    uint32_t q[kCap];
+    int32_t c[GEN ? kTile : 1];
+};
+
+__device__ __forceinline__ uint64_t wave_ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+
+__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
 __device__ __forceinline__ double hop_mean(double d, uint32_t x, double wq, double tau, int nc) {
@@ -1039,49 +1041,137 @@ __device__ __forceinline__ float hop_mean_f(double d, uint32_t x, float w, float
     return hop_active(d, x, nc) ? tauf * (((float)d * (float)x) * w) : 0.0f;
 }
 
-// Balance b of species s at subvolume u: LDS when u is in the tile.
-__device__ __forceinline__ void add_balance(const KernelArgs& a, const RealInfo& ri,
-                                            unsigned long long (*s_del)[kTile], uint32_t v0, int s, uint32_t u,
-                                            long long b) {
-    if (u - v0 < (uint32_t)kTile) atomicAdd(&s_del[s][u - v0], (unsigned long long)b);
+// Balance b of species s at subvolume u.  In the tile: 32 bits in LDS for
+// |b| < 2^11 (a row takes part in fewer than 2^20 draws of a pass, so the sum
+// stays below 2^31), else straight to the 64-bit global balance.
+template <int MS, bool GEN>
+__device__ __forceinline__ void add_balance(const KernelArgs& a, const RealInfo& ri, LeapLds<MS, GEN>& L, uint32_t v0,
+                                            int s, uint32_t u, long long b) {
+    if (u - v0 < (uint32_t)kTile && b > -2048 && b < 2048) atomicAdd(&L.del[s][u - v0], (int32_t)b);
     else atomicAdd(&a.gdelta[ri.x_off + (uint64_t)s * ri.N + u], (unsigned long long)b);
 }
 
-// The lane's draws: its forward entries (both directions of every species
-// of an undirected edge), then the reactions of its subvolume.  Walk: the
-// zero shortcut on the coarse bytes, draws it leaves open queued; returns
-// the queue count (wave-uniform; above kQueue when the tile goes to the
-// redo pass).  REDO: the open draws, with the complete sampler, applied.
-// Control flow stays wave-uniform around every queue append: the loops run
-// the same trip count on every lane, lanes without work carry flags.
-template <int MS, int MR, bool REDO>
-__device__ __forceinline__ uint32_t walk_fwd_draws(const KernelArgs& a, const NetView& n, const RealInfo& ri,
-                                                   const uint32_t* X, uint32_t v0, const StepView& sv,
-                                                   const uint32_t (*s_x)[kTile],
-                                                   unsigned long long (*s_del)[kTile], uint32_t eb, uint32_t ee,
-                                                   const int32_t* s_c, uint2* s_q, unsigned long long& fire) {
-    static_assert(MS <= 8, "one coarse block per edge; hop codes hold w = 2s + direction in 4 bits");
+// One queued draw: its fine bits complete the word the walk queued the
+// coarse byte of (one Philox call, whichever the kind), then the sampler,
+// applied to the balances.  big: the mean may be 10 or more.
+template <int MS, bool GEN>
+__device__ __forceinline__ void drain_draw(const KernelArgs& a, const NetView& n, const RealInfo& ri,
+                                           const uint32_t* X, uint32_t v0, const StepView& sv, LeapLds<MS, GEN>& L,
+                                           uint32_t eb, uint32_t code, unsigned long long& fire, bool& big) {
+    const bool react = (code & kQueueReact) != 0u;
+    const uint32_t hb = code & 255u;
+    uint32_t i, c1, w, c3;
+    bool fwd = true;
+    float lf;
+    double lam;
+    if (react) {
+        i = (code >> 16) & 63u;
+        w = (code >> 8) & 255u;
+        double aj = n.k[(n.C > 1 ? L.c[GEN ? i : 0] : 0) * n.R + (int)w];
+        const int nr = n.nrs[w];
+        for (int r = 0; r < nr; ++r) aj = aj * binom_d(L.x[n.rs[w * 3 + r]][i], n.rr[w * 3 + r]);
+        lam = sv.tau * aj;
+        lf = (float)lam;
+        c1 = kSelfId;
+        c3 = ctr_word3(sv.real, sv.attempt, kReact, kFineBlock + (w >> 2));
+        big = big || !(lam < kPoissonInvMax);
+    } else {
+        const uint64_t e = ri.fe_off + eb + (code >> 12);
+        const uint64_t cw = a.fcw[e];
+        w = (code >> 8) & 15u;
+        i = (uint32_t)cw >> 26;
+        c1 = (uint32_t)cw & kFwdIdMask;
+        fwd = (w & 1u) == 0u;
+        const int s = (int)(w >> 1);
+        float wf = __uint_as_float((uint32_t)(cw >> 32));
+        if constexpr (GEN)
+            if (!fwd && a.frw) wf = a.frw[e];
+        double d;
+        uint32_t xs;
+        const bool local = c1 - v0 < (uint32_t)kTile;
+        if (fwd) {
+            d = n.d[(n.C > 1 ? L.c[GEN ? i : 0] : 0) * n.S + s];
+            xs = L.x[s][i];
+        } else {
+            const int cu = n.C > 1 ? (local ? L.c[GEN ? c1 - v0 : 0] : a.comp[ri.comp_off + c1]) : 0;
+            d = n.d[cu * n.S + s];
+            xs = local ? L.x[s][c1 - v0] : X[ri.x_off + (uint64_t)s * ri.N + c1];
+        }
+        lam = hop_mean(d, xs, (double)wf, sv.tau, a.n_critical);
+        lf = hop_mean_f(d, xs, wf, (float)sv.tau, a.n_critical);
+        c3 = ctr_word3(sv.real, sv.attempt, kHop, kFineBlock + (w >> 2));
+        big = big || lf > kPtrsMaybeF;
+    }
+    const uint32_t word = draw_word(hb, philox10(v0 + i, c1, sv.step, c3, a.seed_lo, a.seed_hi), w);
+    long long k = lf < kSqueezeMaxF ? poisson_squeeze(lf, __uint2float_rn(word) * 0x1p-32f) : -1;
+    if (k < 0) {
+        if (lam < kPoissonInvMax) k = inversion_search(lam, word);
+        else k = ptrs_draw(lam, DrawId{v0 + i, c1, sv.step, c3, a.seed_lo, a.seed_hi, w & 3u});
+    }
+    if (k == 0) return;
+    fire += (unsigned long long)k;
+    if (react) {
+        for (int s = 0; s < n.S; ++s) {
+            const int nu = n.nu[s * n.R + (int)w];
+            if (nu != 0) add_balance(a, ri, L, v0, s, v0 + i, k * (long long)nu);
+        }
+    } else {
+        const int s = (int)(w >> 1);
+        const long long b = fwd ? -k : k;  // balance of v0 + i
+        add_balance(a, ri, L, v0, s, v0 + i, b);
+        add_balance(a, ri, L, v0, s, c1, -b);
+    }
+}
+
+// The draws of one tile into the global balances.  Control flow stays
+// wave-uniform around every queue append: the loops run the same trip count
+// on every lane, lanes without work carry flags.  Returns whether the tile
+// counts as beyond its queue.  GEN: several compartments or an asymmetric
+// topology.
+template <int MS, int MR, bool GEN>
+__device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetView& n, const RealInfo& ri,
+                                                const uint32_t* X, uint32_t v0, const StepView& sv,
+                                                LeapLds<MS, GEN>& L, unsigned long long& fire) {
+    static_assert(MS <= 8 && MR <= 16, "one coarse block per pair and per subvolume; hop codes hold w in 4 bits");
+    constexpr uint32_t kCap = LeapLds<MS, GEN>::kCap;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t N = ri.N;
+    const uint32_t v = v0 + lane;
+    const bool vok = v < N;
     const int nc = a.n_critical;
-    const uint64_t* cwp = a.fcw + ri.fe_off;  // neighbour, row in the tile and weight in one load
-    const double tau = sv.tau;
-    const float tauf = (float)tau;
-    const uint32_t k0 = a.seed_lo, k1 = a.seed_hi;
-    const uint32_t c3hop = ctr_word3(sv.real, sv.attempt, kHop, 0u);
-    uint32_t qn = 0u;
-    bool defer = false;
-    // one compartment: the diffusion constants as float and the species
-    // that hop at all (hop_mean_f's operands and test, loaded once)
     const uint32_t nc1 = nc > 1 ? (uint32_t)nc : 1u;
-    float df[MS];
+    const double tau = sv.tau;
+    const uint32_t k0 = a.seed_lo, k1 = a.seed_hi;
+    const float scale = (float)tau * kCoarseScale;
+    const int cl = (GEN && n.C > 1 && vok) ? a.comp[ri.comp_off + v] : 0;
+    float dt[MS];    // one compartment: the species' rate per molecule
     bool dpos[MS];
 #pragma unroll
     for (int s = 0; s < MS; ++s) {
         const double d = n.d[s < n.S ? s : 0];
-        df[s] = (float)d;
+        dt[s] = (float)d * scale;
         dpos[s] = s < n.S && d > 0.0;
+        const uint32_t x = (vok && s < n.S) ? X[ri.x_off + (uint64_t)s * N + v] : 0u;
+        L.x[s][lane] = x;
+        L.del[s][lane] = 0;
+        if (GEN && n.C > 1) {
+            const double dc = n.d[cl * n.S + (s < n.S ? s : 0)];
+            L.rate[s][lane] = (s < n.S && dc > 0.0 && x >= nc1) ? ((float)dc * scale) * (float)x : kNoHop;
+        } else {
+            L.rate[s][lane] = (dpos[s] && x >= nc1) ? dt[s] * (float)x : kNoHop;
+        }
     }
+    if constexpr (GEN) L.c[lane] = cl;
+    const uint32_t eb = wave_uniform(a.frp[ri.rp_off + v0]);
+    const uint32_t ee = wave_uniform(a.frp[ri.rp_off + min(v0 + (uint32_t)kTile, N)]);
+    lds_wave_sync();
+    const uint64_t* cwp = a.fcw + ri.fe_off;  // neighbour, row in the tile and weight in one load
+    const float* rwp = GEN && a.frw ? a.frw + ri.fe_off : nullptr;
+    const uint32_t c3hop = ctr_word3(sv.real, sv.attempt, kHop, 0u);
+    const uint32_t c3react = ctr_word3(sv.real, sv.attempt, kReact, 0u);
+    const uint32_t nit = (ee - eb + (uint32_t)kTile - 1u) / (uint32_t)kTile;
+    uint32_t qn = 0u, opened = 0u;
+    bool big = false;
     // software pipeline: an entry's neighbour counts are requested one
     // iteration ahead, its neighbour id and weight two iterations ahead
     // (counts of a neighbour inside the tile are read from global memory
@@ -1090,278 +1180,112 @@ __device__ __forceinline__ uint32_t walk_fwd_draws(const KernelArgs& a, const Ne
 #pragma unroll
         for (int s = 0; s < MS; ++s) xo[s] = X[ri.x_off + (uint64_t)(s < n.S ? s : n.S - 1) * N + u];
     };
-    const uint32_t e0 = eb + lane;
-    const uint64_t cw0 = e0 < ee ? cwp[e0] : (uint64_t)v0 | kOneW;
-    const uint64_t cw1 = e0 + (uint32_t)kTile < ee ? cwp[e0 + kTile] : (uint64_t)v0 | kOneW;
-    uint32_t u_cur = (uint32_t)cw0 & kFwdIdMask, u_next = (uint32_t)cw1 & kFwdIdMask;
-    uint32_t i_cur = (uint32_t)cw0 >> 26, i_next = (uint32_t)cw1 >> 26;
-    float w_cur = __uint_as_float((uint32_t)(cw0 >> 32));
-    float w_next = __uint_as_float((uint32_t)(cw1 >> 32));
-    uint32_t xn[MS];
+    uint32_t it = 0u;
+    int j = 0;
+    for (bool all = false; !all;) {
+        if (it < nit) {
+            uint32_t e = eb + it * (uint32_t)kTile + lane;
+            const uint64_t none = (uint64_t)v0 | kOneW;
+            uint64_t cw = e < ee ? cwp[e] : none, cw_next = e + (uint32_t)kTile < ee ? cwp[e + kTile] : none;
+            uint32_t xn[MS];
+            counts((uint32_t)cw & kFwdIdMask, xn);
+            for (; it < nit; ++it, e += (uint32_t)kTile) {
+                const bool valid = e < ee;
+                const uint32_t i = (uint32_t)cw >> 26;            // the entry's row in the tile
+                const uint32_t u = (uint32_t)cw & kFwdIdMask;     // u > v0 + i
+                const float w0 = __uint_as_float((uint32_t)(cw >> 32));
+                float w1 = w0;
+                if constexpr (GEN)
+                    if (rwp && valid) w1 = rwp[e];
+                uint32_t xc[MS];
 #pragma unroll
-    for (int s = 0; s < MS; ++s) xn[s] = 0u;
-    if (e0 < ee) counts(u_cur, xn);
-    const uint32_t nit = (ee - eb + (uint32_t)kTile - 1u) / (uint32_t)kTile;
-    for (uint32_t it = 0; it < nit; ++it) {
-        const uint32_t e = e0 + it * (uint32_t)kTile;
-        const bool valid = e < ee;
-        const uint32_t i = i_cur;  // the edge's row in the tile
-        const uint32_t vo = v0 + i;
-        const uint32_t u = u_cur;  // u > vo: vo is the edge's lower end
-        const float wf = w_cur;
-        uint32_t xc[MS];
+                for (int s = 0; s < MS; ++s) xc[s] = xn[s];
+                cw = cw_next;
+                if (e + (uint32_t)kTile < ee) {
+                    counts((uint32_t)cw & kFwdIdMask, xn);
+                    if (e + 2u * (uint32_t)kTile < ee) cw_next = cwp[e + 2u * kTile];
+                }
+                int cu = 0;
+                if (GEN && n.C > 1 && valid)
+                    cu = u - v0 < (uint32_t)kTile ? L.c[GEN ? u - v0 : 0] : a.comp[ri.comp_off + u];
+                // rates of the draws w = 2s + direction (0: v0 + i -> u)
+                float rate[2 * MS];
+                bool any = false;
 #pragma unroll
-        for (int s = 0; s < MS; ++s) xc[s] = xn[s];
-        u_cur = u_next;
-        w_cur = w_next;
-        i_cur = i_next;
-        if (e + (uint32_t)kTile < ee) {
-            counts(u_cur, xn);
-            if (e + 2u * (uint32_t)kTile < ee) {
-                const uint64_t cw2 = cwp[e + 2u * kTile];
-                u_next = (uint32_t)cw2 & kFwdIdMask;
-                i_next = (uint32_t)cw2 >> 26;
-                w_next = __uint_as_float((uint32_t)(cw2 >> 32));
+                for (int s = 0; s < MS; ++s) {
+                    rate[2 * s] = L.rate[s][i];
+                    bool on = xc[s] >= nc1;
+                    float r;
+                    if (GEN && n.C > 1) {
+                        const double d = n.d[cu * n.S + (s < n.S ? s : 0)];
+                        on = on && s < n.S && d > 0.0;
+                        r = ((float)d * scale) * (float)xc[s];
+                    } else {
+                        on = on && dpos[s];
+                        r = dt[s] * (float)xc[s];
+                    }
+                    rate[2 * s + 1] = on ? r : kNoHop;
+                    any = any || on || rate[2 * s] > 0.0f;
+                }
+                if (wave_ballot(any && valid) == 0ull) continue;
+                const U4 o = philox10(v0 + i, u, sv.step, c3hop, k0, k1);
+                bool open[2 * MS];
+                uint32_t total = 0u;
+#pragma unroll
+                for (int w = 0; w < 2 * MS; ++w) {
+                    open[w] = valid && __builtin_fmaf(rate[w], (w & 1) ? w1 : w0, (float)coarse_byte(o, (uint32_t)w)) > kCoarseTop;
+                    total += (uint32_t)__popcll(wave_ballot(open[w]));
+                }
+                if (qn + total > kCap) break;  // drawn below, then this entry again
+                opened += total;
+                const uint32_t code = (e - eb) << 12;
+#pragma unroll
+                for (int w = 0; w < 2 * MS; ++w) {
+                    const uint64_t m = wave_ballot(open[w]);
+                    if (m == 0ull) continue;
+                    if (open[w]) L.q[qn + lanes_below(m)] = code | ((uint32_t)w << 8) | coarse_byte(o, (uint32_t)w);
+                    qn += (uint32_t)__popcll(m);
+                }
             }
         }
-        const bool local = u - v0 < (uint32_t)kTile;
-        const int co = n.C > 1 ? s_c[i] : 0;
-        const int cu = (n.C > 1 && valid) ? (local ? s_c[u - v0] : a.comp[ri.comp_off + u]) : 0;
-        const uint32_t ecode = (e - eb) << 4;
-        // the means of the edge's draws w = 2s + direction (0: vo -> u) and
-        // their coarse bounds
-        float lw[2 * MS], gw[2 * MS];
-        bool any = false;
-#pragma unroll
-        for (int s = 0; s < MS; ++s) {
-            const int sq = s < n.S ? s : 0;
-            if (n.C > 1) {
-                const bool on = valid && s < n.S;
-                lw[2 * s] = on ? hop_mean_f(n.d[co * n.S + sq], s_x[sq][i], wf, tauf, nc) : 0.0f;
-                lw[2 * s + 1] = on ? hop_mean_f(n.d[cu * n.S + sq], xc[s], wf, tauf, nc) : 0.0f;
-            } else {
-                const bool on = valid && dpos[s];
-                const uint32_t xo = s_x[sq][i], xu = xc[s];
-                lw[2 * s] = (on && xo >= nc1) ? tauf * ((df[s] * (float)xo) * wf) : 0.0f;
-                lw[2 * s + 1] = (on && xu >= nc1) ? tauf * ((df[s] * (float)xu) * wf) : 0.0f;
+        if (it == nit) {
+            // reactions of subvolume v, propensities and criticality as react_props
+            // computes them (same operations, one reaction at a time)
+            const U4 o = philox10(v, kSelfId, sv.step, c3react, k0, k1);
+            for (; j < n.R; ++j) {
+                double aj = n.k[cl * n.R + j];
+                bool low = false;
+                const int nr = n.nrs[j];
+                for (int q = 0; q < nr; ++q) {
+                    const int sq = n.rs[j * 3 + q], rq = n.rr[j * 3 + q];
+                    const uint32_t xs = L.x[sq][lane];
+                    aj = aj * binom_d(xs, rq);
+                    low = low || below_nc(xs, rq, nc);
+                }
+                const uint32_t hb = coarse_byte(o, (uint32_t)j);
+                const bool open = vok && !(n.order[j] > 0 && low) && aj > 0.0 && !coarse_zero(tau * aj, hb);
+                const uint64_t m = wave_ballot(open);
+                const uint32_t cnt = (uint32_t)__popcll(m);
+                if (qn + cnt > kCap) break;
+                opened += cnt;
+                if (open) L.q[qn + lanes_below(m)] = kQueueReact | (lane << 16) | ((uint32_t)j << 8) | hb;
+                qn += cnt;
             }
+            all = j >= n.R;
         }
-#pragma unroll
-        for (int w = 0; w < 2 * MS; ++w) {
-            gw[w] = coarse_bound(lw[w]);
-            any = any || lw[w] > 0.0f;
-            if constexpr (!REDO) defer = defer || lw[w] > kPtrsMaybeF;
-        }
-        if (__ballot(any) == 0ull) continue;
-        const U4 o = philox10(vo, u, sv.step, c3hop, k0, k1);  // the coarse block (MS <= 8)
-#pragma unroll
-        for (int w = 0; w < 2 * MS; ++w) {
-            const uint32_t hb = coarse_byte(o, (uint32_t)w);
-            const bool open = (float)hb > gw[w];
-            if constexpr (REDO) {
-                if (!open) continue;
-                const int s = w >> 1;
-                const bool fwd = (w & 1) == 0;
-                const uint32_t fb = c3hop | (kFineBlock + ((uint32_t)w >> 2));
-                const U4 f = philox10(vo, u, sv.step, fb, k0, k1);
-                const uint32_t word = draw_word(hb, f, (uint32_t)w);
-                if (poisson_zero_f(lw[w], word) >= 0) continue;
-                const double lam = fwd ? hop_mean(n.d[co * n.S + s], s_x[s][i], (double)wf, tau, nc)
-                                       : hop_mean(n.d[cu * n.S + s], xc[s], (double)wf, tau, nc);
-                const long long k = poisson(lam, word, DrawId{vo, u, sv.step, fb, k0, k1, (uint32_t)w & 3u});
-                if (k == 0) continue;
-                fire += (unsigned long long)k;
-                const long long bv = fwd ? -k : k;  // balance of vo
-                atomicAdd(&s_del[s][i], (unsigned long long)bv);
-                add_balance(a, ri, s_del, v0, s, u, -bv);
-            } else {
-                q_append(s_q, qn, open, ecode | (uint32_t)w, hb);
-            }
-        }
+        lds_wave_sync();
+        for (uint32_t q = lane; q < qn; q += (uint32_t)kTile)
+            drain_draw<MS, GEN>(a, n, ri, X, v0, sv, L, eb, L.q[q], fire, big);
+        lds_wave_sync();
+        qn = 0u;
     }
-    const uint32_t v = v0 + lane;
-    const bool vok = v < N;
-    // reactions of subvolume v, propensities and criticality as react_props
-    // computes them (same operations, one reaction at a time)
-    const int c = (n.C > 1 && vok) ? s_c[lane] : 0;
-    uint32_t blk = 0xFFFFFFFFu;
-    U4 o{0, 0, 0, 0};
-    const uint32_t c3base = ctr_word3(sv.real, sv.attempt, kReact, 0u);
-    for (int j = 0; j < n.R; ++j) {
-        double aj = n.k[c * n.R + j];
-        bool low = false;
-        const int nr = n.nrs[j];
-        for (int q = 0; q < nr; ++q) {
-            const int sq = n.rs[j * 3 + q], rq = n.rr[j * 3 + q];
-            const uint32_t xs = s_x[sq][lane];
-            aj = aj * binom_d(xs, rq);
-            low = low || below_nc(xs, rq, nc);
-        }
-        const bool live = vok && !(n.order[j] > 0 && low) && aj > 0.0;
-        const uint32_t b = (uint32_t)j >> 4;
-        if (b != blk) {
-            o = philox10(v, kSelfId, sv.step, c3base | b, k0, k1);
-            blk = b;
-        }
-        const uint32_t hb = coarse_byte(o, (uint32_t)j);
-        const double lam = tau * aj;
-        const bool open = live && !coarse_zero(lam, hb);
-        if constexpr (REDO) {
-            if (!open) continue;
-            const long long k = leap_draw(lam, hb, v, kSelfId, sv.step, c3base, k0, k1, (uint32_t)j);
-            if (k == 0) continue;
-            fire += (unsigned long long)k;
-            for (int s = 0; s < n.S; ++s) {
-                const int nu = n.nu[s * n.R + j];
-                if (nu != 0) atomicAdd(&s_del[s][lane], (unsigned long long)(k * (long long)nu));
-            }
-        } else {
-            defer = defer || (open && !(lam < kPoissonInvMax));
-            q_append(s_q, qn, open, kQueueReact | (lane << 8) | (uint32_t)j, hb);
-        }
-    }
-    // a mean >= 10 (PTRS) anywhere: the tile goes to the redo pass
-    if (__ballot(defer) != 0ull) qn += kQueueDefer;
-    return qn;
-}
-
-// A queued hop, decoded: owner i, neighbour u, draw w = 2s + direction,
-// species s and the mean in double.
-struct QueuedHop {
-    uint32_t i, u, w;
-    int s;
-    bool fwd;  // the hop v0 + i -> u
-    double lam;
-    float lf;  // the mean as the walk formed it in single precision
-};
-
-template <int MS>
-__device__ __forceinline__ QueuedHop queued_hop(const KernelArgs& a, const NetView& n, const RealInfo& ri,
-                                                const uint32_t* X, uint32_t v0, const StepView& sv,
-                                                const uint32_t (*s_x)[kTile], uint32_t eb,
-                                                const int32_t* s_c, uint32_t code) {
-    QueuedHop h;
-    const uint32_t e = eb + (code >> 4);
-    h.w = code & 15u;
-    const uint64_t cw = a.fcw[ri.fe_off + e];
-    h.i = (uint32_t)cw >> 26;
-    h.u = (uint32_t)cw & kFwdIdMask;
-    h.s = (int)(h.w >> 1);
-    h.fwd = (h.w & 1u) == 0u;
-    const float wf = __uint_as_float((uint32_t)(cw >> 32));
-    const double wq = (double)wf;
-    double d;
-    uint32_t xs;
-    if (h.fwd) {
-        d = n.d[(n.C > 1 ? s_c[h.i] : 0) * n.S + h.s];
-        xs = s_x[h.s][h.i];
-    } else {
-        const bool local = h.u - v0 < (uint32_t)kTile;
-        const int cu = n.C > 1 ? (local ? s_c[h.u - v0] : a.comp[ri.comp_off + h.u]) : 0;
-        d = n.d[cu * n.S + h.s];
-        xs = local ? s_x[h.s][h.u - v0] : X[ri.x_off + (uint64_t)h.s * ri.N + h.u];
-    }
-    h.lam = hop_mean(d, xs, wq, sv.tau, a.n_critical);
-    h.lf = hop_mean_f(d, xs, wf, (float)sv.tau, a.n_critical);
-    return h;
-}
-
-// One queued draw: its fine bits complete the word the walk queued the
-// coarse byte of (one Philox call, whichever the kind), then the float
-// squeeze on the mean rounded to float, the double search where it cannot
-// decide (the drain runs only when every queued mean is below 10), applied
-// to the balances.
-template <int MS>
-__device__ __forceinline__ void drain_fwd_draw(const KernelArgs& a, const NetView& n, const RealInfo& ri,
-                                               const uint32_t* X, uint32_t v0, const StepView& sv,
-                                               const uint32_t (*s_x)[kTile], unsigned long long (*s_del)[kTile],
-                                               uint32_t eb, const int32_t* s_c, uint2 q,
-                                               unsigned long long& fire) {
-    const uint32_t code = q.x, hb = q.y;
-    const bool react = (code & kQueueReact) != 0u;
-    uint32_t i, c1, w, c3;
-    float lf;
-    double lam;
-    QueuedHop h{};
-    if (react) {
-        i = (code >> 8) & 63u;
-        w = code & 255u;
-        double aj = n.k[(n.C > 1 ? s_c[i] : 0) * n.R + (int)w];
-        const int nr = n.nrs[w];
-        for (int r = 0; r < nr; ++r) aj = aj * binom_d(s_x[n.rs[w * 3 + r]][i], n.rr[w * 3 + r]);
-        lam = sv.tau * aj;
-        lf = (float)lam;
-        c1 = kSelfId;
-        c3 = ctr_word3(sv.real, sv.attempt, kReact, kFineBlock + (w >> 2));
-    } else {
-        h = queued_hop<MS>(a, n, ri, X, v0, sv, s_x, eb, s_c, code);
-        i = h.i;
-        w = h.w;
-        lam = h.lam;
-        lf = h.lf;
-        c1 = h.u;
-        c3 = ctr_word3(sv.real, sv.attempt, kHop, kFineBlock + (w >> 2));
-    }
-    const uint32_t word = draw_word(hb, philox10(v0 + i, c1, sv.step, c3, a.seed_lo, a.seed_hi), w);
-    long long k = lf < kSqueezeMaxF ? poisson_squeeze(lf, __uint2float_rn(word) * 0x1p-32f) : -1;
-    if (k < 0) k = inversion_search(lam, word);
-    if (k == 0) return;
-    fire += (unsigned long long)k;
-    if (react) {
-        for (int s = 0; s < n.S; ++s) {
-            const int nu = n.nu[s * n.R + (int)w];
-            if (nu != 0) atomicAdd(&s_del[s][i], (unsigned long long)(k * (long long)nu));
-        }
-    } else {
-        const long long b = h.fwd ? -k : k;  // balance of v0 + i
-        atomicAdd(&s_del[h.s][i], (unsigned long long)b);
-        add_balance(a, ri, s_del, v0, h.s, h.u, -b);
-    }
-}
-
-// The draws of one tile into the global balances.  Returns false when the
-// tile's open draws are left to phase_b_redo_kernel (its settled draws are
-// applied either way).
-template <int MS, int MR, bool REDO>
-__device__ __forceinline__ bool leap_tile_fwd(const KernelArgs& a, const NetView& n, const RealInfo& ri,
-                                              const uint32_t* X, uint32_t v0, const StepView& sv,
-                                              uint32_t (*s_x)[kTile], unsigned long long (*s_del)[kTile],
-                                              int32_t* s_c, uint2* s_q,
-                                              unsigned long long& fire) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t N = ri.N;
-    const uint32_t v = v0 + lane;
-    const bool active = v < N;
-#pragma unroll
-    for (int s = 0; s < MS; ++s) {
-        s_x[s][lane] = (active && s < n.S) ? X[ri.x_off + (uint64_t)s * N + v] : 0u;
-        s_del[s][lane] = 0ull;
-    }
-    s_c[lane] = (n.C > 1 && active) ? a.comp[ri.comp_off + v] : 0;
-    const uint32_t eb = wave_uniform(a.frp[ri.rp_off + v0]);
-    const uint32_t ee = wave_uniform(a.frp[ri.rp_off + min(v0 + (uint32_t)kTile, N)]);
-    lds_wave_sync();
-    const uint32_t qn = walk_fwd_draws<MS, MR, REDO>(a, n, ri, X, v0, sv, s_x, s_del, eb, ee, s_c, s_q, fire);
-    lds_wave_sync();
-    bool complete = true;
-    if constexpr (!REDO) {
-        const uint32_t cnt = wave_uniform(qn);
-        // (a deferred tile's count is above kQueue: a draw whose mean may be
-        // 10 or more needs PTRS, so nothing queued is drawn and the redo
-        // pass draws all of it)
-        complete = cnt <= kQueue;
-        if (complete) {
-            for (uint32_t q = lane; q < cnt; q += (uint32_t)kTile)
-                drain_fwd_draw<MS>(a, n, ri, X, v0, sv, s_x, s_del, eb, s_c, s_q[q], fire);
-            lds_wave_sync();
-        }
-    }
-    if (active) {
+    if (vok) {
 #pragma unroll
         for (int s = 0; s < MS; ++s)
-            if (s < n.S && s_del[s][lane] != 0ull) atomicAdd(&a.gdelta[ri.x_off + (uint64_t)s * N + v], s_del[s][lane]);
+            if (s < n.S && L.del[s][lane] != 0)
+                atomicAdd(&a.gdelta[ri.x_off + (uint64_t)s * N + v], (unsigned long long)(long long)L.del[s][lane]);
     }
-    return complete;
+    return opened > kQueue || wave_ballot(big) != 0ull;
 }
 
 // The end of the leap pass for one tile: new counts = counts + global
@@ -1411,9 +1335,15 @@ __device__ __forceinline__ void finish_tile(const KernelArgs& a, const NetView& 
     }
 }
 
+// PartB::bad of two sets of tiles: bit 0 (a negative count) or-ed, the number
+// of tiles beyond their queue above it added.
+__device__ __forceinline__ uint32_t merge_bad(uint32_t p, uint32_t q) {
+    return ((p & ~1u) + (q & ~1u)) | ((p | q) & 1u);
+}
+
 __device__ __forceinline__ void reduce_partB(unsigned long long& fire, uint32_t& bad, uint32_t& viol) {
     fire = wave_fold_u64(0ull, fire, [](unsigned long long p, unsigned long long q) { return p + q; });
-    bad = __ballot(bad != 0u) != 0ull ? 1u : 0u;
+    if (__ballot(bad != 0u) != 0ull) bad = wave_fold_u32(0u, bad, merge_bad);
     if (__ballot(viol != 0u) != 0ull)
         viol = wave_fold_u32(0u, viol, [](uint32_t p, uint32_t q) { return p + q; });
 }
@@ -1423,6 +1353,8 @@ __device__ __forceinline__ void reduce_partB(unsigned long long& fire, uint32_t&
 // decided).  lead: the one thread that counts a finished realization in.
 __device__ bool commit_step(const KernelArgs& a, const RealInfo& ri, unsigned long long fire, uint32_t bad,
                             uint32_t viol, RealCtl& c, bool lead) {
+    if (bad >> 1 && lead) atomicAdd(a.redo_total, (unsigned long long)(bad >> 1));
+    bad &= 1u;
     // A learned proposal is judged by Cao's leap condition after the fact: it
     // is kept only without negative populations and with no more violating
     // subvolumes than the plain method produces -- mean mu = viol_rate_max N,
@@ -1498,85 +1430,49 @@ __device__ __forceinline__ StepView step_view(const RealInfo& ri, cptr<RealCtl> 
     return sv;
 }
 
-// Phase B of one tile.  EP: the draws of an edge-parallel tile into the
-// global balances (REDO: the open draws, complete sampler); the tile's
-// firings go to its partial and phase_b_finish_kernel completes the leap.
-// Otherwise one lane walks one subvolume's out- and in-edges and finishes it.
-template <int MS, int MR, bool EP, bool REDO>
-__device__ __forceinline__ void phase_b_tile(const KernelArgs& a, const NetView& n, uint32_t t,
-                                             uint32_t (*s_x)[kTile], unsigned long long (*s_del)[kTile],
-                                             int32_t* s_c, uint2* s_q) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const TileEnt te = ld_ro(a.tiles + t);
-    const uint32_t r = wave_uniform(te.r);
-    const RealInfo ri = ld_ro(a.info + r);
-    const cptr<RealCtl> cp = ro(a.ctl + r);
-    if (wave_uniform(cp->done)) return;
-    const StepView sv = step_view(ri, cp);
-    const uint32_t cur = wave_uniform(cp->cur);
-    const uint32_t* X = cur ? a.x1 : a.x0;
-    uint32_t* Xn = cur ? a.x0 : a.x1;
-    unsigned long long fire = 0;
-    uint32_t bad = 0, viol = 0;
-    if constexpr (EP) {
-        const bool complete = leap_tile_fwd<MS, MR, REDO>(a, n, ri, X, te.v0, sv, s_x, s_del, s_c, s_q, fire);
-        reduce_partB(fire, bad, viol);
-        if (lane == 0) {
-            if (!complete) {
-                const uint32_t slot = atomicAdd(a.redo_count, 1u);
-                if (slot < a.ntiles) a.redo_tiles[slot] = t;  // one entry per tile per pass
-            }
-            // the redo pass adds the firings of the open draws
-            a.partB_tile[t] = PartB{(REDO ? a.partB_tile[t].fire : 0ull) + fire, 0u, 0u};
-        }
-        return;
-    } else {
-        const uint32_t v = te.v0 + lane;
-        if (v < ri.N) bad = leap_subvolume<MS, MR>(a, n, ri, X, Xn, v, sv, fire, viol) ? 1u : 0u;
-    }
-    reduce_partB(fire, bad, viol);
-    if (lane == 0) a.partB_tile[t] = PartB{fire, bad, viol};
-}
-
-// The one-compartment edge-parallel leap of up to 5 species: asking for 6
-// waves per SIMD holds it to 80 VGPRs (16 bytes of spill per lane), which
-// measures faster than 85 VGPRs at 5 waves (the walk waits on gathers and
-// LDS, more waves hide it).
-template <int MS, int MR, bool EP, bool MC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EP && !MC && MS <= 5 ? 6 : 1)))
+// The leap pass.  EP: the draws of every tile into the global balances; the
+// tile's firings go to its partial and phase_b_finish_kernel completes the
+// leap.  Otherwise one lane walks one subvolume's out- and in-edges and
+// finishes it (networks beyond 8 species or 16 reactions, topologies beyond
+// an entry's or a code's bits).  GEN: several compartments, or (EP) an
+// asymmetric topology.
+//
+// The edge-parallel leap of up to 5 species, one compartment, runs at 5 waves
+// per SIMD (96 VGPRs): at 6 the sampler spills (1M-subvolume Brusselator mesh
+// 83.6 -> 94.5 us), at 4 fewer waves hide the walk's gathers (88 us).
+template <int MS, int MR, bool EP, bool GEN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EP && !GEN && MS <= 5 ? 5 : 1)))
 void phase_b_kernel(KernelArgs a) {
-    const uint32_t wv = wave_uniform(threadIdx.x >> 6);
-    // LDS staging for the edge-parallel path (up to 4 waves per block)
-    constexpr int LS = EP ? MS : 1;
-    __shared__ uint32_t s_x[4][LS][kTile];
-    __shared__ unsigned long long s_del[4][LS][kTile];
-    __shared__ int32_t s_c[4][kTile];
-    __shared__ uint2 s_q[4][EP ? kQueue : 1];
+    const uint32_t wv = wave_uniform(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    __shared__ LeapLds<EP ? MS : 1, GEN> s_l[EP ? 4 : 1];  // (up to 4 waves per block)
     for (uint32_t it = 0;; ++it) {
         const uint32_t t = tile_at(it, a.ntiles, a.waves_per_block);
         if (t == 0xFFFFFFFFu) break;
         KernelArgs al = a;  // network tables through per-tile opaque pointers, as in phase_a_kernel
         asm volatile("" : "+s"(al.net_i), "+s"(al.net_d));
-        const NetView n = net_view<MC>(al);
-        phase_b_tile<MS, MR, EP, false>(a, n, t, s_x[wv], s_del[wv], s_c[wv], s_q[wv]);
+        const NetView n = net_view<GEN>(al);
+        const TileEnt te = ld_ro(a.tiles + t);
+        const uint32_t r = wave_uniform(te.r);
+        const RealInfo ri = ld_ro(a.info + r);
+        const cptr<RealCtl> cp = ro(a.ctl + r);
+        if (wave_uniform(cp->done)) continue;
+        const StepView sv = step_view(ri, cp);
+        const uint32_t cur = wave_uniform(cp->cur);
+        const uint32_t* X = cur ? a.x1 : a.x0;
+        unsigned long long fire = 0;
+        uint32_t bad = 0, viol = 0;
+        if constexpr (EP) {
+            const bool over = leap_tile_draws<MS, MR, GEN>(a, n, ri, X, te.v0, sv, s_l[wv], fire);
+            reduce_partB(fire, bad, viol);
+            if (lane == 0) a.partB_tile[t] = PartB{fire, over && a.count_redo ? 2u : 0u, 0u};
+        } else {
+            const uint32_t v = te.v0 + lane;
+            uint32_t* Xn = cur ? a.x0 : a.x1;
+            if (v < ri.N) bad = leap_subvolume<MS, MR>(a, n, ri, X, Xn, v, sv, fire, viol) ? 1u : 0u;
+            reduce_partB(fire, bad, viol);
+            if (lane == 0) a.partB_tile[t] = PartB{fire, bad, viol};
+        }
     }
-}
-
-// Tiles phase_b_kernel left on the redo list: their open draws, drawn with
-// the complete sampler.  The list is emptied by decide_kernel before each leap pass.
-template <int MS, int MR, bool MC>
-__global__ __launch_bounds__(256) void phase_b_redo_kernel(KernelArgs a) {
-    const NetView n = net_view<MC>(a);
-    const uint32_t wv = wave_uniform(threadIdx.x >> 6);
-    const uint32_t wpb = blockDim.x >> 6;
-    __shared__ uint32_t s_x[4][MS][kTile];
-    __shared__ unsigned long long s_del[4][MS][kTile];
-    __shared__ int32_t s_c[4][kTile];
-    const uint32_t cnt = min(wave_uniform(*a.redo_count), a.ntiles);
-    if (blockIdx.x == 0 && threadIdx.x == 0 && cnt != 0u) *a.redo_total += cnt;
-    for (uint32_t q = blockIdx.x * wpb + wv; q < cnt; q += gridDim.x * wpb)
-        phase_b_tile<MS, MR, true, true>(a, n, wave_uniform(a.redo_tiles[q]), s_x[wv], s_del[wv], s_c[wv],
-                                         nullptr);
 }
 
 // The end of the edge-parallel leap pass: every tile adds the global
@@ -1606,7 +1502,10 @@ void phase_b_finish_kernel(KernelArgs a) {
         finish_tile<MS, MR>(a, n, ri, cur ? a.x1 : a.x0, cur ? a.x0 : a.x1, te.v0, sv, fire, bad, viol, x, nx,
                             a.judge_on != 0);
         reduce_partB(fire, bad, viol);
-        if (lane == 0) a.partB_tile[t] = PartB{a.partB_tile[t].fire + fire, bad, viol};
+        if (lane == 0) {
+            const PartB p = a.partB_tile[t];
+            a.partB_tile[t] = PartB{p.fire + fire, merge_bad(p.bad, bad), viol};
+        }
     }
 }
 
@@ -1632,7 +1531,7 @@ static __global__ __launch_bounds__(1024) void commit_kernel(KernelArgs a) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             fire += p[i].fire;
-            bad |= p[i].bad;
+            bad = merge_bad(bad, p[i].bad);
             viol += p[i].viol;
         }
     }
@@ -1647,7 +1546,7 @@ static __global__ __launch_bounds__(1024) void commit_kernel(KernelArgs a) {
     if (threadIdx.x == 0) {
         for (uint32_t w = 1; w < (blockDim.x >> 6); ++w) {
             fire += s_f[w];
-            bad |= s_b[w];
+            bad = merge_bad(bad, s_b[w]);
             viol += s_v[w];
         }
         finalize_B(a, ri, r, fire, bad, viol, c0);
@@ -1667,7 +1566,6 @@ template <int MS, int MR>
 __global__ __launch_bounds__(decide_threads<MS>()) void commit_decide_kernel(KernelArgs a) {
     const uint32_t nch = a.decide_chunks;
     const uint32_t r = blockIdx.x / nch, chunk = blockIdx.x % nch;
-    if (blockIdx.x == 0u && threadIdx.x == 0u) *a.redo_count = 0u;  // the coming leap pass's redo list
     if (r >= a.nreal) return;
     const RealInfo ri = ld_ro(a.info + r);
     const RealCtl c0 = ld_ro(a.ctl + r);
@@ -1697,7 +1595,7 @@ __global__ __launch_bounds__(decide_threads<MS>()) void commit_decide_kernel(Ker
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             fire += b[i].fire;
-            bad |= b[i].bad;
+            bad = merge_bad(bad, b[i].bad);
             viol += b[i].viol;
             merge_partA(tp, t2, v2, p[i].tp, p[i].t2, p[i].v2);
         }
@@ -1714,7 +1612,7 @@ __global__ __launch_bounds__(decide_threads<MS>()) void commit_decide_kernel(Ker
     if (wv == 0)  // the first wavefront, every lane alike
         for (uint32_t w = 1; w < (blockDim.x >> 6); ++w) {
             fire += s_f[w];
-            bad |= s_b[w];
+            bad = merge_bad(bad, s_b[w]);
             viol += s_v[w];
         }
     if (nch > 1u) {

@@ -13,7 +13,7 @@ struct LaunchEnv {
     hipStream_t stream;
     hipEvent_t* split_ev;  // profiling: events between the leap pass's kernels, or nullptr
     uint32_t blocks, wpb, nreal, decide_chunks, cus, finish_bpc, learned_bpc;
-    bool mc, gelu, learned_on, edge_parallel;
+    bool mc, asym, gelu, learned_on, edge_parallel;
 };
 
 // decide_kernel and commit_decide_kernel: most blocks per realization
@@ -23,5 +23,11 @@ constexpr uint32_t kDecideChunks = 16;
 // MR reactions (plis_variant.hip).
 template <int MS, int MR>
 void launch_variant(const LaunchEnv& c, int which, const KernelArgs& a);
+
+// The learned kernels of the instantiation (plis_variant_learned.hip; at most
+// 8 species and 16 reactions).
+enum LearnedKernel { kLearnedTau, kLearnedFinish, kLearnedRecords };
+template <int MS, int MR>
+void launch_learned(const LaunchEnv& c, int which, const KernelArgs& a);
 
 }  // namespace plis

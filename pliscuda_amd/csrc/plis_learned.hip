@@ -235,7 +235,10 @@ __global__ __launch_bounds__(256) void learned_finish_kernel(KernelArgs a) {
             viol = leap_condition_broken<MS, MR>(n, c, a.n_critical, a.epsilon, a.theta, x, nx, av0, crit0, av1);
         }
         reduce_partB(fire, bad, viol);
-        if (lane == 0) a.partB_tile[t] = PartB{a.partB_tile[t].fire + fire, bad, viol};
+        if (lane == 0) {
+            const PartB p = a.partB_tile[t];
+            a.partB_tile[t] = PartB{p.fire + fire, merge_bad(p.bad, bad), viol};
+        }
         propose_tile<MS, MR, ACT>(a, n, ri, W, xn, av1, crit1, act, v, sv.step + 1u, sv.tau, t);
     }
 }

@@ -95,8 +95,10 @@ __device__ __forceinline__ bool coarse_zero(double lam, uint32_t hb) {
 // of rounding, less than the 2^-12 taken off), so (hb + 1) 2^-8 < 1 - lam
 // <= e^-lam: every word with that top byte gives 0.  A mean above 1 is
 // never settled here.
+constexpr float kCoarseTop = 0x1.fdffe0p+7f;   // 255 - 2^-12
+constexpr float kCoarseScale = 0x1.00004p+8f;  // 256 + 2^-10
 __device__ __forceinline__ float coarse_bound(float lf) {
-    return lf > 0.0f ? 0x1.fdffe0p+7f - lf * 0x1.00004p+8f : 256.0f;
+    return lf > 0.0f ? kCoarseTop - lf * kCoarseScale : 256.0f;
 }
 
 __device__ __forceinline__ double uniform01(uint32_t w) { return ((double)w + 0.5) * 0x1p-32; }
@@ -129,27 +131,42 @@ __device__ __forceinline__ double dexp(double x) {
 
 // log(x) for normal x > 0: x = m 2^e with m in (sqrt2/2, sqrt2],
 // log m = 2 atanh(s), s = (m-1)/(m+1), odd series through s^21.
-__device__ __attribute__((noinline)) double dlog(double x) {
+// The series' coefficients 1/21, 1/19, ..., 1/3.
+constexpr double kLogSeries[10] = {
+    0x1.8618618618618p-5, 0x1.af286bca1af28p-5, 0x1.e1e1e1e1e1e1ep-5, 0x1.1111111111111p-4, 0x1.3b13b13b13b14p-4,
+    0x1.745d1745d1746p-4, 0x1.c71c71c71c71cp-4, 0x1.2492492492492p-3, 0x1.999999999999ap-3, 0x1.5555555555555p-2};
+
+__device__ __forceinline__ double dlog_series(double x, const double (&c)[10]) {
     const unsigned long long b = (unsigned long long)__double_as_longlong(x);
     int e = (int)((b >> 52) & 0x7FF) - 1023;
     double m = __longlong_as_double((long long)((b & 0x000FFFFFFFFFFFFFull) | 0x3FF0000000000000ull));
     if (m > kSqrt2) { m = m * 0.5; e += 1; }
     const double s = (m - 1.0) / (m + 1.0);
     const double z = s * s;
-    double P = 0x1.8618618618618p-5;                 // 1/21
-    P = __builtin_fma(P, z, 0x1.af286bca1af28p-5);   // 1/19
-    P = __builtin_fma(P, z, 0x1.e1e1e1e1e1e1ep-5);   // 1/17
-    P = __builtin_fma(P, z, 0x1.1111111111111p-4);   // 1/15
-    P = __builtin_fma(P, z, 0x1.3b13b13b13b14p-4);   // 1/13
-    P = __builtin_fma(P, z, 0x1.745d1745d1746p-4);   // 1/11
-    P = __builtin_fma(P, z, 0x1.c71c71c71c71cp-4);   // 1/9
-    P = __builtin_fma(P, z, 0x1.2492492492492p-3);   // 1/7
-    P = __builtin_fma(P, z, 0x1.999999999999ap-3);   // 1/5
-    P = __builtin_fma(P, z, 0x1.5555555555555p-2);   // 1/3
+    double P = c[0];
+#pragma unroll
+    for (int i = 1; i < 10; ++i) P = __builtin_fma(P, z, c[i]);
     P = __builtin_fma(P, z, 1.0);
     const double t = (2.0 * s) * P;
     const double ed = (double)e;
     return __builtin_fma(ed, kLn2Hi, __builtin_fma(ed, kLn2Lo, t));
+}
+
+__device__ __attribute__((noinline)) double dlog(double x) { return dlog_series(x, kLogSeries); }
+
+// For the inside of a rare loop: the coefficients come from memory through a
+// pointer made opaque here, so that they are not held in registers around it.
+static __constant__ const double kLogSeriesMem[10] = {
+    kLogSeries[0], kLogSeries[1], kLogSeries[2], kLogSeries[3], kLogSeries[4],
+    kLogSeries[5], kLogSeries[6], kLogSeries[7], kLogSeries[8], kLogSeries[9]};
+__device__ __forceinline__ double dlog_lean(double x) {
+    typedef const double __attribute__((address_space(4)))* cp;
+    cp p = (cp)kLogSeriesMem;
+    asm volatile("" : "+s"(p));
+    double c[10];
+#pragma unroll
+    for (int i = 0; i < 10; ++i) c[i] = p[i];
+    return dlog_series(x, c);
 }
 
 // sqrt by six Newton-Heron steps from an exponent-halving first guess.
@@ -162,8 +179,9 @@ __device__ __forceinline__ double dsqrt(double x) {
     return y;
 }
 
-// log k!: exact table below 10, Stirling series through 1/z^5 above.
-__device__ __forceinline__ double dlogfact(long long k) {
+// log k!: exact table below 10, Stirling series through 1/z^5 above (logz =
+// log(k + 1)).
+__device__ __forceinline__ double dlogfact(long long k, double logz) {
     if (k < 10) {
         switch ((int)k) {
             case 2: return 0x1.62e42fefa39efp-1;
@@ -179,7 +197,7 @@ __device__ __forceinline__ double dlogfact(long long k) {
     }
     const double z = (double)k + 1.0;
     const double z2 = z * z;
-    return (((double)k + 0.5) * dlog(z) - z) + kHalfLog2Pi + (kC12 - (kC360 - kC1260 / z2) / z2) / z;
+    return (((double)k + 0.5) * logz - z) + kHalfLog2Pi + (kC12 - (kC360 - kC1260 / z2) / z2) / z;
 }
 
 // Draw identity: main counter (c0..c3 with purpose/block), key, word in block.
@@ -196,14 +214,20 @@ __device__ __forceinline__ double extra_uniform(const DrawId& id, uint32_t q) {
     return uniform01(pick(o, q & 3u));
 }
 
-__device__ __attribute__((noinline)) long long poisson_ptrs(double lam, DrawId id) {
+// (inline in kernels that must not make a call, see leap_tile_draws)
+__device__ __forceinline__ long long ptrs_draw(double lam, const DrawId& id) {
     const double slam = dsqrt(lam);
-    const double loglam = dlog(lam);
     const double b = 0.931 + 2.53 * slam;
     const double a = -0.059 + 0.02483 * b;
     const double invalpha = 1.1239 + 1.1328 / (b - 3.4);
     const double vr = 0.9277 - 3.6224 / (b - 2.0);
-    const double loginvalpha = dlog(invalpha);
+    double loglam = 0.0, loginvalpha = 0.0;
+#pragma unroll 1
+    for (uint32_t i = 0; i < 2u; ++i) {
+        const double l = dlog_lean(i ? invalpha : lam);
+        if (i) loginvalpha = l;
+        else loglam = l;
+    }
     const uint32_t c3 = (id.c3 & ~(7u << 7)) | (kExtra << 7);
     // iteration it uses uniforms 2it, 2it+1 of the draw's stream; one Philox
     // call (4 words) covers two iterations
@@ -219,14 +243,25 @@ __device__ __attribute__((noinline)) long long poisson_ptrs(double lam, DrawId i
             const double kd = __builtin_floor((2.0 * a / us + b) * U + lam + 0.43);
             if (us >= 0.07 && V <= vr) return (long long)kd;
             if (kd < 0.0 || (us < 0.013 && V > us)) continue;
-            const long long k = (long long)kd;
-            const double lhs = (dlog(V) + loginvalpha) - dlog(a / (us * us) + b);
-            const double rhs = (-lam + kd * loglam) - dlogfact(k);
-            if (lhs <= rhs) return k;
+            // log V, log(a / us^2 + b) and, for k >= 10, the log of Stirling's z
+            double l[3] = {0.0, 0.0, 0.0};
+            const double z = kd + 1.0;
+#pragma unroll 1
+            for (uint32_t i = 0; i < 3u; ++i) {
+                const double x = i == 0u ? V : (i == 1u ? a / (us * us) + b : z);
+                const double y = dlog_lean(x);
+                if (i == 0u) l[0] = y;
+                else if (i == 1u) l[1] = y;
+                else l[2] = y;
+            }
+            const double lhs = (l[0] + loginvalpha) - l[1];
+            const double rhs = (-lam + kd * loglam) - dlogfact((long long)kd, l[2]);
+            if (lhs <= rhs) return (long long)kd;
         }
     }
     return (long long)__builtin_floor(lam);
 }
+__device__ __attribute__((noinline)) long long poisson_ptrs(double lam, DrawId id) { return ptrs_draw(lam, id); }
 
 // Slow path of the sampler: full sequential-search inversion (mean < 10) or
 // PTRS (mean >= 10).  Kept out of line so the common no-event case below
@@ -335,45 +370,5 @@ __device__ __forceinline__ long long leap_draw(double lam, uint32_t hb, uint32_t
 // below it is within 8 2^-24 (relative) of a double mean below 10, so the
 // double sampler would use the inversion search too.
 constexpr float kSqueezeMaxF = 9.9999f;
-
-// The fast part of a draw whose mean lf was formed in single precision
-// (float operands and products, within 8 2^-24 lf of the double mean lam):
-// 0 for lf <= 0; 0 when u_f <= (1 - lf) - 2^-19, which implies u <= e^-lam
-// (u_f is within 2^-25 + 2^-33 of u, the margin covers both roundings and
-// the mean's error for lf <= 1); the float squeeze below kSqueezeMaxF (its
-// guard band 2^-15 covers the mean's error, <= 5e-6 there); -1 otherwise.
-// A decided value is the one poisson() returns from the double mean.
-__device__ __forceinline__ int poisson_fast_f(float lf, uint32_t u0) {
-    if (!(lf > 0.0f)) return 0;
-    const float u = __uint2float_rn(u0) * 0x1p-32f;
-    if (u <= (1.0f - lf) - 0x1p-19f) return 0;
-    if (!(lf < kSqueezeMaxF)) return -1;
-    return poisson_squeeze(lf, u);
-}
-
-// The zero shortcuts alone: 0 when the draw is certainly 0 (the value
-// poisson() returns), -1 when it may not be.  poisson_zero_f takes a float
-// mean (as poisson_fast_f), poisson_zero a double one (as poisson()).
-__device__ __forceinline__ int poisson_zero_f(float lf, uint32_t u0) {
-    if (!(lf > 0.0f)) return 0;
-    const float u = __uint2float_rn(u0) * 0x1p-32f;
-    return u <= (1.0f - lf) - 0x1p-19f ? 0 : -1;
-}
-__device__ __forceinline__ int poisson_zero(double lam, uint32_t u0) {
-    if (!(lam > 0.0)) return 0;
-    return uniform01(u0) <= (1.0 - lam) - 0x1p-50 ? 0 : -1;
-}
-
-// The fast part of poisson() for kernels that defer the rare hard cases:
-// the zero shortcut and the float squeeze settle the draw (k >= 0, the value
-// poisson() returns); -1 leaves it to the double search (inversion_search)
-// or, for mean >= 10, to PTRS.
-__device__ __forceinline__ int poisson_fast(double lam, uint32_t u0) {
-    if (!(lam > 0.0)) return 0;
-    if (!(lam < kPoissonInvMax)) return -1;
-    const double u = uniform01(u0);
-    if (u <= (1.0 - lam) - 0x1p-50) return 0;
-    return poisson_squeeze((float)lam, (float)u);
-}
 
 }  // namespace plis

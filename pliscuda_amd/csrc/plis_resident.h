@@ -14,7 +14,6 @@ constexpr uint32_t kResidentLdsMax = 160u * 1024u - 2048u;  // dynamic LDS, next
 struct ResidentArgs {
     KernelArgs k;
     uint32_t iters;         // iterations to make at most
-    uint32_t count_redo;    // tiles beyond a wavefront's queue are counted (edge-parallel contexts)
     const int4* rx;         // reaction tables as ResTables describes them
     const int2 *sp, *spe, *jp, *jpe, *hm;
     uint32_t nspe;          // entries of spe and of jpe

@@ -483,7 +483,7 @@ static __global__ __launch_bounds__(1024) void resident_kernel(ResidentArgs ra) 
                         if (v >= N) open = cnt = 0u;
                         code = kResReact | (v << 7) | j0;
                     }
-                    if (ra.count_redo && cnt != 0u) atomicAdd(&tcnt[tile], cnt);
+                    if (a.count_redo && cnt != 0u) atomicAdd(&tcnt[tile], cnt);
                     item += nw;
                 }
                 const unsigned long long any = __ballot(open != 0u);
@@ -528,7 +528,7 @@ static __global__ __launch_bounds__(1024) void resident_kernel(ResidentArgs ra) 
                 V.xn[i] = (uint32_t)y;
             }
             if (bad) s_bad = 1u;
-            if (ra.count_redo)
+            if (a.count_redo)
                 for (uint32_t t = threadIdx.x; t < nt; t += blockDim.x) {
                     if (tcnt[t] > kQueue) atomicAdd(a.redo_total, 1ull);
                     tcnt[t] = 0u;

@@ -17,8 +17,8 @@ namespace plis {
 
 constexpr int kTile = 64;        // subvolumes per tile (one wavefront)
 constexpr uint32_t kFwdIdMask = (1u << 26) - 1u;  // neighbour id bits of a forward entry
-// forward entries of a tile: the leap pass's hop codes hold an entry's offset in 27 bits
-constexpr uint32_t kMaxTileEdges = 1u << 27;
+// forward entries of a tile: the leap pass's hop codes hold an entry's offset in 19 bits
+constexpr uint32_t kMaxTileEdges = 1u << 19;
 constexpr int kMaxS = 64;
 constexpr int kMaxR = 128;
 
@@ -83,7 +83,7 @@ struct PartA {
 };
 struct PartB {
     unsigned long long fire;
-    uint32_t bad, viol;
+    uint32_t bad, viol;  // bad: bit 0 a negative count, above it the tiles beyond their queue
 };
 
 struct KernelArgs {
@@ -117,8 +117,6 @@ struct KernelArgs {
     uint32_t decide_chunks;  // decide_kernel: blocks per realization (1 .. kDecideChunks)
     PartB* partB_tile;
     uint32_t* ndone;
-    uint32_t* redo_count;    // tiles phase B left to the redo pass (reset by decide)
-    uint32_t* redo_tiles;
     // forward CSR (row_ptr layout of rp; entries v -> u with u > v) and the
     // leap pass's global per-subvolume balances (counts layout, zero between
     // passes).  An entry is one 8-byte word: u in bits 0..25, the index of
@@ -127,8 +125,10 @@ struct KernelArgs {
     // pass have fewer than 2^26 subvolumes.
     const uint32_t* frp;
     const uint64_t* fcw;
+    const float* frw;         // asymmetric topologies: weights of the hops back (entries' upper to lower ends)
     unsigned long long* gdelta;
-    unsigned long long* redo_total;  // tiles redone since the context was made
+    unsigned long long* redo_total;  // tiles beyond a wavefront's queue since the context was made
+    uint32_t count_redo;             // those tiles are counted
     double epsilon;
     int32_t n_critical;
     uint32_t seed_lo, seed_hi;

@@ -6,7 +6,7 @@
 #include <algorithm>
 
 #include "plis_launch.h"
-#include "plis_learned.hip"
+#include "plis_kernels.hip"
 
 namespace plis {
 
@@ -22,22 +22,11 @@ void launch_variant(const LaunchEnv& c, int which, const KernelArgs& a) {
     const dim3 grid(c.blocks), block(64 * c.wpb), rgrid(c.nreal), rblock(1024), dblock(decide_threads<MS>());
     const dim3 dgrid(c.nreal * c.decide_chunks);
     const bool mc = c.mc;  // several compartments: per-subvolume rate tables
-    const bool gelu = c.gelu;
-    // learned kernels stage the network in LDS once per block: fewer, longer-lived blocks
-    // the redo list is usually empty or short: two blocks per CU walk it
-    const dim3 rgrid2(std::max<uint32_t>(8u, std::min<uint32_t>(c.blocks, (c.cus * 2u + 7u) & ~7u)));
-    const dim3 fgrid(std::max<uint32_t>(8u, std::min<uint32_t>(c.blocks, (c.cus * c.finish_bpc + 7u) & ~7u)));
-    const dim3 lgrid(std::max<uint32_t>(8u, std::min<uint32_t>(c.blocks, (c.cus * c.learned_bpc + 7u) & ~7u)));
     switch (which) {
         case 0:
             if constexpr (MS <= 8) {
                 if (c.learned_on) {
-                    // one pass covers fallbacks and refreshes; in steady state
-                    // it skips every tile, so it runs on a small grid
-                    if (mc && gelu) hipLaunchKernelGGL((learned_tau_kernel<MS, MR, true, 1>), lgrid, block, 0, c.stream, a);
-                    else if (mc) hipLaunchKernelGGL((learned_tau_kernel<MS, MR, true, 0>), lgrid, block, 0, c.stream, a);
-                    else if (gelu) hipLaunchKernelGGL((learned_tau_kernel<MS, MR, false, 1>), lgrid, block, 0, c.stream, a);
-                    else hipLaunchKernelGGL((learned_tau_kernel<MS, MR, false, 0>), lgrid, block, 0, c.stream, a);
+                    launch_learned<MS, MR>(c, kLearnedTau, a);
                     break;
                 }
             }
@@ -50,29 +39,12 @@ void launch_variant(const LaunchEnv& c, int which, const KernelArgs& a) {
         case 2:
             if constexpr (MS <= 8) {
                 if (c.edge_parallel) {
-                    if (mc) {
-                        hipLaunchKernelGGL((phase_b_kernel<MS, MR, true, true>), grid, block, 0, c.stream, a);
-                        if (c.split_ev) (void)hipEventRecord(c.split_ev[0], c.stream);
-                        hipLaunchKernelGGL((phase_b_redo_kernel<MS, MR, true>), rgrid2, block, 0, c.stream, a);
-                        if (c.split_ev) (void)hipEventRecord(c.split_ev[1], c.stream);
-                        if (!c.learned_on)
-                            hipLaunchKernelGGL((phase_b_finish_kernel<MS, MR, true>), grid, block, 0, c.stream, a);
-                        else if (gelu)
-                            hipLaunchKernelGGL((learned_finish_kernel<MS, MR, true, 1>), fgrid, block, 0, c.stream, a);
-                        else
-                            hipLaunchKernelGGL((learned_finish_kernel<MS, MR, true, 0>), fgrid, block, 0, c.stream, a);
-                    } else {
-                        hipLaunchKernelGGL((phase_b_kernel<MS, MR, true, false>), grid, block, 0, c.stream, a);
-                        if (c.split_ev) (void)hipEventRecord(c.split_ev[0], c.stream);
-                        hipLaunchKernelGGL((phase_b_redo_kernel<MS, MR, false>), rgrid2, block, 0, c.stream, a);
-                        if (c.split_ev) (void)hipEventRecord(c.split_ev[1], c.stream);
-                        if (!c.learned_on)
-                            hipLaunchKernelGGL((phase_b_finish_kernel<MS, MR, false>), grid, block, 0, c.stream, a);
-                        else if (gelu)
-                            hipLaunchKernelGGL((learned_finish_kernel<MS, MR, false, 1>), fgrid, block, 0, c.stream, a);
-                        else
-                            hipLaunchKernelGGL((learned_finish_kernel<MS, MR, false, 0>), fgrid, block, 0, c.stream, a);
-                    }
+                    if (mc || c.asym) hipLaunchKernelGGL((phase_b_kernel<MS, MR, true, true>), grid, block, 0, c.stream, a);
+                    else hipLaunchKernelGGL((phase_b_kernel<MS, MR, true, false>), grid, block, 0, c.stream, a);
+                    if (c.split_ev) (void)hipEventRecord(*c.split_ev, c.stream);
+                    if (c.learned_on) launch_learned<MS, MR>(c, kLearnedFinish, a);
+                    else if (mc) hipLaunchKernelGGL((phase_b_finish_kernel<MS, MR, true>), grid, block, 0, c.stream, a);
+                    else hipLaunchKernelGGL((phase_b_finish_kernel<MS, MR, false>), grid, block, 0, c.stream, a);
                     break;
                 }
             }
@@ -93,7 +65,7 @@ void launch_variant(const LaunchEnv& c, int which, const KernelArgs& a) {
             hipLaunchKernelGGL((commit_decide_kernel<MS, MR>), dgrid, dblock, 0, c.stream, a);
             break;
         case 5:
-            if constexpr (MS <= 8) hipLaunchKernelGGL((records_kernel<MS, MR>), grid, block, 0, c.stream, a);
+            if constexpr (MS <= 8) launch_learned<MS, MR>(c, kLearnedRecords, a);
             break;
         default:
             break;
