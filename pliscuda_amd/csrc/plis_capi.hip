@@ -72,6 +72,10 @@ struct plis_ctx {
     uint64_t model_hash = 0;  // network tables, every realization's CSR and compartments
     std::vector<RealInfo> info;
     std::vector<RealCtl> ctl_host;
+    bool ctl_fresh = false;  // ctl_host equals the device's controls, nothing launched since
+    char* h_stage = nullptr;  // pinned, two halves of stage_half bytes (fetch)
+    size_t stage_half = 0;
+    hipEvent_t stage_ev[2] = {};
     // device buffers
     int32_t* d_net_i = nullptr;
     double* d_net_d = nullptr;
@@ -397,6 +401,7 @@ static const int kVariantS[] = {1, 3, 5, 8, 64};
 static const int kVariantR[] = {4, 4, 8, 16, 128};
 
 static void launch_kernel(plis_ctx* c, int which, const KernelArgs& a) {
+    c->ctl_fresh = false;
     const LaunchEnv e{c->stream,     c->split_ev,   c->blocks, c->wpb,        c->nreal,
                       c->decide_chunks, (uint32_t)c->cus, c->finish_bpc, c->learned_bpc, c->nh.C > 1,
                       c->d_frw != nullptr, c->mlp_act == 1, c->learned_on != 0, c->edge_parallel};
@@ -489,6 +494,7 @@ static int graph_iters(plis_ctx* c, uint32_t n) {
             }
         }
     }
+    c->ctl_fresh = false;
     while (n > 0) {
         int k = kGraphSizes - 1;
         while ((1u << k) > n) --k;
@@ -525,6 +531,9 @@ extern "C" void plis_destroy(plis_ctx* c) {
     drop_graphs(c);
     for (void* p : c->allocs) (void)hipFree(p);
     if (c->h_ndone) (void)hipHostFree(c->h_ndone);
+    if (c->h_stage) (void)hipHostFree(c->h_stage);
+    for (auto e : c->stage_ev)
+        if (e) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -539,7 +548,7 @@ static bool resident_fit(plis_ctx* c, const NetHeader& h, const std::vector<doub
         nf = std::max<uint64_t>(nf, frp[ri.rp_off + ri.N]);
         ne = std::max<uint64_t>(ne, ri.n_in);
     }
-    if (huge) return false;
+    if (huge || maxN > kResidentMaxN) return false;
     // One CU makes a step of N subvolumes in about 5 us + N (2 + 0.84 S deg +
     // 2.8 R) ns (measured: A-B-C 7.6 us at 64, 15 at 512, 26 at 1,000, 41 at
     // 1,728; diffusion of one species 21 at 1,728; Brusselator mesh 25 at 512,
@@ -573,6 +582,7 @@ static bool resident(const plis_ctx* c) { return c->resident_fits && !c->learned
 static int resident_iters(plis_ctx* c, uint32_t n) {
     ResidentArgs a = c->res;
     a.k = make_args(c);
+    c->ctl_fresh = false;
     // (a launch makes at most 4,096 iterations, some tens of milliseconds)
     while (n > 0) {
         a.iters = std::min(n, 4096u);
@@ -622,6 +632,13 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
     std::vector<uint32_t> hx, hrp, hcol, hirp, hicol, hfrp;
     std::vector<float> hw, hiw;
     std::vector<uint64_t> hcw, hicw, hfcw;  // interleaved id + weight bits
+    auto weight_of = [](uint64_t cw) {
+        const uint32_t b = (uint32_t)(cw >> 32);
+        float w;
+        std::memcpy(&w, &b, 4);
+        return w;
+    };
+    bool small = true;  // every realization so far may be stepped by resident_kernel
     std::vector<uint32_t> hfsrc;
     std::vector<float> hfrw;
     auto idw = [](uint32_t u, float w) {
@@ -664,16 +681,19 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         hcol.insert(hcol.end(), g.col.begin(), g.col.end());
         Csr in;
         if (!sym) transpose(g, N, in);
+        small = small && N <= kResidentMaxN;
         // forward CSR: each pair of linked subvolumes once, in the row of its
         // lower end, with the weights of both hops (an asymmetric topology's
         // may differ, or one of them be absent: weight 0)
         ri.fe_off = hfcw.size();
+        if (!sym)  // the first asymmetric realization: the weights back of those before it
+            for (size_t e = hfrw.size(); e < ri.fe_off; ++e) hfrw.push_back(weight_of(hfcw[e]));
         for (uint32_t v = 0; v < N; ++v) {
             hfrp.push_back((uint32_t)(hfcw.size() - ri.fe_off));
             auto put = [&](uint32_t u, float wf, float wr) {
                 hfcw.push_back(idw((u & kFwdIdMask) | ((v % kTile) << 26), wf));
-                hfsrc.push_back(v);
-                hfrw.push_back(wr);
+                if (small) hfsrc.push_back(v);
+                if (!sym || any_asym) hfrw.push_back(wr);
             };
             uint32_t q = g.rp[v], qe = g.rp[v + 1];
             if (sym) {
@@ -807,17 +827,22 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         plis_destroy(c);
         return rc;
     }
-    if (ep && ((rc = upload(c, &c->d_gdelta, std::vector<unsigned long long>(hx.size(), 0ull))) ||
-               (any_asym && (rc = upload(c, &c->d_frw, hfrw))))) {
+    if (ep && ((rc = dev_alloc(c, &c->d_gdelta, hx.size())) || (any_asym && (rc = upload(c, &c->d_frw, hfrw))))) {
         g_create_err = c->err;
         plis_destroy(c);
         return rc;
     }
+    if (ep && (hipMemsetAsync(c->d_gdelta, 0, hx.size() * sizeof(unsigned long long), c->stream) != hipSuccess ||
+               hipStreamSynchronize(c->stream) != hipSuccess)) {
+        g_create_err = "clearing the balances failed";
+        plis_destroy(c);
+        return PLIS_ERR_HIP;
+    }
     if (c->resident_fits) {
         std::vector<uint4> fwd(hfcw.size());
         for (size_t e = 0; e < fwd.size(); ++e) {
-            uint32_t back;
-            std::memcpy(&back, &hfrw[e], 4);
+            uint32_t back = (uint32_t)(hfcw[e] >> 32);
+            if (any_asym) std::memcpy(&back, &hfrw[e], 4);
             fwd[e] = {(uint32_t)hfcw[e] & kFwdIdMask, (uint32_t)(hfcw[e] >> 32), hfsrc[e], back};
         }
         int4* rx = nullptr;
@@ -862,10 +887,48 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
     return PLIS_OK;
 }
 
+// The realizations' controls on the host; the stream has drained when it
+// returns.  Nothing is read where nothing was launched since the last time
+// (a program that asks for the state and statistics of every realization after
+// a run read the whole table twice per realization: 64 boxes of 512
+// subvolumes, 3.8 ms of a 9.9 ms pass).
 static int pull_ctl(plis_ctx* c) {
+    if (c->ctl_fresh) return 0;
     HIPCHK(c, hipMemcpyAsync(c->ctl_host.data(), c->d_ctl, c->ctl_host.size() * sizeof(RealCtl),
                              hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->ctl_fresh = true;
+    return 0;
+}
+
+// Device memory to the caller's through the context's pinned buffer: the copy
+// of one half overlaps the copy out of the other.  (hipMemcpy to pageable
+// memory stages too, but one piece at a time and with its own launch.)
+static int fetch(plis_ctx* c, void* to, const void* from, size_t bytes) {
+    if (!c->h_stage) {
+        const size_t half = std::min<size_t>(1u << 21, ((size_t)c->total_counts * sizeof(uint32_t) + 4095) & ~(size_t)4095);
+        HIPCHK(c, hipHostMalloc((void**)&c->h_stage, 2 * half));
+        c->stage_half = half;
+        for (auto& e : c->stage_ev) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
+    char* dst = static_cast<char*>(to);
+    const char* src = static_cast<const char*>(from);
+    size_t sent = 0, done = 0;
+    auto send = [&](int h) {
+        const size_t n = std::min(c->stage_half, bytes - sent);
+        hipError_t e = hipMemcpyAsync(c->h_stage + h * c->stage_half, src + sent, n, hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess) e = hipEventRecord(c->stage_ev[h], c->stream);
+        sent += n;
+        return e;
+    };
+    HIPCHK(c, send(0));
+    for (int h = 0; done < bytes; h ^= 1) {
+        if (sent < bytes) HIPCHK(c, send(h ^ 1));
+        HIPCHK(c, hipEventSynchronize(c->stage_ev[h]));
+        const size_t n = std::min(c->stage_half, bytes - done);
+        std::memcpy(dst + done, c->h_stage + h * c->stage_half, n);
+        done += n;
+    }
     return 0;
 }
 
@@ -1069,7 +1132,7 @@ extern "C" int plis_get_state(plis_ctx* c, int32_t r, uint32_t* x) {
     if (int rc = pull_ctl(c)) return rc;
     const RealInfo& ri = c->info[r];
     const uint32_t* X = c->ctl_host[r].cur ? c->d_x1 : c->d_x0;
-    HIPCHK(c, hipMemcpy(x, X + ri.x_off, (size_t)c->S * ri.N * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    if (int rc = fetch(c, x, X + ri.x_off, (size_t)c->S * ri.N * sizeof(uint32_t))) return rc;
     return PLIS_OK;
 }
 
@@ -1130,8 +1193,7 @@ extern "C" int plis_checkpoint(plis_ctx* c, void* buf, uint64_t bytes) {
     for (uint32_t r = 0; r < c->nreal; ++r) {
         const RealInfo& ri = c->info[r];
         const uint32_t* X = c->ctl_host[r].cur ? c->d_x1 : c->d_x0;
-        HIPCHK(c, hipMemcpy(p + 4ull * ri.x_off, X + ri.x_off, (size_t)c->S * ri.N * sizeof(uint32_t),
-                            hipMemcpyDeviceToHost));
+        if (int rc = fetch(c, p + 4ull * ri.x_off, X + ri.x_off, (size_t)c->S * ri.N * sizeof(uint32_t))) return rc;
     }
     return PLIS_OK;
 }
@@ -1181,6 +1243,7 @@ extern "C" int plis_restore(plis_ctx* c, const void* buf, uint64_t bytes) {
     HIPCHK(c, hipMemcpy(c->d_x0, p, c->total_counts * sizeof(uint32_t), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_ctl, ctl.data(), ctl.size() * sizeof(RealCtl), hipMemcpyHostToDevice));
     c->ctl_host = ctl;
+    c->ctl_fresh = true;
     return PLIS_OK;
 }
 

@@ -9,6 +9,7 @@
 namespace plis {
 
 constexpr uint32_t kResidentQueue = 192;  // queued draws per wavefront
+constexpr uint32_t kResidentMaxN = 16384; // subvolumes of a realization, whatever the network
 constexpr uint32_t kResidentLdsMax = 160u * 1024u - 2048u;  // dynamic LDS, next to the kernel's own
 
 struct ResidentArgs {

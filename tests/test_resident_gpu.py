@@ -52,6 +52,9 @@ def _case(name):
     if name == "asymmetric":
         t = H.asym_topology(90, 4)
         return abc, [t], [W.poisson_state(3, 90, 30.0, 5)], 0.03
+    if name == "mixed":  # symmetric, weighted, asymmetric and symmetric again in one context
+        ts = [_grid(5, 4, 2), W.random_mesh(4, 4, 4, 3), H.asym_topology(70, 2), _grid(4, 4, 4)]
+        return abc, ts, [W.poisson_state(3, t["N"], 30.0, 5 + i) for i, t in enumerate(ts)], 0.03
     if name == "order3":
         net, t, x = H.third_order_case()
         return net, [t], [x], 0.03
@@ -86,7 +89,7 @@ def _case(name):
 
 
 CASES = ["abc_1", "abc_2", "abc_63", "abc_64", "abc_65", "abc_129", "uneven", "low", "leapback", "compartments",
-         "asymmetric", "order3", "mesh", "large_means", "dense", "no_reactions", "topology_outside_lds", "many_species",
+         "asymmetric", "mixed", "order3", "mesh", "large_means", "dense", "no_reactions", "topology_outside_lds", "many_species",
          "many_species_compartments", "arrays_outside_lds"]
 
 
