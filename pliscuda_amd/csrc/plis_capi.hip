@@ -82,13 +82,15 @@ struct plis_ctx {
     RealInfo* d_info = nullptr;
     RealCtl* d_ctl = nullptr;
     TileEnt* d_tiles = nullptr;
-    uint32_t *d_x0 = nullptr, *d_x1 = nullptr;
+    uint32_t* d_x = nullptr;  // count buffers, total_counts each: 4 for the edge-parallel leap, else 2
     uint32_t *d_rp = nullptr, *d_col = nullptr, *d_irp = nullptr, *d_icol = nullptr;
     double* d_wsum = nullptr;  // per subvolume, row_ptr layout
     uint32_t* d_frp = nullptr;  // forward CSR: row pointers
     uint64_t* d_fcw = nullptr;  // its entries: neighbour id, row's index in its tile, weight
     float* d_frw = nullptr;     // weights of the hops back, if some topology is not symmetric
-    unsigned long long* d_gdelta = nullptr;        // leap balances, counts layout
+    unsigned long long* d_gdelta = nullptr;  // wide leap balances, counts layout
+    uint32_t* d_wide = nullptr;              // tiles that hold one
+    int32_t narrow = 2048;
     float *d_w = nullptr, *d_iw = nullptr;
     uint64_t *d_cw = nullptr, *d_icw = nullptr;  // interleaved id + weight
     int32_t* d_comp = nullptr;
@@ -354,8 +356,10 @@ static KernelArgs make_args(plis_ctx* c) {
     a.tiles = c->d_tiles;
     a.ntiles = c->ntiles;
     a.nreal = c->nreal;
-    a.x0 = c->d_x0;
-    a.x1 = c->d_x1;
+    a.x = c->d_x;
+    a.x_stride = c->total_counts;
+    a.ep = c->edge_parallel ? 1u : 0u;
+    a.finish_in_tau = c->edge_parallel && !c->learned_on && !(c->theta > 0.0) ? 1u : 0u;
     a.rp = c->d_rp;
     a.wsum = c->d_wsum;
     a.col = c->d_col;
@@ -377,6 +381,8 @@ static KernelArgs make_args(plis_ctx* c) {
     a.frp = c->d_frp;
     a.frw = c->d_frw;
     a.gdelta = c->d_gdelta;
+    a.wide = c->d_wide;
+    a.narrow = c->narrow;
     a.redo_total = reinterpret_cast<unsigned long long*>(c->d_cnt + 2);
     a.count_redo = c->edge_parallel && !c->d_frw ? 1u : 0u;
     a.epsilon = c->eps;
@@ -396,6 +402,8 @@ static KernelArgs make_args(plis_ctx* c) {
     a.mlp_norm = c->d_norm;
     return a;
 }
+
+static uint32_t* count_buf(plis_ctx* c, uint32_t i) { return c->d_x + (uint64_t)i * c->total_counts; }
 
 static const int kVariantS[] = {1, 3, 5, 8, 64};
 static const int kVariantR[] = {4, 4, 8, 16, 128};
@@ -429,12 +437,14 @@ static void launch_step(plis_ctx* c, const KernelArgs& a) {
         for (int k = 0; k < 4; ++k) launch_kernel(c, k, a);
 }
 
-// Before the first iteration of a call in the folded order: the tau pass on
+// Before the first iteration of a call: the edge-parallel leap's target
+// buffer and, in the folded order, the tau pass on
 // the current counts and the decision, which each folded iteration makes
 // for the next one at its end.  Recomputing a decision that is already in
 // place gives the same values (every input is the same), so a call may
 // always start with it.
 static void launch_prologue(plis_ctx* c, const KernelArgs& a) {
+    if (c->edge_parallel) launch_kernel(c, 7, a);
     if (!folded(c)) return;
     launch_kernel(c, 0, a);
     launch_kernel(c, 1, a);
@@ -582,6 +592,7 @@ static bool resident(const plis_ctx* c) { return c->resident_fits && !c->learned
 static int resident_iters(plis_ctx* c, uint32_t n) {
     ResidentArgs a = c->res;
     a.k = make_args(c);
+    a.k.ep = 0u;  // two count buffers
     c->ctl_fresh = false;
     // (a launch makes at most 4,096 iterations, some tens of milliseconds)
     while (n > 0) {
@@ -710,6 +721,12 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
             }
         }
         hfrp.push_back((uint32_t)(hfcw.size() - ri.fe_off));
+        // a subvolume's balances below `narrow` must add up to less than 2^31:
+        // it takes part in at most two hops of a species per neighbour, 16
+        // reactions and the critical event, (2 deg + 17) (narrow - 1) < 2^31
+        // (16 for a subvolume with a sixteenth of the widest id range's links)
+        for (uint32_t v = 0; v < N; ++v)
+            if ((uint64_t)g.rp[v + 1] - g.rp[v] + (sym ? 0u : in.rp[v + 1] - in.rp[v]) >= 1u << 19) c->narrow = 16;
         if (N > kFwdIdMask) huge_tile = true;  // ids take 26 bits of a forward entry
         for (uint32_t v = 0; v < N; v += kTile)  // entry offsets of a tile's queue codes
             if (hfrp[rpoff + std::min(v + (uint32_t)kTile, N)] - hfrp[rpoff + v] >= kMaxTileEdges) huge_tile = true;
@@ -795,13 +812,15 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         rc.t_pause = __builtin_huge_val();
         rc.done = 1u;
         rc.ev_idx = -1;
+        rc.tgt = 1u;
     }
+    const bool ep = !huge_tile && c->variant <= 3;
     int rc = 0;
     std::vector<uint32_t> zeros_cnt(4, 0u);
     if ((rc = upload(c, &c->d_net_i, I)) || (rc = upload(c, &c->d_net_d, D)) ||
         (rc = upload(c, &c->d_info, c->info)) || (rc = upload(c, &c->d_ctl, c->ctl_host)) ||
-        (rc = upload(c, &c->d_tiles, tiles)) || (rc = upload(c, &c->d_x0, hx)) ||
-        (rc = dev_alloc(c, &c->d_x1, hx.size())) || (rc = upload(c, &c->d_rp, hrp)) ||
+        (rc = upload(c, &c->d_tiles, tiles)) ||
+        (rc = dev_alloc(c, &c->d_x, (ep ? 4 : 2) * hx.size())) || (rc = upload(c, &c->d_rp, hrp)) ||
         (rc = upload(c, &c->d_wsum, hwsum)) ||
         (rc = upload(c, &c->d_col, hcol)) ||
         (rc = upload(c, &c->d_w, any_weighted ? hw : std::vector<float>())) ||
@@ -817,9 +836,13 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         plis_destroy(c);
         return rc;
     }
+    if (hipMemcpy(c->d_x, hx.data(), hx.size() * sizeof(uint32_t), hipMemcpyHostToDevice) != hipSuccess) {
+        g_create_err = "copying the counts failed";
+        plis_destroy(c);
+        return PLIS_ERR_HIP;
+    }
     // the forward CSR serves the edge-parallel leap and the resident kernel,
     // the zeroed balances the former
-    const bool ep = !huge_tile && c->variant <= 3;
     const ResLists lists = res_lists(nh, I);
     c->resident_fits = resident_fit(c, nh, D, lists, hfrp, huge_tile);
     if ((ep || c->resident_fits) && ((rc = upload(c, &c->d_frp, hfrp)) || (rc = upload(c, &c->d_fcw, hfcw)))) {
@@ -827,7 +850,8 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         plis_destroy(c);
         return rc;
     }
-    if (ep && ((rc = dev_alloc(c, &c->d_gdelta, hx.size())) || (any_asym && (rc = upload(c, &c->d_frw, hfrw))))) {
+    if (ep && ((rc = dev_alloc(c, &c->d_gdelta, hx.size())) ||
+               (rc = upload(c, &c->d_wide, std::vector<uint32_t>(c->ntiles, 0u))) || (any_asym && (rc = upload(c, &c->d_frw, hfrw))))) {
         g_create_err = c->err;
         plis_destroy(c);
         return rc;
@@ -1122,7 +1146,7 @@ extern "C" int plis_set_state(plis_ctx* c, int32_t r, const uint32_t* x) {
     if (!c || !x || r < 0 || (uint32_t)r >= c->nreal) return PLIS_ERR_ARG;
     if (int rc = pull_ctl(c)) return rc;
     const RealInfo& ri = c->info[r];
-    uint32_t* X = c->ctl_host[r].cur ? c->d_x1 : c->d_x0;
+    uint32_t* X = count_buf(c, c->ctl_host[r].cur);
     HIPCHK(c, hipMemcpy(X + ri.x_off, x, (size_t)c->S * ri.N * sizeof(uint32_t), hipMemcpyHostToDevice));
     return invalidate_props(c);
 }
@@ -1131,7 +1155,7 @@ extern "C" int plis_get_state(plis_ctx* c, int32_t r, uint32_t* x) {
     if (!c || !x || r < 0 || (uint32_t)r >= c->nreal) return PLIS_ERR_ARG;
     if (int rc = pull_ctl(c)) return rc;
     const RealInfo& ri = c->info[r];
-    const uint32_t* X = c->ctl_host[r].cur ? c->d_x1 : c->d_x0;
+    const uint32_t* X = count_buf(c, c->ctl_host[r].cur);
     if (int rc = fetch(c, x, X + ri.x_off, (size_t)c->S * ri.N * sizeof(uint32_t))) return rc;
     return PLIS_OK;
 }
@@ -1192,7 +1216,7 @@ extern "C" int plis_checkpoint(plis_ctx* c, void* buf, uint64_t bytes) {
     p += c->nreal * sizeof(RealCtl);
     for (uint32_t r = 0; r < c->nreal; ++r) {
         const RealInfo& ri = c->info[r];
-        const uint32_t* X = c->ctl_host[r].cur ? c->d_x1 : c->d_x0;
+        const uint32_t* X = count_buf(c, c->ctl_host[r].cur);
         if (int rc = fetch(c, p + 4ull * ri.x_off, X + ri.x_off, (size_t)c->S * ri.N * sizeof(uint32_t))) return rc;
     }
     return PLIS_OK;
@@ -1237,10 +1261,11 @@ extern "C" int plis_restore(plis_ctx* c, const void* buf, uint64_t bytes) {
     p += c->nreal * sizeof(RealCtl);
     for (auto& q : ctl) {
         q.cur = 0u;  // counts go to buffer 0
+        q.tgt = 1u;
         q.prop_ok = 0u;  // the blob holds no tile partials
     }
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    HIPCHK(c, hipMemcpy(c->d_x0, p, c->total_counts * sizeof(uint32_t), hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpy(c->d_x, p, c->total_counts * sizeof(uint32_t), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_ctl, ctl.data(), ctl.size() * sizeof(RealCtl), hipMemcpyHostToDevice));
     c->ctl_host = ctl;
     c->ctl_fresh = true;
@@ -1328,8 +1353,9 @@ extern "C" int plis_debug_poison(plis_ctx* c) {
     if (int rc = pull_ctl(c)) return rc;
     for (uint32_t r = 0; r < c->nreal; ++r) {
         const RealInfo& ri = c->info[r];
-        uint32_t* other = c->ctl_host[r].cur ? c->d_x0 : c->d_x1;
-        HIPCHK(c, hipMemsetD32Async(other + ri.x_off, (int)kPoisonCount, (size_t)c->S * ri.N, c->stream));
+        for (uint32_t i = 0; i < (c->edge_parallel ? 4u : 2u); ++i)
+            if (i != c->ctl_host[r].cur)
+                HIPCHK(c, hipMemsetD32Async(count_buf(c, i) + ri.x_off, (int)kPoisonCount, (size_t)c->S * ri.N, c->stream));
     }
     hipLaunchKernelGGL(poison_parts_kernel, dim3(std::min<uint32_t>((c->ntiles + 255) / 256, 1024u)), dim3(256), 0,
                        c->stream, c->d_pa_t, c->d_pb_t, c->ntiles, c->d_pa_c, c->d_pb_c,

@@ -90,6 +90,16 @@ __device__ __forceinline__ uint32_t wave_uniform(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
 }
 
+// The kernel's arguments (its only parameter) through a pointer made opaque
+// per tile: they and the network tables are loaded where a tile's work uses
+// them instead of being hoisted out of the tile loop into (spilled) scalar
+// registers.
+__device__ __forceinline__ const KernelArgs& tile_args() {
+    cptr<KernelArgs> p = (cptr<KernelArgs>)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const KernelArgs*)p;
+}
+
 // Orders one wavefront's LDS writes before its later LDS reads.
 __device__ __forceinline__ void lds_wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -110,6 +120,19 @@ __device__ __forceinline__ uint32_t tile_at(uint32_t it, uint32_t ntiles, uint32
     const uint32_t ce = (uint32_t)(((uint64_t)ntiles * (xcd + 1u)) >> 3);
     const uint32_t t = cb + lb * wpb + wv + it * nbx * wpb;
     return t < ce ? t : 0xFFFFFFFFu;
+}
+
+__device__ __forceinline__ uint32_t* count_buf(const KernelArgs& a, uint32_t i) {
+    return a.x + (uint64_t)i * a.x_stride;
+}
+
+// The two count buffers that are neither the current nor the target one, in
+// ascending order: the pass after an edge-parallel leap copies the new counts
+// to the first and the old ones to the second.
+__device__ __forceinline__ void spare_bufs(uint32_t cur, uint32_t tgt, uint32_t& z, uint32_t& w) {
+    const uint32_t rest = 0xFu & ~(1u << cur) & ~(1u << tgt);
+    z = (uint32_t)__builtin_ctz(rest);
+    w = 31u - (uint32_t)__builtin_clz(rest);
 }
 
 // an interleaved edge entry's high word for weight 1.0 (a padding entry)
@@ -373,12 +396,9 @@ struct TauAcc {
 };
 
 template <int MS, int MR>
-__device__ __forceinline__ void tau_own(const KernelArgs& a, const NetView& n, const RealInfo& ri,
-                                        const uint32_t* X, uint32_t v, int c, TauAcc<MS>& t) {
-    const uint32_t N = ri.N;
+__device__ __forceinline__ void tau_own(const KernelArgs& a, const NetView& n, const RealInfo& ri, uint32_t v, int c,
+                                        TauAcc<MS>& t) {
     const int nc = a.n_critical;
-#pragma unroll
-    for (int s = 0; s < MS; ++s) t.x[s] = s < n.S ? X[ri.x_off + (uint64_t)s * N + v] : 0u;
     double av[MR];
     uint32_t crit[(MR + 31) / 32];
     react_props<MR, MS>(n, t.x, c, nc, av, crit);
@@ -459,16 +479,18 @@ __device__ __forceinline__ double tau_bound(const KernelArgs& a, const NetView& 
     return tp;
 }
 
-// tau' and the critical propensity of one subvolume, the lane walking its
-// own in-edges.
+// tau' and the critical propensity of one subvolume with counts x, the lane
+// walking its own in-edges.
 template <int MS, int MR>
 __device__ __forceinline__ void tau_subvolume(const KernelArgs& a, const NetView& n, const RealInfo& ri,
-                                              const uint32_t* X, uint32_t v, double& tp_out,
+                                              const uint32_t* X, const uint32_t (&x)[MS], uint32_t v, double& tp_out,
                                               double& a0c_out) {
     const uint32_t N = ri.N;
     const int c = n.C > 1 ? a.comp[ri.comp_off + v] : 0;
     TauAcc<MS> t;
-    tau_own<MS, MR>(a, n, ri, X, v, c, t);
+#pragma unroll
+    for (int s = 0; s < MS; ++s) t.x[s] = x[s];
+    tau_own<MS, MR>(a, n, ri, v, c, t);
     const bool sym = (ri.flags & 1u) != 0;
     // in-edges: neighbour id and weight in one 8-byte load
     const uint64_t* icw = sym ? a.cw + ri.e_off : a.icw + ri.ie_off;
@@ -602,7 +624,7 @@ __device__ void finalize_A(const KernelArgs& a, const NetView& n, const RealInfo
     decide(c);
     // the event is needed only if tau'' <= tau' (a leap-back halves tau' and
     // can lift the clamp to t_end, but never makes a larger tau'' fire)
-    if (t2 < kInf && t2 <= tp) choose_event<MS, MR>(a, n, ri, c, c.cur ? a.x1 : a.x0);
+    if (t2 < kInf && t2 <= tp) choose_event<MS, MR>(a, n, ri, c, count_buf(a, c.cur));
     if (lead) a.ctl[r] = c;
 }
 
@@ -619,20 +641,67 @@ __device__ __forceinline__ void merge_partA(double& tp, double& t2, uint32_t& v2
     }
 }
 
+// Completes the edge-parallel leap at subvolume v of tile t: x and y its counts
+// before and after (y mod 2^32), nx the latter in full; their copies go to the
+// two buffers left over.  Returns whether a count left its range.
+template <int MS>
+__device__ __forceinline__ bool finish_counts(const KernelArgs& a, int S, const RealInfo& ri, uint32_t cur,
+                                              uint32_t tgt, uint32_t t, uint32_t v, uint32_t (&x)[MS],
+                                              uint32_t (&y)[MS], long long (&nx)[MS]) {
+    uint32_t z, w;
+    spare_bufs(cur, tgt, z, w);
+    const uint32_t* X = count_buf(a, cur);
+    const uint32_t* Y = count_buf(a, tgt);
+    uint32_t *Z = count_buf(a, z), *W = count_buf(a, w);
+    const bool wide = wave_uniform(ro(a.wide)[t]) != 0u;
+#pragma unroll
+    for (int s = 0; s < MS; ++s) {
+        const uint64_t at = ri.x_off + (uint64_t)s * ri.N + v;
+        x[s] = s < S ? X[at] : 0u;
+        y[s] = s < S ? Y[at] : 0u;
+    }
+    bool out = false;
+#pragma unroll
+    for (int s = 0; s < MS; ++s) {
+        nx[s] = 0;
+        if (s >= S) continue;
+        const uint64_t at = ri.x_off + (uint64_t)s * ri.N + v;
+        long long b = 0;
+        if (wide) {
+            b = (long long)a.gdelta[at];
+            if (b != 0) a.gdelta[at] = 0ull;
+        }
+        b += (long long)(int32_t)(y[s] - x[s] - (uint32_t)b);
+        nx[s] = (long long)x[s] + b;
+        out = out || nx[s] < 0 || nx[s] > 0xFFFFFFFFll;
+        Z[at] = y[s];
+        W[at] = x[s];
+    }
+    if (wide && (v & 63u) == 0u) a.wide[t] = 0u;  // (a tile's first subvolume: lane 0)
+    return out;
+}
+
 // spec: the counts the leap pass just wrote (the buffer that becomes current
-// if the step is accepted) and the next step's counter.
+// if the step is accepted) and the next step's counter; fin: and completes
+// the leap on the way.  (A kernel of its own between the two passes read
+// counts and 64-bit balances and wrote the new counts: 20 us of the step on
+// the 1M-subvolume Brusselator mesh, 4.4 us where the launch was all of it.)
 template <int MS, int MR>
 __device__ __forceinline__ void cao_tau_tile(const KernelArgs& a, const NetView& n, const RealInfo& ri,
                                              const cptr<RealCtl> cp, const TileEnt& te, uint32_t t, bool dbg,
-                                             bool spec = false) {
+                                             bool spec = false, bool fin = false) {
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t cur = wave_uniform(cp->cur) ^ (spec ? 1u : 0u);
-    const uint32_t* X = cur ? a.x1 : a.x0;
+    const uint32_t cur = wave_uniform(cp->cur), tgt = wave_uniform(cp->tgt);
+    const uint32_t* X = count_buf(a, spec ? tgt : cur);
     const uint32_t v = te.v0 + lane;
     double tp = kInf, t2 = kInf, a0c = 0.0;
     uint32_t v2 = v;
+    bool out = false;
     if (v < ri.N) {
-        tau_subvolume<MS, MR>(a, n, ri, X, v, tp, a0c);
+        uint32_t x[MS];
+#pragma unroll
+        for (int s = 0; s < MS; ++s) x[s] = s < n.S ? X[ri.x_off + (uint64_t)s * ri.N + v] : 0u;
+        tau_subvolume<MS, MR>(a, n, ri, X, x, v, tp, a0c);
         if (a0c > 0.0) {
             const uint32_t step = wave_uniform(cp->step) + (spec ? 1u : 0u);
             const U4 o = philox10(v, kSelfId, step, ctr_word3(ri.id, 0u, kTau2, 0u), a.seed_lo, a.seed_hi);
@@ -646,6 +715,12 @@ __device__ __forceinline__ void cao_tau_tile(const KernelArgs& a, const NetView&
         }
     }
     if (dbg) return;
+    if (fin && v < ri.N) {  // (at the end: nothing of the sums is live any more)
+        uint32_t xo[MS], xn[MS];
+        long long nx[MS];
+        out = finish_counts<MS>(a, n.S, ri, cur, tgt, t, v, xo, xn, nx);
+    }
+    if (fin && __ballot(out) != 0ull && lane == 0) a.partB_tile[t].bad |= 1u;
     reduce_partA(tp, t2, v2);
     if (lane == 0) a.partA_tile[t] = PartA{tp, t2, v2, 0u};
 }
@@ -656,16 +731,12 @@ __device__ __forceinline__ void cao_tau_tile(const KernelArgs& a, const NetView&
 // one-species instantiation measured slower with it, 11.3 -> 12.4 us).
 template <int MS, int MR, bool MC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!MC && MS >= 3 && MS <= 5 ? 8 : 1)))
-void phase_a_kernel(KernelArgs a) {
+void phase_a_kernel(KernelArgs a0) {
     for (uint32_t it = 0;; ++it) {
-        const uint32_t t = tile_at(it, a.ntiles, a.waves_per_block);
+        const uint32_t t = tile_at(it, a0.ntiles, a0.waves_per_block);
         if (t == 0xFFFFFFFFu) break;
-        // the network tables are read through pointers made opaque per tile,
-        // so their scalar loads stay inside the tile's work instead of being
-        // hoisted out of the tile loop into (spilled) scalar registers
-        KernelArgs al = a;
-        asm volatile("" : "+s"(al.net_i), "+s"(al.net_d));
-        const NetView n = net_view<MC>(al);
+        const KernelArgs& a = tile_args();
+        const NetView n = net_view<MC>(a);
         const TileEnt te = ld_ro(a.tiles + t);
         const uint32_t r = wave_uniform(te.r);
         const RealInfo ri = ld_ro(a.info + r);
@@ -676,7 +747,7 @@ void phase_a_kernel(KernelArgs a) {
         // realizations that did not leap are skipped)
         const bool spec = a.tau_spec != 0u && !dbg;
         if (!dbg && (done || (retry && !spec))) continue;
-        cao_tau_tile<MS, MR>(a, n, ri, cp, te, t, dbg, spec);
+        cao_tau_tile<MS, MR>(a, n, ri, cp, te, t, dbg, spec, spec && a.finish_in_tau);
     }
 }
 
@@ -983,9 +1054,9 @@ __device__ __forceinline__ bool leap_subvolume(const KernelArgs& a, const NetVie
 // from the pair's coarse Philox block; then lane i draws the reactions of
 // subvolume v0+i (one coarse block per 16 reactions).
 // Balances of the tile's own subvolumes collect in LDS, those of other
-// tiles' subvolumes go straight to the global balances (gdelta); integer
-// atomics keep every sum exact and order-free.  phase_b_finish_kernel adds
-// the balances to the counts once every draw of the pass is in.
+// tiles' subvolumes go straight to the target buffer, which holds a copy of
+// the counts; integer atomics keep every sum exact and order-free.  The next
+// pass completes the leap (finish_counts) once every draw is in.
 //
 // Compacted draws.  Almost every draw of a step is 0 where hop means are
 // small (~1e-3 on the headline mesh), so the walk only applies the zero
@@ -1041,14 +1112,21 @@ __device__ __forceinline__ float hop_mean_f(double d, uint32_t x, float w, float
     return hop_active(d, x, nc) ? tauf * (((float)d * (float)x) * w) : 0.0f;
 }
 
-// Balance b of species s at subvolume u.  In the tile: 32 bits in LDS for
-// |b| < 2^11 (a row takes part in fewer than 2^20 draws of a pass, so the sum
-// stays below 2^31), else straight to the 64-bit global balance.
+// Balance b of species s at subvolume u: through LDS in the tile, else
+// straight to the target buffer Y (see KernelArgs::gdelta for a wide one).
 template <int MS, bool GEN>
-__device__ __forceinline__ void add_balance(const KernelArgs& a, const RealInfo& ri, LeapLds<MS, GEN>& L, uint32_t v0,
-                                            int s, uint32_t u, long long b) {
-    if (u - v0 < (uint32_t)kTile && b > -2048 && b < 2048) atomicAdd(&L.del[s][u - v0], (int32_t)b);
-    else atomicAdd(&a.gdelta[ri.x_off + (uint64_t)s * ri.N + u], (unsigned long long)b);
+__device__ __forceinline__ void add_balance(const KernelArgs& a, const RealInfo& ri, LeapLds<MS, GEN>& L, uint32_t* Y,
+                                            uint32_t v0, int s, uint32_t u, long long b) {
+    const uint64_t at = ri.x_off + (uint64_t)s * ri.N + u;
+    if (b <= -(long long)a.narrow || b >= (long long)a.narrow) {
+        atomicAdd(&a.gdelta[at], (unsigned long long)b);
+        atomicOr(&a.wide[ri.tile_begin + u / (uint32_t)kTile], 1u);
+        atomicAdd(&Y[at], (uint32_t)b);
+    } else if (u - v0 < (uint32_t)kTile) {
+        atomicAdd(&L.del[s][u - v0], (int32_t)b);
+    } else {
+        atomicAdd(&Y[at], (uint32_t)b);
+    }
 }
 
 // One queued draw: its fine bits complete the word the walk queued the
@@ -1056,8 +1134,8 @@ __device__ __forceinline__ void add_balance(const KernelArgs& a, const RealInfo&
 // applied to the balances.  big: the mean may be 10 or more.
 template <int MS, bool GEN>
 __device__ __forceinline__ void drain_draw(const KernelArgs& a, const NetView& n, const RealInfo& ri,
-                                           const uint32_t* X, uint32_t v0, const StepView& sv, LeapLds<MS, GEN>& L,
-                                           uint32_t eb, uint32_t code, unsigned long long& fire, bool& big) {
+                                           const uint32_t* X, uint32_t* Y, uint32_t v0, const StepView& sv,
+                                           LeapLds<MS, GEN>& L, uint32_t eb, uint32_t code, unsigned long long& fire, bool& big) {
     const bool react = (code & kQueueReact) != 0u;
     const uint32_t hb = code & 255u;
     uint32_t i, c1, w, c3;
@@ -1113,24 +1191,25 @@ __device__ __forceinline__ void drain_draw(const KernelArgs& a, const NetView& n
     if (react) {
         for (int s = 0; s < n.S; ++s) {
             const int nu = n.nu[s * n.R + (int)w];
-            if (nu != 0) add_balance(a, ri, L, v0, s, v0 + i, k * (long long)nu);
+            if (nu != 0) add_balance(a, ri, L, Y, v0, s, v0 + i, k * (long long)nu);
         }
     } else {
         const int s = (int)(w >> 1);
         const long long b = fwd ? -k : k;  // balance of v0 + i
-        add_balance(a, ri, L, v0, s, v0 + i, b);
-        add_balance(a, ri, L, v0, s, c1, -b);
+        add_balance(a, ri, L, Y, v0, s, v0 + i, b);
+        add_balance(a, ri, L, Y, v0, s, c1, -b);
     }
 }
 
-// The draws of one tile into the global balances.  Control flow stays
+// The draws of one tile, and the critical event if it is the tile's, into the
+// target buffer Y.  Control flow stays
 // wave-uniform around every queue append: the loops run the same trip count
 // on every lane, lanes without work carry flags.  Returns whether the tile
 // counts as beyond its queue.  GEN: several compartments or an asymmetric
 // topology.
 template <int MS, int MR, bool GEN>
 __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetView& n, const RealInfo& ri,
-                                                const uint32_t* X, uint32_t v0, const StepView& sv,
+                                                const uint32_t* X, uint32_t* Y, uint32_t v0, const StepView& sv,
                                                 LeapLds<MS, GEN>& L, unsigned long long& fire) {
     static_assert(MS <= 8 && MR <= 16, "one coarse block per pair and per subvolume; hop codes hold w in 4 bits");
     constexpr uint32_t kCap = LeapLds<MS, GEN>::kCap;
@@ -1275,27 +1354,38 @@ __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetVi
         }
         lds_wave_sync();
         for (uint32_t q = lane; q < qn; q += (uint32_t)kTile)
-            drain_draw<MS, GEN>(a, n, ri, X, v0, sv, L, eb, L.q[q], fire, big);
+            drain_draw<MS, GEN>(a, n, ri, X, Y, v0, sv, L, eb, L.q[q], fire, big);
         lds_wave_sync();
         qn = 0u;
+    }
+    if (sv.crit && sv.vstar - v0 < (uint32_t)kTile) {
+        if (v == sv.vstar && (sv.ev_kind == 1 || sv.ev_kind == 2)) {
+            fire += 1ull;
+            if (sv.ev_kind == 1) {
+                for (int s = 0; s < n.S; ++s)
+                    add_balance(a, ri, L, Y, v0, s, v, (long long)n.nu[s * n.R + sv.ev_idx]);
+            } else {
+                add_balance(a, ri, L, Y, v0, sv.ev_idx, v, -1ll);
+                if (sv.ev_dst != v) add_balance(a, ri, L, Y, v0, sv.ev_idx, sv.ev_dst, 1ll);
+            }
+        }
+        lds_wave_sync();
     }
     if (vok) {
 #pragma unroll
         for (int s = 0; s < MS; ++s)
             if (s < n.S && L.del[s][lane] != 0)
-                atomicAdd(&a.gdelta[ri.x_off + (uint64_t)s * N + v], (unsigned long long)(long long)L.del[s][lane]);
+                atomicAdd(&Y[ri.x_off + (uint64_t)s * N + v], (uint32_t)L.del[s][lane]);
     }
     return opened > kQueue || wave_ballot(big) != 0ull;
 }
 
-// The end of the leap pass for one tile: new counts = counts + global
-// balances (which are cleared again), the critical event, the negativity
-// check, the post-leap leap condition (when the judge is on) and the tile's
-// statistics.  nx returns the lane's new counts (any sign).
+// Completes the leap of one tile (finish_counts) where the post-leap leap
+// condition is judged: its violations too.  nx returns the lane's new counts
+// (any sign).
 template <int MS, int MR>
 __device__ __forceinline__ void finish_tile(const KernelArgs& a, const NetView& n, const RealInfo& ri,
-                                            const uint32_t* X, uint32_t* Xn, uint32_t v0, const StepView& sv,
-                                            unsigned long long& fire, uint32_t& bad, uint32_t& viol,
+                                            cptr<RealCtl> cp, uint32_t t, uint32_t v0, uint32_t& bad, uint32_t& viol,
                                             uint32_t (&x)[MS], long long (&nx)[MS], bool judge) {
     const uint32_t v = v0 + (threadIdx.x & 63u);
 #pragma unroll
@@ -1304,28 +1394,8 @@ __device__ __forceinline__ void finish_tile(const KernelArgs& a, const NetView& 
         nx[s] = 0;
     }
     if (v >= ri.N) return;
-    const bool at_star = sv.crit && v == sv.vstar && (sv.ev_kind == 1 || sv.ev_kind == 2);
-    const bool at_dst = sv.crit && sv.ev_kind == 2 && v == sv.ev_dst && sv.ev_dst != sv.vstar;
-    if (at_star) fire += 1ull;
-    bool neg = false;
-#pragma unroll
-    for (int s = 0; s < MS; ++s) {
-        if (s >= n.S) break;
-        const uint64_t at = ri.x_off + (uint64_t)s * ri.N + v;
-        x[s] = X[at];
-        const unsigned long long d = a.gdelta[at];
-        if (d != 0ull) a.gdelta[at] = 0ull;
-        long long y = (long long)x[s] + (long long)d;
-        if (at_star) {
-            if (sv.ev_kind == 1) y += n.nu[s * n.R + sv.ev_idx];
-            else if (s == sv.ev_idx) y -= 1;
-        }
-        if (at_dst && s == sv.ev_idx) y += 1;
-        neg = neg || y < 0 || y > 0xFFFFFFFFll;
-        Xn[at] = (uint32_t)y;
-        nx[s] = y;
-    }
-    bad = neg ? 1u : 0u;
+    uint32_t y[MS];
+    bad = finish_counts<MS>(a, n.S, ri, wave_uniform(cp->cur), wave_uniform(cp->tgt), t, v, x, y, nx) ? 1u : 0u;
     if (judge) {
         const int c = n.C > 1 ? a.comp[ri.comp_off + v] : 0;
         double av[MR];
@@ -1363,6 +1433,8 @@ __device__ bool commit_step(const KernelArgs& a, const RealInfo& ri, unsigned lo
     // step is redone with Cao's tau and fresh draws.
     const double mu = a.viol_rate_max * (double)ri.N;
     const bool learned_reject = c.learned && (bad || (double)viol > mu + 3.0 * sqrt(mu) + 2.0);
+    uint32_t z, w;
+    spare_bufs(c.cur, c.tgt, z, w);
     if (bad || learned_reject) {
         c.attempt += 1u;
         if (learned_reject) {
@@ -1384,12 +1456,15 @@ __device__ bool commit_step(const KernelArgs& a, const RealInfo& ri, unsigned lo
             c.retry = 1u;
         }
         c.prop_ok = 0u;
+        if (a.ep) c.tgt = w;
         return false;
     }
     // the leap pass of a learned context proposed the next step's tau from
     // the state it produced (edge-parallel pass only)
     c.prop_ok = a.props_in_finish ? 1u : 0u;
-    c.cur ^= 1u;
+    const uint32_t old = c.cur;
+    c.cur = c.tgt;
+    c.tgt = a.ep ? z : old;
     c.t = c.last ? c.t_end : c.t + c.tau;
     c.step += 1u;
     c.steps += 1;
@@ -1430,9 +1505,8 @@ __device__ __forceinline__ StepView step_view(const RealInfo& ri, cptr<RealCtl> 
     return sv;
 }
 
-// The leap pass.  EP: the draws of every tile into the global balances; the
-// tile's firings go to its partial and phase_b_finish_kernel completes the
-// leap.  Otherwise one lane walks one subvolume's out- and in-edges and
+// The leap pass.  EP: the draws of every tile into the target buffer; the
+// tile's firings go to its partial and the next pass completes the leap.  Otherwise one lane walks one subvolume's out- and in-edges and
 // finishes it (networks beyond 8 species or 16 reactions, topologies beyond
 // an entry's or a code's bits).  GEN: several compartments, or (EP) an
 // asymmetric topology.
@@ -1442,32 +1516,30 @@ __device__ __forceinline__ StepView step_view(const RealInfo& ri, cptr<RealCtl> 
 // 83.6 -> 94.5 us), at 4 fewer waves hide the walk's gathers (88 us).
 template <int MS, int MR, bool EP, bool GEN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EP && !GEN && MS <= 5 ? 5 : 1)))
-void phase_b_kernel(KernelArgs a) {
+void phase_b_kernel(KernelArgs a0) {
     const uint32_t wv = wave_uniform(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     __shared__ LeapLds<EP ? MS : 1, GEN> s_l[EP ? 4 : 1];  // (up to 4 waves per block)
     for (uint32_t it = 0;; ++it) {
-        const uint32_t t = tile_at(it, a.ntiles, a.waves_per_block);
+        const uint32_t t = tile_at(it, a0.ntiles, a0.waves_per_block);
         if (t == 0xFFFFFFFFu) break;
-        KernelArgs al = a;  // network tables through per-tile opaque pointers, as in phase_a_kernel
-        asm volatile("" : "+s"(al.net_i), "+s"(al.net_d));
-        const NetView n = net_view<GEN>(al);
+        const KernelArgs& a = tile_args();
+        const NetView n = net_view<GEN>(a);
         const TileEnt te = ld_ro(a.tiles + t);
         const uint32_t r = wave_uniform(te.r);
         const RealInfo ri = ld_ro(a.info + r);
         const cptr<RealCtl> cp = ro(a.ctl + r);
         if (wave_uniform(cp->done)) continue;
         const StepView sv = step_view(ri, cp);
-        const uint32_t cur = wave_uniform(cp->cur);
-        const uint32_t* X = cur ? a.x1 : a.x0;
+        const uint32_t* X = count_buf(a, wave_uniform(cp->cur));
+        uint32_t* Xn = count_buf(a, wave_uniform(cp->tgt));
         unsigned long long fire = 0;
         uint32_t bad = 0, viol = 0;
         if constexpr (EP) {
-            const bool over = leap_tile_draws<MS, MR, GEN>(a, n, ri, X, te.v0, sv, s_l[wv], fire);
+            const bool over = leap_tile_draws<MS, MR, GEN>(a, n, ri, X, Xn, te.v0, sv, s_l[wv], fire);
             reduce_partB(fire, bad, viol);
             if (lane == 0) a.partB_tile[t] = PartB{fire, over && a.count_redo ? 2u : 0u, 0u};
         } else {
             const uint32_t v = te.v0 + lane;
-            uint32_t* Xn = cur ? a.x0 : a.x1;
             if (v < ri.N) bad = leap_subvolume<MS, MR>(a, n, ri, X, Xn, v, sv, fire, viol) ? 1u : 0u;
             reduce_partB(fire, bad, viol);
             if (lane == 0) a.partB_tile[t] = PartB{fire, bad, viol};
@@ -1475,14 +1547,11 @@ void phase_b_kernel(KernelArgs a) {
     }
 }
 
-// The end of the edge-parallel leap pass: every tile adds the global
-// balances to its counts (see finish_tile) after all draws are in.  Up to 5
-// species it fits 8 waves per SIMD (otherwise its scalar registers hold it
-// at 7): more loads in flight for an HBM-bound kernel, 20.9 -> 20.5 us on
-// the Brusselator mesh.
+// The end of the edge-parallel leap pass of plain contexts that judge the
+// post-leap leap condition (a check, off in ordinary runs): finish_tile in a
+// pass of its own, so that the tau pass keeps its registers.
 template <int MS, int MR, bool MC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MS <= 5 ? 8 : 1)))
-void phase_b_finish_kernel(KernelArgs a) {
+__global__ __launch_bounds__(256) void phase_b_finish_kernel(KernelArgs a) {
     const NetView n = net_view<MC>(a);
     const uint32_t lane = threadIdx.x & 63u;
     for (uint32_t it = 0;; ++it) {
@@ -1493,19 +1562,36 @@ void phase_b_finish_kernel(KernelArgs a) {
         const RealInfo ri = ld_ro(a.info + r);
         const cptr<RealCtl> cp = ro(a.ctl + r);
         if (wave_uniform(cp->done)) continue;
-        const StepView sv = step_view(ri, cp);
-        const uint32_t cur = wave_uniform(cp->cur);
         unsigned long long fire = 0;
         uint32_t bad = 0, viol = 0;
         uint32_t x[MS];
         long long nx[MS];
-        finish_tile<MS, MR>(a, n, ri, cur ? a.x1 : a.x0, cur ? a.x0 : a.x1, te.v0, sv, fire, bad, viol, x, nx,
-                            a.judge_on != 0);
+        finish_tile<MS, MR>(a, n, ri, cp, t, te.v0, bad, viol, x, nx, true);
         reduce_partB(fire, bad, viol);
         if (lane == 0) {
             const PartB p = a.partB_tile[t];
-            a.partB_tile[t] = PartB{p.fire + fire, merge_bad(p.bad, bad), viol};
+            a.partB_tile[t] = PartB{p.fire, merge_bad(p.bad, bad), viol};
         }
+    }
+}
+
+// Copies every running realization's counts to its target buffer, where the
+// next edge-parallel leap adds its balances (the first kernel of a call: what
+// was done to the buffers between calls does not matter).
+static __global__ __launch_bounds__(256) void sync_target_kernel(KernelArgs a) {
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint32_t it = 0;; ++it) {
+        const uint32_t t = tile_at(it, a.ntiles, a.waves_per_block);
+        if (t == 0xFFFFFFFFu) break;
+        const TileEnt te = ld_ro(a.tiles + t);
+        const uint32_t r = wave_uniform(te.r);
+        const RealInfo ri = ld_ro(a.info + r);
+        const cptr<RealCtl> cp = ro(a.ctl + r);
+        const uint32_t v = te.v0 + lane;
+        if (wave_uniform(cp->done) || v >= ri.N) continue;
+        const uint32_t* X = count_buf(a, wave_uniform(cp->cur)) + ri.x_off;
+        uint32_t* Y = count_buf(a, wave_uniform(cp->tgt)) + ri.x_off;
+        for (int s = 0; s < a.nh.S; ++s) Y[(uint64_t)s * ri.N + v] = X[(uint64_t)s * ri.N + v];
     }
 }
 

@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256) void learned_tau_kernel(KernelArgs a) {
             continue;
         }
         if (wave_uniform(cp->prop_ok)) continue;
-        const uint32_t* X = wave_uniform(cp->cur) ? a.x1 : a.x0;
+        const uint32_t* X = count_buf(a, wave_uniform(cp->cur));
         const uint32_t v = te.v0 + lane;
         const bool act = v < ri.N;
         uint32_t x[MS];
@@ -212,13 +212,11 @@ __global__ __launch_bounds__(256) void learned_finish_kernel(KernelArgs a) {
         const RealInfo ri = ld_ro(a.info + r);
         const cptr<RealCtl> cp = ro(a.ctl + r);
         if (wave_uniform(cp->done)) continue;
-        const StepView sv = step_view(ri, cp);
-        const uint32_t cur = wave_uniform(cp->cur);
         unsigned long long fire = 0;
         uint32_t bad = 0, viol = 0;
         uint32_t x[MS];
         long long nx[MS];
-        finish_tile<MS, MR>(a, n, ri, cur ? a.x1 : a.x0, cur ? a.x0 : a.x1, te.v0, sv, fire, bad, viol, x, nx, false);
+        finish_tile<MS, MR>(a, n, ri, cp, t, te.v0, bad, viol, x, nx, false);
         const uint32_t v = te.v0 + lane;
         const bool act = v < ri.N;
         const int c = n.C > 1 && act ? a.comp[ri.comp_off + v] : 0;
@@ -237,9 +235,10 @@ __global__ __launch_bounds__(256) void learned_finish_kernel(KernelArgs a) {
         reduce_partB(fire, bad, viol);
         if (lane == 0) {
             const PartB p = a.partB_tile[t];
-            a.partB_tile[t] = PartB{p.fire + fire, merge_bad(p.bad, bad), viol};
+            a.partB_tile[t] = PartB{p.fire, merge_bad(p.bad, bad), viol};
         }
-        propose_tile<MS, MR, ACT>(a, n, ri, W, xn, av1, crit1, act, v, sv.step + 1u, sv.tau, t);
+        propose_tile<MS, MR, ACT>(a, n, ri, W, xn, av1, crit1, act, v,
+                                  wave_uniform(cp->step) + 1u, cp->tau, t);
     }
 }
 
@@ -262,7 +261,7 @@ __global__ __launch_bounds__(256) void records_kernel(KernelArgs a) {
         if (te.r != a.rec_real) continue;
         const RealInfo ri = a.info[te.r];
         const RealCtl* cp = &a.ctl[te.r];
-        const uint32_t* X = cp->cur ? a.x1 : a.x0;
+        const uint32_t* X = count_buf(a, cp->cur);
         const double prev = cp->tau;
         const float prev_logtau = prev > 0.0 ? __logf((float)prev) : 0.0f;
         const uint32_t step = cp->step;
@@ -281,7 +280,7 @@ __global__ __launch_bounds__(256) void records_kernel(KernelArgs a) {
             react_props<MR, MS>(n, x, n.C > 1 ? a.comp[ri.comp_off + v] : 0, a.n_critical, av, crit);
             features_and_crit<MS, MR>(a, n, ri, x, av, crit, v, prev_logtau, f, a0c, live);
         }
-        tau_subvolume<MS, MR>(a, n, ri, X, v, tp, a0c2);
+        tau_subvolume<MS, MR>(a, n, ri, X, x, v, tp, a0c2);
 #pragma unroll
         for (int k = 0; k < 12; ++k) a.rec_feats[(size_t)v * 12 + k] = f[k];
         a.rec_ylog[v] = tp < 1e6 ? (float)dlog(tp) : (float)dlog(1e6);

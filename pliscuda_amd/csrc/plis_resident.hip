@@ -257,7 +257,7 @@ static __global__ __launch_bounds__(1024) void resident_kernel(ResidentArgs ra) 
             V.in = reinterpret_cast<const uint2*>(g_in);
             V.comp = a.comp + ri.comp_off;
         }
-        const uint32_t* X = c0.cur ? a.x1 : a.x0;
+        const uint32_t* X = count_buf(a, c0.cur);
         for (uint32_t i = threadIdx.x; i < S * N; i += blockDim.x) {
             V.x[i] = X[ri.x_off + i];
             V.del[i] = 0ull;
@@ -553,14 +553,14 @@ static __global__ __launch_bounds__(1024) void resident_kernel(ResidentArgs ra) 
         }
         __syncthreads();
         if (s_c.cur != cur) {
-            cur ^= 1u;
+            cur = s_c.cur;
             cb ^= 1u;
         } else {  // leap-back: the propensities of the counts before the step again
             props(V.x);
             __syncthreads();
         }
     }
-    uint32_t* X = s_c.cur ? a.x1 : a.x0;
+    uint32_t* X = count_buf(a, s_c.cur);
     for (uint32_t i = threadIdx.x; i < S * N; i += blockDim.x) X[ri.x_off + i] = xb[cb * S * N + i];
     if (threadIdx.x == 0u) a.ctl[r] = s_c;
 }

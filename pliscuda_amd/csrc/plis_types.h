@@ -1,7 +1,9 @@
 // plis_types.h -- device-resident layout of a batch of RDME realizations.
 //
 // HBM layout (one context = one batch of realizations sharing a reaction network):
-//   counts  : two ping-pong uint32 buffers; realization r occupies
+//   counts  : uint32 buffers, RealCtl::cur the one that holds a realization's
+//             counts, RealCtl::tgt the one its next leap writes; two of them,
+//             or four for the edge-parallel leap; realization r occupies
 //             [x_off, x_off + S*N) species-major ([s*N + v], coalesced per
 //             species like the reference's GET_SPI, PLISCuda/include/cuda/constants.cuh:27)
 //   topology: canonical CSR per realization (row_ptr relative to e_off, col
@@ -60,7 +62,7 @@ struct RealCtl {
     uint64_t steps, leapbacks, firings, subvolume_leaps, crit_events;
     uint32_t step, attempt, vstar, ev_dst;
     int32_t crit, last, ev_kind, ev_idx;
-    uint32_t done, retry, cur;
+    uint32_t done, retry, cur;  // cur: buffer of the counts
     int32_t status;
     // learned tau: this step's tau came from the network / the step after a
     // rejected proposal uses Cao's formula
@@ -69,7 +71,12 @@ struct RealCtl {
     // the tile partials hold the network's proposals for the current state
     // (written by the leap pass that produced it); cleared whenever the
     // state or the network changes otherwise
-    uint32_t prop_ok, pad2;
+    uint32_t prop_ok;
+    // buffer the leap writes.  The edge-parallel leap adds its balances to it,
+    // so it holds a copy of the counts when a leap starts; the pass after the
+    // leap copies the new counts and the old ones to the two buffers left
+    // over, the target after an accepted step and after a leap-back
+    uint32_t tgt;
 };
 
 struct TileEnt {
@@ -95,8 +102,10 @@ struct KernelArgs {
     const TileEnt* tiles;
     uint32_t ntiles;
     uint32_t nreal;
-    uint32_t* x0;
-    uint32_t* x1;
+    uint32_t* x;             // count buffers, x_stride elements each
+    uint64_t x_stride;
+    uint32_t ep;             // the leap pass is the edge-parallel one
+    uint32_t finish_in_tau;  // the tau pass on the new counts completes the leap
     const uint32_t* rp;
     const double* wsum;       // sum of out-edge weights per subvolume (row_ptr layout)
     const uint32_t* col;
@@ -118,15 +127,21 @@ struct KernelArgs {
     PartB* partB_tile;
     uint32_t* ndone;
     // forward CSR (row_ptr layout of rp; entries v -> u with u > v) and the
-    // leap pass's global per-subvolume balances (counts layout, zero between
-    // passes).  An entry is one 8-byte word: u in bits 0..25, the index of
+    // leap pass's balances.  An entry is one 8-byte word: u in bits 0..25, the index of
     // its row v within v's tile in bits 26..31, the weight's float bits in
     // the high word (1.0 unweighted); realizations of the edge-parallel
     // pass have fewer than 2^26 subvolumes.
     const uint32_t* frp;
     const uint64_t* fcw;
     const float* frw;         // asymmetric topologies: weights of the hops back (entries' upper to lower ends)
+    // A leap's balances are added to the target buffer mod 2^32.  Those of
+    // `narrow` molecules or more are added to gdelta too (counts layout, 64
+    // bits, zero between passes) and mark the subvolume's tile in wide: the
+    // rest of a subvolume's balance fits 32 bits, so the difference of the two
+    // buffers gives it back.
     unsigned long long* gdelta;
+    uint32_t* wide;
+    int32_t narrow;
     unsigned long long* redo_total;  // tiles beyond a wavefront's queue since the context was made
     uint32_t count_redo;             // those tiles are counted
     double epsilon;

@@ -13,7 +13,7 @@ namespace plis {
 // Kernel groups: 0 tau pass (learned and/or Cao), 1 decide, 2 leap pass,
 // 3 commit; 4 tau pass on the counts the leap pass wrote and 6 commit +
 // decide (the folded order of plain tau); 5 = training records of one
-// realization.  In a learned
+// realization; 7 = the target buffer before a call's first leap.  In a learned
 // context the end of the edge-parallel leap pass also proposes the next
 // step's tau (learned_finish_kernel); learned_tau_kernel covers the steps
 // whose proposals it could not make.
@@ -43,6 +43,7 @@ void launch_variant(const LaunchEnv& c, int which, const KernelArgs& a) {
                     else hipLaunchKernelGGL((phase_b_kernel<MS, MR, true, false>), grid, block, 0, c.stream, a);
                     if (c.split_ev) (void)hipEventRecord(*c.split_ev, c.stream);
                     if (c.learned_on) launch_learned<MS, MR>(c, kLearnedFinish, a);
+                    else if (!a.judge_on) break;
                     else if (mc) hipLaunchKernelGGL((phase_b_finish_kernel<MS, MR, true>), grid, block, 0, c.stream, a);
                     else hipLaunchKernelGGL((phase_b_finish_kernel<MS, MR, false>), grid, block, 0, c.stream, a);
                     break;
@@ -61,6 +62,9 @@ void launch_variant(const LaunchEnv& c, int which, const KernelArgs& a) {
             else hipLaunchKernelGGL((phase_a_kernel<MS, MR, false>), grid, block, 0, c.stream, as);
             break;
         }
+        case 7:  // before a call's first step: the leap's target buffer
+            hipLaunchKernelGGL(sync_target_kernel, grid, block, 0, c.stream, a);
+            break;
         case 6:  // folded order: commit and decide
             hipLaunchKernelGGL((commit_decide_kernel<MS, MR>), dgrid, dblock, 0, c.stream, a);
             break;

@@ -1,0 +1,74 @@
+"""The edge-parallel leap adds its balances to a copy of the counts and the pass
+after it completes the leap: wide balances, ranges of the target buffers over
+leap-backs and split calls, critical events at tile borders, a hub whose links
+bound the balances.  All against the oracle, bit for bit, on contexts too large
+for the one-block kernel."""
+import numpy as np
+import pytest
+
+from oracle import ffi
+from pliscuda_amd import capi
+from pliscuda_amd import workloads as W
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(net, topo, x0, eps, nc, seed, calls, **expect):
+    ctx = capi.Context(net, [topo], [x0], eps=eps, nc=nc, seed=seed)
+    made = 0
+    for n in calls:
+        made += n
+        ctx.run(np.inf, step_limit=made)
+    x = np.array(x0, dtype=np.uint32).copy()
+    st = ffi.run(ffi.Model(net, topo), x, eps, nc, seed, np.inf, step_limit=made)
+    g, gs = ctx.get_state(0), ctx.stats(0)
+    ctx.close()
+    assert np.array_equal(g, x)
+    for f in ("steps", "leapbacks", "firings", "crit_events", "t", "status"):
+        assert gs[f] == getattr(st, f), f
+    for f, lo in expect.items():
+        assert gs[f] >= lo, f
+
+
+@pytest.mark.parametrize("count", [300_000, 2_000_000_000, 4_294_000_000])
+def test_wide_balances(count):
+    """Draws of thousands to millions of molecules; at the end counts past 2^31 and near 2^32."""
+    topo = W.cubic_grid(13, 11, 15, periodic=False)
+    x0 = W.uniform_state(topo["N"], count - 1000, count + 1000, 3)
+    net = W.network(["A"], [({"A": 1}, {"A": 1})], [0.0], [5.0])
+    _check(net, topo, x0, 0.05, 10, 4, [3, 4])
+
+
+def test_wide_and_narrow_species():
+    topo = W.random_mesh(16, 12, 12, 9)
+    net = W.brusselator_network(W.SEED_BRUSS)
+    x0 = W.poisson_state(5, topo["N"], [2e5, 30, 5e4, 100, 12], 6)
+    _check(net, topo, x0, 0.03, 10, 5, [6, 1, 5])
+
+
+@pytest.mark.parametrize("asym", [False, True])
+def test_leapbacks(asym):
+    net = W.abc_network()
+    topo = H.asym_topology(2000, 3) if asym else W.cubic_grid(13, 13, 11, periodic=False)
+    x0 = W.poisson_state(3, topo["N"], [2.0, 2.0, 1.0], 8)
+    _check(net, topo, x0, 0.9, 0, 9, [5, 1, 1, 18], leapbacks=3)
+
+
+def test_critical_events():
+    net = W.abc_network()
+    topo = W.cubic_grid(13, 13, 11, periodic=False)
+    x0 = W.poisson_state(3, topo["N"], [11.0, 11.0, 9.0], 8)
+    _check(net, topo, x0, 0.03, 10, 9, [30, 1, 29], crit_events=30)
+
+
+def test_hub():
+    """Every subvolume linked to the last one: its links bound the balances."""
+    N = (1 << 19) + 70
+    hub = np.full(N - 1, N - 1, dtype=np.int64)
+    leaf = np.arange(N - 1, dtype=np.int64)
+    topo = W.csr_from_edges(N, np.concatenate([leaf, hub]), np.concatenate([hub, leaf]), np.ones(2 * (N - 1)))
+    net = W.network(["A"], [({"A": 1}, {"A": 1})], [0.0], [0.5])
+    x0 = W.uniform_state(N, 500, 900, 3)
+    x0[N - 1] = 400_000_000
+    _check(net, topo, x0, 0.5, 10, 4, [2, 2])
