@@ -1541,13 +1541,14 @@ static int upload_records(plis_ctx* c, const float* feats, const float* ylog, co
 }
 
 static void train_launch(plis_ctx* c, uint64_t n, uint32_t batch, uint32_t step, uint64_t seed, int full,
-                         int32_t adam_t, float lr) {
+                         int32_t adam_t, float lr, float* loss) {
     TrainArgs ta;
     ta.m = MlpDev{c->d_w32, c->d_q, c->d_norm};
     ta.feats = c->d_rf;
     ta.ylog = c->d_ry;
     ta.ycrit = c->d_rc;
     ta.n = n;
+    ta.n_inv = ~0ull / n;
     ta.batch = batch;
     ta.step = step;
     ta.seed_lo = (uint32_t)seed;
@@ -1555,13 +1556,11 @@ static void train_launch(plis_ctx* c, uint64_t n, uint32_t batch, uint32_t step,
     ta.full_pass = full;
     ta.partial = c->d_partial;
     const uint32_t blocks = std::min<uint32_t>(c->train_blocks, batch / 64);
-    if (c->mlp_act == 1) hipLaunchKernelGGL(mlp_train_kernel<1>, dim3(blocks), dim3(64), 0, c->stream, ta);
-    else hipLaunchKernelGGL(mlp_train_kernel<0>, dim3(blocks), dim3(64), 0, c->stream, ta);
-    AdamArgs aa{c->d_w32, c->d_m, c->d_v, c->d_grad, c->d_partial, blocks, adam_t, lr, 0.9f, 0.999f, 1e-8f};
+    if (c->mlp_act == 1) hipLaunchKernelGGL(mlp_train_kernel<1>, dim3(blocks), dim3(256), 0, c->stream, ta);
+    else hipLaunchKernelGGL(mlp_train_kernel<0>, dim3(blocks), dim3(256), 0, c->stream, ta);
+    AdamArgs aa{c->d_w32, c->d_m, c->d_v, c->d_grad, loss, c->d_q, c->d_partial, blocks, adam_t, lr, 0.9f, 0.999f, 1e-8f};
     hipLaunchKernelGGL(mlp_adam_kernel, dim3((kPTotal + 1 + kAdamParams - 1) / kAdamParams), dim3(256), 0,
                        c->stream, aa);
-    if (adam_t > 0)
-        hipLaunchKernelGGL(mlp_pack_kernel, dim3((kQTotal + 255) / 256), dim3(256), 0, c->stream, c->d_w32, c->d_q);
 }
 
 extern "C" int plis_mlp_loss_grad(plis_ctx* c, const float* feats, const float* ylog, const float* ycrit, uint32_t n,
@@ -1575,7 +1574,7 @@ extern "C" int plis_mlp_loss_grad(plis_ctx* c, const float* feats, const float* 
         return PLIS_ERR_STATE;
     }
     if (int rc = upload_records(c, feats, ylog, ycrit, n)) return rc;
-    train_launch(c, n, n, 0, 0, 1, 0, 0.0f);
+    train_launch(c, n, n, 0, 0, 1, 0, 0.0f, nullptr);
     HIPCHK(c, hipGetLastError());
     std::vector<float> g(kPTotal + 1);
     HIPCHK(c, hipMemcpyAsync(g.data(), c->d_grad, (kPTotal + 1) * sizeof(float), hipMemcpyDeviceToHost, c->stream));
@@ -1598,11 +1597,8 @@ extern "C" int plis_mlp_train(plis_ctx* c, const float* feats, const float* ylog
     if (int rc = upload_records(c, feats, ylog, ycrit, n)) return rc;
     float* d_losses = nullptr;
     if (losses) HIPCHK(c, hipMalloc((void**)&d_losses, (size_t)steps * sizeof(float)));
-    for (uint32_t t = 0; t < steps; ++t) {
-        train_launch(c, n, batch, t, seed, 0, ++c->adam_t, lr);
-        if (d_losses)
-            (void)hipMemcpyAsync(d_losses + t, c->d_grad + kPTotal, sizeof(float), hipMemcpyDeviceToDevice, c->stream);
-    }
+    for (uint32_t t = 0; t < steps; ++t)
+        train_launch(c, n, batch, t, seed, 0, ++c->adam_t, lr, d_losses ? d_losses + t : nullptr);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e == hipSuccess && losses) {

@@ -20,6 +20,9 @@
 namespace plis {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kNin = 16, kNh = 64, kNo = 2, kNoPad = 32;
@@ -78,95 +81,41 @@ __device__ __forceinline__ float act_d(float z) {
 // row (l % 32) starting at k = 8*(l/32); B fragment = 8 consecutive k of
 // column (l % 32); accumulator element i of lane l sits at
 // row 8*(i/4) + 4*(l/32) + i%4, column l % 32.
-__device__ __forceinline__ bf16x8 lds_frag(const __bf16* M, int ld, int row0, int k0) {
-    const int l = threadIdx.x & 63;
+__device__ __forceinline__ bf16x8 lds_frag(const __bf16* M, int ld, int row0, int k0,
+                                           int l = threadIdx.x & 63) {
     return *reinterpret_cast<const bf16x8*>(M + (row0 + (l & 31)) * ld + k0 + 8 * (l >> 5));
 }
-__device__ __forceinline__ bf16x8 glb_frag(const __bf16* M, int ld, int row0, int k0) {
-    const int l = threadIdx.x & 63;
+__device__ __forceinline__ bf16x8 glb_frag(const __bf16* M, int ld, int row0, int k0,
+                                           int l = threadIdx.x & 63) {
     return *reinterpret_cast<const bf16x8*>(M + (row0 + (l & 31)) * ld + k0 + 8 * (l >> 5));
 }
 __device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ int acc_row(int i) { return 8 * (i >> 2) + 4 * ((threadIdx.x & 63) >> 5) + (i & 3); }
-__device__ __forceinline__ int acc_col() { return threadIdx.x & 31; }
+__device__ __forceinline__ int acc_row(int i, int l = threadIdx.x & 63) { return 8 * (i >> 2) + 4 * (l >> 5) + (i & 3); }
+__device__ __forceinline__ int acc_col(int l = threadIdx.x & 63) { return l & 31; }
 
+// One training tile's staging: 39,680 bytes, so that four blocks share a CU.
+// Row-major activations serve only the next layer of the forward pass; the
+// backward pass stages its gradients in their place.
 struct MlpLds {
-    __bf16 x[64 * kLdX];      // standardised inputs [row][16]
-    __bf16 xt[16 * kLdH];     // transposed [feature][row]
-    __bf16 h1[64 * kLdH], h1t[64 * kLdH];
-    __bf16 h2[64 * kLdH], h2t[64 * kLdH];
-    __bf16 dz[64 * kLdH], dzt[64 * kLdH];
-    __bf16 g1[64 * kLdH], g2[64 * kLdH];  // act'(z) of the hidden layers
+    __bf16 xt[kNin * kLdH];    // standardised inputs, transposed [feature][row]
+    __bf16 h1t[64 * kLdH];     // hidden activations, transposed [unit][row]
+    union {
+        __bf16 x[64 * kLdX];   // inputs [row][16] (until layer 1 is done)
+        __bf16 h2t[64 * kLdH];
+    };
+    union {
+        __bf16 h1[64 * kLdH];  // [row][unit] (until layer 2 is done)
+        __bf16 dzt[64 * kLdH];
+    };
+    union {
+        __bf16 h2[64 * kLdH];  // (until the output layer is done)
+        __bf16 dz[64 * kLdH];
+    };
     float out[64 * 2];
 };
-
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Standardise lane's feature row into LDS row r (stride ld; lane r owns row r).
-__device__ __forceinline__ void stage_inputs(__bf16* x, __bf16* xt, const MlpDev& m, const float (&f)[12],
-                                             bool valid, int ld = kLdX) {
-    const int r = threadIdx.x & 63;
-#pragma unroll
-    for (int k = 0; k < kNin; ++k) {
-        float z = 0.0f;
-        if (k < 12 && valid) z = (f[k] - m.norm[k]) * (1.0f / m.norm[12 + k]);
-        const __bf16 b = (__bf16)z;
-        x[r * ld + k] = b;
-        if (xt) xt[k * kLdH + r] = b;
-    }
-}
-
-// One dense layer on the 64-row tile: out[64][N] = act(in[64][K] . W + b).
-// Writes bf16 activations (row-major and transposed) and, for the hidden
-// layers, act'(z) in bf16 (g) for the backward pass.
-template <int K, int NB, bool ACTON, int ACT>
-__device__ __forceinline__ void dense(const __bf16* in, int ldin, const __bf16* wt, const float* bias,
-                                      __bf16* h, __bf16* ht, __bf16* g, float* out2) {
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            f32x16 c = {};
-#pragma unroll
-            for (int kb = 0; kb < K / 16; ++kb)
-                c = mfma(lds_frag(in, ldin, mb * 32, kb * 16), glb_frag(wt, K, nb * 32, kb * 16), c);
-            const int col = nb * 32 + acc_col();
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int row = mb * 32 + acc_row(i);
-                if (ACTON) {
-                    const float z = c[i] + bias[col];
-                    const __bf16 a = (__bf16)act_f<ACT>(z);
-                    h[row * kLdH + col] = a;
-                    if (ht) ht[col * kLdH + row] = a;
-                    g[row * kLdH + col] = (__bf16)act_d<ACT>(z);
-                } else if (col < kNo) {
-                    out2[row * 2 + col] = c[i] + bias[col];
-                }
-            }
-        }
-}
-
-// Forward pass of the tile; returns the lane's two outputs.
-template <int ACT>
-__device__ __forceinline__ void mlp_forward_tile(MlpLds& s, const MlpDev& m, float& o0, float& o1) {
-    wave_sync();
-    dense<16, 2, true, ACT>(s.x, kLdX, m.q + kQW1t, m.w32 + kPB1, s.h1, s.h1t, s.g1, nullptr);
-    wave_sync();
-    dense<64, 2, true, ACT>(s.h1, kLdH, m.q + kQW2t, m.w32 + kPB2, s.h2, s.h2t, s.g2, nullptr);
-    wave_sync();
-    dense<64, 1, false, ACT>(s.h2, kLdH, m.q + kQW3t, m.w32 + kPB3, nullptr, nullptr, nullptr, s.out);
-    wave_sync();
-    const int r = threadIdx.x & 63;
-    o0 = s.out[r * 2];
-    o1 = s.out[r * 2 + 1];
-}
+static_assert(4 * sizeof(MlpLds) <= 160 * 1024, "four blocks per CU");
 
 // ---------------------------------------------------------------------------
 // training: forward + backward over tiles of 64 samples, per-wave gradient
@@ -177,7 +126,7 @@ struct TrainArgs {
     const float* feats;      // [n][12]
     const float* ylog;       // [n] standardised log tau target
     const float* ycrit;      // [n] 0/1
-    uint64_t n;              // records
+    uint64_t n, n_inv;       // records; floor((2^64 - 1) / n)
     uint32_t batch;          // samples per step (multiple of 64)
     uint32_t step;           // selects the minibatch
     uint32_t seed_lo, seed_hi;
@@ -185,158 +134,217 @@ struct TrainArgs {
     float* partial;          // [gridDim.x][kPTotal + 1] (last = loss sum)
 };
 
+// The 32x32 block (mb, nb) of in[64][K] . W, W given transposed as fragments.
+template <int K>
+__device__ __forceinline__ f32x16 mfma_block(const __bf16* in, int ldin, int mb, int l, const bf16x8 (&w)[K / 16]) {
+    f32x16 c = {};
+#pragma unroll
+    for (int kb = 0; kb < K / 16; ++kb) c = mfma(lds_frag(in, ldin, mb * 32, kb * 16, l), w[kb], c);
+    return c;
+}
+
+template <int K>
+__device__ __forceinline__ void load_frags(const __bf16* wt, int nb, int l, bf16x8 (&w)[K / 16]) {
+#pragma unroll
+    for (int kb = 0; kb < K / 16; ++kb) w[kb] = glb_frag(wt, K, nb * 32, kb * 16, l);
+}
+
+// Four consecutive rows of a column at once (an accumulator holds them).
+__device__ __forceinline__ void store4(__bf16* p, const bf16x4& v) { *reinterpret_cast<bf16x4*>(p) = v; }
+
+// A hidden layer's block: bf16 activations (row-major and transposed); d
+// keeps act'(z), rounded to bf16, for the backward pass of the same block.
 template <int ACT>
-__global__ __launch_bounds__(64) void mlp_train_kernel(TrainArgs a) {
+__device__ __forceinline__ void activate_block(const f32x16& c, float bias, int mb, int nb, int l, __bf16* h, __bf16* ht,
+                                               u32x8& d) {
+    const int col = nb * 32 + acc_col(l);
+    bf16x16 g;
+    bf16x4 t;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int row = mb * 32 + acc_row(i, l);
+        const float z = c[i] + bias;
+        t[i & 3] = (__bf16)act_f<ACT>(z);
+        h[row * kLdH + col] = t[i & 3];
+        if ((i & 3) == 3) store4(ht + col * kLdH + row - 3, t);
+        g[i] = (__bf16)act_d<ACT>(z);
+    }
+    // formed here: sunk to their use, they would keep z live instead
+    d = __builtin_bit_cast(u32x8, g);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(d[i]));
+}
+
+__device__ __forceinline__ void grad_block(const f32x16& c, const u32x8& d, int mb, int nb, int l, MlpLds& s) {
+    const int col = nb * 32 + acc_col(l);
+    const bf16x16 g = __builtin_bit_cast(bf16x16, d);
+    bf16x4 t;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int row = mb * 32 + acc_row(i, l);
+        t[i & 3] = (__bf16)(c[i] * (float)g[i]);
+        s.dz[row * kLdH + col] = t[i & 3];
+        if ((i & 3) == 3) store4(s.dzt + col * kLdH + row - 3, t);
+    }
+}
+
+// One 64-sample tile per block of four wavefronts.  Wavefront (mb, nb) forms
+// the same 32x32 block of every 64x64 product -- activations, their
+// derivatives (which stay in its registers) and gradients -- so each layer is
+// one MFMA chain deep; dW3, dW1 and the bias sums are shared out.  What
+// bounds it is that chain of layers and barriers, not the matrix cores.  (One
+// wavefront per tile with 79 KB of LDS put two wavefronts on a CU: 60 us for
+// a batch of 65,536, in two rounds; four blocks of four now fit: 23 us.)
+template <int ACT>
+__global__ __launch_bounds__(256, 4) void mlp_train_kernel(TrainArgs a) {
     __shared__ MlpLds s;
-    const int l = threadIdx.x & 63;
-    f32x16 dw1[2], dw2[4], dw3[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) dw1[i] = f32x16{};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dw2[i] = f32x16{};
-#pragma unroll
-    for (int i = 0; i < 2; ++i) dw3[i] = f32x16{};
-    float db1 = 0.f, db2 = 0.f, db3 = 0.f, loss = 0.f;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int mb = w >> 1, nb = w & 1;
+    f32x16 dw2 = {}, dw13 = {};  // dw13: dW3 rows 32w.. in wavefronts 0, 1; dW1 columns 32(w-2).. in 2, 3
+    float db = 0.f, db3 = 0.f, loss = 0.f;  // db: b2 in wavefront 1, b1 in 0
+    
     const uint32_t ntile = a.batch / 64u;
     for (uint32_t t = blockIdx.x; t < ntile; t += gridDim.x) {
+        // (opaque: fragments and LDS addresses held over the loop would spill)
+        const __bf16* wq = a.m.q;
+        int l = lane;
+        asm volatile("" : "+s"(wq), "+v"(l));
         const uint32_t sidx = t * 64u + (uint32_t)l;
         uint64_t rec;
         if (a.full_pass) {
             rec = sidx;
         } else {
             const U4 o = philox10(sidx, a.step, 0x4D4C50u, 0u, a.seed_lo, a.seed_hi);
-            rec = (((uint64_t)o.y << 32) | o.x) % a.n;
+            // x mod n: n_inv = floor((2^64 - 1) / n) gives a quotient at most 2 too small
+            const uint64_t x = ((uint64_t)o.y << 32) | o.x;
+            rec = x - __umul64hi(x, a.n_inv) * a.n;
+            if (rec >= a.n) rec -= a.n;
+            if (rec >= a.n) rec -= a.n;
         }
-        float f[12];
-#pragma unroll
-        for (int k = 0; k < 12; ++k) f[k] = a.feats[rec * 12 + k];
-        stage_inputs(s.x, s.xt, a.m, f, true);
-        float o0, o1;
-        mlp_forward_tile<ACT>(s, a.m, o0, o1);
-        const float y = a.ylog[rec], c = a.ycrit[rec];
-        const float sp = fmaxf(o1, 0.f) + log1pf(expf(-fabsf(o1)));
-        loss += (o0 - y) * (o0 - y) + sp - c * o1;
-        const float inv_b = 1.0f / (float)a.batch;
-        const float d0 = 2.0f * (o0 - y) * inv_b;
-        const float d1 = (1.0f / (1.0f + expf(-o1)) - c) * inv_b;
-        // dO staged as bf16 [row][32] (cols 0,1) and transposed
-        for (int q = 0; q < 32; ++q) {
-            s.dz[l * kLdH + q] = (__bf16)(q == 0 ? d0 : (q == 1 ? d1 : 0.0f));
-            s.dzt[q * kLdH + l] = (__bf16)(q == 0 ? d0 : (q == 1 ? d1 : 0.0f));
+        // wavefront w standardises features 3w .. 3w+2 and clears input 12+w
+        float y = 0.f, c = 0.f;
+        if (w == 0) {
+            y = a.ylog[rec];
+            c = a.ycrit[rec];
         }
-        wave_sync();
-        // dW3[hid][out] += H2^T . dO ; db3
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+        for (int q = 0; q < 4; ++q) {
+            const int k = q < 3 ? 3 * w + q : 12 + w;
+            float z = 0.0f;
+            if (q < 3) z = (a.feats[rec * 12 + k] - a.m.norm[k]) * (1.0f / a.m.norm[12 + k]);
+            const __bf16 b = (__bf16)z;
+            s.x[l * kLdX + k] = b;
+            s.xt[k * kLdH + l] = b;
+        }
+        u32x8 g1, g2;
+        {
+            bf16x8 w1[1];
+            load_frags<16>(wq + kQW1t, nb, l, w1);
+            __syncthreads();
+            activate_block<ACT>(mfma_block<16>(s.x, kLdX, mb, l, w1), a.m.w32[kPB1 + nb * 32 + acc_col(l)], mb, nb, l, s.h1, s.h1t, g1);
+            bf16x8 w2[4];
+            load_frags<64>(wq + kQW2t, nb, l, w2);
+            __syncthreads();
+            activate_block<ACT>(mfma_block<64>(s.h1, kLdH, mb, l, w2), a.m.w32[kPB2 + nb * 32 + acc_col(l)], mb, nb, l, s.h2, s.h2t, g2);
+        }
+        {
+            bf16x8 w3[4];
+            if (w < 2) load_frags<64>(wq + kQW3t, 0, l, w3);
+            __syncthreads();
+            if (w < 2) {
+                const f32x16 o = mfma_block<64>(s.h2, kLdH, w, l, w3);
+                if (acc_col(l) < kNo) {
+                    const float b3 = a.m.w32[kPB3 + acc_col(l)];
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) s.out[(w * 32 + acc_row(i, l)) * 2 + acc_col(l)] = o[i] + b3;
+                }
+            }
+        }
+        bf16x8 w3[2];
+        load_frags<32>(wq + kQW3, nb, l, w3);
+        __syncthreads();
+        // dO staged as bf16 [row][32] (columns 0, 1) and transposed
+        float d0 = 0.f, d1 = 0.f;
+        if (w == 0) {
+            const float o0 = s.out[l * 2], o1 = s.out[l * 2 + 1];
+            const float sp = fmaxf(o1, 0.f) + log1pf(expf(-fabsf(o1)));
+            loss += (o0 - y) * (o0 - y) + sp - c * o1;
+            const float inv_b = 1.0f / (float)a.batch;
+            d0 = 2.0f * (o0 - y) * inv_b;
+            d1 = (1.0f / (1.0f + expf(-o1)) - c) * inv_b;
+        }
+        bf16x8 dO = {};
+        dO[0] = (__bf16)d0;
+        dO[1] = (__bf16)d1;
+        *reinterpret_cast<bf16x8*>(s.dz + l * kLdH + 8 * w) = dO;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s.dzt[(8 * w + q) * kLdH + l] = dO[q];
+        __syncthreads();
+        // dW3[hid][out] += H2^T . dO ; db3 ; dH2 = dO . W3^T
+        f32x16 dh = mfma_block<32>(s.dz, kLdH, mb, l, w3);
+        if (w < 2) {
 #pragma unroll
             for (int kb = 0; kb < 4; ++kb)
-                dw3[mb] = mfma(lds_frag(s.h2t, kLdH, mb * 32, kb * 16), lds_frag(s.dzt, kLdH, 0, kb * 16), dw3[mb]);
-        if (l < kNo)
+                dw13 = mfma(lds_frag(s.h2t, kLdH, w * 32, kb * 16, l), lds_frag(s.dzt, kLdH, 0, kb * 16, l), dw13);
+        } else if (w == 2 && l < kNo) {
+#pragma unroll 8
             for (int r = 0; r < 64; ++r) db3 += (float)s.dz[r * kLdH + l];
-        // dH2 = dO . W3^T -> dZ2 = dH2 * relu'(Z2)
-        f32x16 dh[4];
+        }
+        __syncthreads();
+        grad_block(dh, g2, mb, nb, l, s);
+        bf16x8 w2[4];
+        load_frags<64>(wq + kQW2, nb, l, w2);
+        __syncthreads();
+        // dW2[in][out] += H1^T . dZ2 ; db2 ; dH1 = dZ2 . W2^T
+        dh = mfma_block<64>(s.dz, kLdH, mb, l, w2);
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
-                f32x16 cc = {};
-#pragma unroll
-                for (int kb = 0; kb < 2; ++kb)
-                    cc = mfma(lds_frag(s.dz, kLdH, mb * 32, kb * 16), glb_frag(a.m.q + kQW3, kNoPad, nb * 32, kb * 16), cc);
-                dh[mb * 2 + nb] = cc;
-            }
-        wave_sync();
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int row = mb * 32 + acc_row(i), col = nb * 32 + acc_col();
-                    const __bf16 v = (__bf16)(dh[mb * 2 + nb][i] * (float)s.g2[row * kLdH + col]);
-                    s.dz[row * kLdH + col] = v;
-                    s.dzt[col * kLdH + row] = v;
-                }
-        wave_sync();
-        // dW2[in][out] += H1^T . dZ2 ; db2
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-                for (int kb = 0; kb < 4; ++kb)
-                    dw2[mb * 2 + nb] = mfma(lds_frag(s.h1t, kLdH, mb * 32, kb * 16),
-                                            lds_frag(s.dzt, kLdH, nb * 32, kb * 16), dw2[mb * 2 + nb]);
-        for (int r = 0; r < 64; ++r) db2 += (float)s.dz[r * kLdH + l];
-        // dH1 = dZ2 . W2^T -> dZ1
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
-                f32x16 cc = {};
-#pragma unroll
-                for (int kb = 0; kb < 4; ++kb)
-                    cc = mfma(lds_frag(s.dz, kLdH, mb * 32, kb * 16), glb_frag(a.m.q + kQW2, kNh, nb * 32, kb * 16), cc);
-                dh[mb * 2 + nb] = cc;
-            }
-        wave_sync();
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int row = mb * 32 + acc_row(i), col = nb * 32 + acc_col();
-                    const __bf16 v = (__bf16)(dh[mb * 2 + nb][i] * (float)s.g1[row * kLdH + col]);
-                    s.dz[row * kLdH + col] = v;
-                    s.dzt[col * kLdH + row] = v;
-                }
-        wave_sync();
+        for (int kb = 0; kb < 4; ++kb)
+            dw2 = mfma(lds_frag(s.h1t, kLdH, mb * 32, kb * 16, l), lds_frag(s.dzt, kLdH, nb * 32, kb * 16, l), dw2);
+        if (w == 1) {
+#pragma unroll 8
+            for (int r = 0; r < 64; ++r) db += (float)s.dz[r * kLdH + l];
+        }
+        __syncthreads();
+        grad_block(dh, g1, mb, nb, l, s);
+        __syncthreads();
         // dW1[in][hid] += X^T . dZ1 (M = 16 inputs padded to 32 rows) ; db1
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
+        if (w >= 2) {
 #pragma unroll
             for (int kb = 0; kb < 4; ++kb) {
                 bf16x8 af;
                 const int mrow = l & 31, k0 = kb * 16 + 8 * (l >> 5);
 #pragma unroll
                 for (int j = 0; j < 8; ++j) af[j] = mrow < kNin ? s.xt[mrow * kLdH + k0 + j] : (__bf16)0.0f;
-                dw1[nb] = mfma(af, lds_frag(s.dzt, kLdH, nb * 32, kb * 16), dw1[nb]);
+                dw13 = mfma(af, lds_frag(s.dzt, kLdH, (w - 2) * 32, kb * 16, l), dw13);
             }
-        for (int r = 0; r < 64; ++r) db1 += (float)s.dz[r * kLdH + l];
-        wave_sync();
+        } else if (w == 0) {
+#pragma unroll 8
+            for (int r = 0; r < 64; ++r) db += (float)s.dz[r * kLdH + l];
+        }
+        __syncthreads();
     }
     // write this block's partial gradient in blob order
     float* P = a.partial + (size_t)blockIdx.x * (kPTotal + 1);
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int row = acc_row(i), col = nb * 32 + acc_col();
-            if (row < kNin) P[kPW1 + row * kNh + col] = dw1[nb][i];
+    for (int i = 0; i < 16; ++i) {
+        P[kPW2 + (mb * 32 + acc_row(i)) * kNh + nb * 32 + acc_col()] = dw2[i];
+        const int row = acc_row(i), col = acc_col();
+        if (w < 2) {
+            if (col < kNo) P[kPW3 + (w * 32 + row) * kNo + col] = dw13[i];
+        } else if (row < kNin) {
+            P[kPW1 + row * kNh + (w - 2) * 32 + col] = dw13[i];
         }
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int row = mb * 32 + acc_row(i), col = nb * 32 + acc_col();
-                P[kPW2 + row * kNh + col] = dw2[mb * 2 + nb][i];
-            }
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int row = mb * 32 + acc_row(i), col = acc_col();
-            if (col < kNo) P[kPW3 + row * kNo + col] = dw3[mb][i];
-        }
-    P[kPB1 + l] = db1;
-    P[kPB2 + l] = db2;
-    if (l < kNo) P[kPB3 + l] = db3;
-    // loss: wave sum
-    for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
-    if (l == 0) P[kPTotal] = loss;
+    }
+    if (w == 0) {
+        P[kPB1 + lane] = db;
+        // loss: wave sum
+        for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
+        if (lane == 0) P[kPTotal] = loss;
+    } else if (w == 1) {
+        P[kPB2 + lane] = db;
+    } else if (w == 2 && lane < kNo) {
+        P[kPB3 + lane] = db3;
+    }
 }
 
 // Sum the per-block partials in a fixed order; optional Adam update.
@@ -345,6 +353,8 @@ struct AdamArgs {
     float* m;
     float* v;
     float* grad;             // out: summed gradient (+ loss at [kPTotal])
+    float* loss;             // out: the loss sum (nullptr: not wanted)
+    __bf16* q;               // packed bf16 copies, updated with the parameters
     const float* partial;
     uint32_t nparts;
     int32_t t;               // Adam step (1-based); 0 = only reduce
@@ -353,22 +363,35 @@ struct AdamArgs {
 
 // Block b reduces parameters 64b..64b+63: wave w sums partials w, w+4, ...
 // (coalesced rows), then the four sums are combined in a fixed order, so the
-// gradient is deterministic.
+// gradient is deterministic.  22 MB of partials at a batch of 65,536: 128 loads
+// in flight per lane hide their latency (8 us; 16 with 32 loads, 23 with 4).  Each updated
+// parameter goes to its bf16 copies at once (a pass of its own took 5 us).
 constexpr int kAdamParams = 64;
+constexpr uint32_t kAdamLoads = 128;
 static __global__ __launch_bounds__(256) void mlp_adam_kernel(AdamArgs a) {
     __shared__ float s_g[4][kAdamParams];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int p = blockIdx.x * kAdamParams + lane;
     float g = 0.f;
     if (p <= kPTotal) {
+        const float* P = a.partial + p;
+        uint32_t q = (uint32_t)w;
+        for (; q + 4u * (kAdamLoads - 1u) < a.nparts; q += 4u * kAdamLoads) {
+            float part[kAdamLoads];
+#pragma unroll
+            for (uint32_t i = 0; i < kAdamLoads; ++i) part[i] = P[(size_t)(q + 4u * i) * (kPTotal + 1)];
+#pragma unroll
+            for (uint32_t i = 0; i < kAdamLoads; ++i) g += part[i];
+        }
 #pragma unroll 4
-        for (uint32_t q = (uint32_t)w; q < a.nparts; q += 4u) g += a.partial[(size_t)q * (kPTotal + 1) + p];
+        for (; q < a.nparts; q += 4u) g += P[(size_t)q * (kPTotal + 1)];
     }
     s_g[w][lane] = g;
     __syncthreads();
     if (w != 0 || p > kPTotal) return;
     g = (s_g[0][lane] + s_g[1][lane]) + (s_g[2][lane] + s_g[3][lane]);
     a.grad[p] = g;
+    if (p == kPTotal && a.loss) *a.loss = g;
     if (p == kPTotal || a.t <= 0) return;
     if (p >= 12 * kNh && p < kNin * kNh) return;  // padding rows of W1 stay zero
     const float m = a.b1 * a.m[p] + (1.0f - a.b1) * g;
@@ -377,7 +400,20 @@ static __global__ __launch_bounds__(256) void mlp_adam_kernel(AdamArgs a) {
     a.v[p] = v;
     const float mh = m / (1.0f - powf(a.b1, (float)a.t));
     const float vh = v / (1.0f - powf(a.b2, (float)a.t));
-    a.w32[p] -= a.lr * mh / (sqrtf(vh) + a.eps);
+    const float wn = a.w32[p] - a.lr * mh / (sqrtf(vh) + a.eps);
+    a.w32[p] = wn;
+    const __bf16 b = (__bf16)wn;
+    if (p < kPB1) {
+        a.q[kQW1t + (p % kNh) * kNin + p / kNh] = b;
+    } else if (p >= kPW2 && p < kPB2) {
+        const int e = p - kPW2;
+        a.q[kQW2t + (e % kNh) * kNh + e / kNh] = b;
+        a.q[kQW2 + e] = b;
+    } else if (p >= kPW3 && p < kPB3) {
+        const int e = p - kPW3;
+        a.q[kQW3t + (e % kNo) * kNh + e / kNo] = b;
+        a.q[kQW3 + (e / kNo) * kNoPad + e % kNo] = b;
+    }
 }
 
 // fp32 master -> packed bf16 copies
