@@ -44,7 +44,8 @@ def build_lib():
         # phase_a_kernel 72.8 -> 68.6 us on the 1M-subvolume Brusselator mesh
         jobs.append((f"plis_variant_{s}_{r}", "plis_variant.hip", [*defs, "-mllvm", "-disable-machine-licm"]))
         if s <= 8:
-            jobs.append((f"plis_variant_learned_{s}_{r}", "plis_variant_learned.hip", defs))
+            jobs.append((f"plis_variant_learned_{s}_{r}", "plis_variant_learned.hip",
+                         [*defs, "-mllvm", "-disable-machine-licm"]))
 
     def compile_one(job):
         name, src, defs = job

@@ -197,16 +197,23 @@ __global__ __launch_bounds__(256) void learned_tau_kernel(KernelArgs a) {
 // network's proposals for step + 1 on the new counts, from one evaluation
 // of their propensities.  Proposals of a realization whose step is rejected
 // are never read (commit clears prop_ok).
+//
+// Latency-bound at its occupancy: with its arguments loaded per tile, no
+// constants hoisted and 3 waves per SIMD (168 registers, 8 spilled) 42 us on
+// the 262,144-subvolume Brusselator mesh; 46 at 2 waves, 52 at 4 (spills).
+// Networks of 8 species would spill a hundred registers at 3.
 template <int MS, int MR, bool MC, int ACT>
-__global__ __launch_bounds__(256) void learned_finish_kernel(KernelArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MS <= 5 ? 3 : 1)))
+void learned_finish_kernel(KernelArgs a0) {
     __shared__ MlpLdsW W;
-    stage_weights(W, MlpDev{a.mlp_w32, (const __bf16*)a.mlp_q, a.mlp_norm});
+    stage_weights(W, MlpDev{a0.mlp_w32, (const __bf16*)a0.mlp_q, a0.mlp_norm});
     __syncthreads();
-    const NetView n = net_view<MC>(a);
     const uint32_t lane = threadIdx.x & 63u;
     for (uint32_t it = 0;; ++it) {
-        const uint32_t t = tile_at(it, a.ntiles, a.waves_per_block);
+        const uint32_t t = tile_at(it, a0.ntiles, a0.waves_per_block);
         if (t == 0xFFFFFFFFu) break;
+        const KernelArgs& a = tile_args();
+        const NetView n = net_view<MC>(a);
         const TileEnt te = ld_ro(a.tiles + t);
         const uint32_t r = wave_uniform(te.r);
         const RealInfo ri = ld_ro(a.info + r);

@@ -1,8 +1,6 @@
 // plis_variant_learned.hip -- the learned-tau kernels of one (species,
 // reactions) bound and their launches; compiled once per bound, like
-// plis_variant.hip, but with the compiler's loop-invariant code motion on:
-// without it learned_finish_kernel loses a wave per SIMD (42 -> 69 us on the
-// 262,144-subvolume Brusselator mesh).
+// plis_variant.hip.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
