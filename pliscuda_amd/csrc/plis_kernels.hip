@@ -352,7 +352,7 @@ __device__ void choose_event(const KernelArgs& a, const NetView& n, const RealIn
         const double d = n.d[cc * n.S + s];
         if (d > 0.0 && !hop_active(d, x[s], a.n_critical)) a0c += (d * (double)x[s]) * W;
     }
-    const U4 o = philox10(v, kSelfId, c.step, ctr_word3(ri.id, 0u, kCrit, 0u), a.seed_lo, a.seed_hi);
+    const U4 o = philox10_u(v, kSelfId, c.step, ctr_word3(ri.id, 0u, kCrit, 0u), a.seed_lo, a.seed_hi);
     const double target = uniform01(o.x) * a0c;
     double acc = 0.0;
     int kind = 0, idx = -1;
@@ -704,7 +704,7 @@ __device__ __forceinline__ void cao_tau_tile(const KernelArgs& a, const NetView&
         tau_subvolume<MS, MR>(a, n, ri, X, x, v, tp, a0c);
         if (a0c > 0.0) {
             const uint32_t step = wave_uniform(cp->step) + (spec ? 1u : 0u);
-            const U4 o = philox10(v, kSelfId, step, ctr_word3(ri.id, 0u, kTau2, 0u), a.seed_lo, a.seed_hi);
+            const U4 o = philox10_u(v, kSelfId, step, ctr_word3(ri.id, 0u, kTau2, 0u), a.seed_lo, a.seed_hi);
             t2 = -dlog(uniform01(o.x)) / a0c;
         }
         if (dbg) {
@@ -891,7 +891,7 @@ __device__ __forceinline__ bool leap_subvolume(const KernelArgs& a, const NetVie
             if (is_crit<MR>(crit, j) || !(av[j] > 0.0)) continue;
             const uint32_t b = (uint32_t)j >> 4;
             if (b != blk) {
-                o = philox10(v, kSelfId, sv.step, c3base | b, k0, k1);
+                o = philox10_u(v, kSelfId, sv.step, c3base | b, k0, k1);
                 blk = b;
             }
             const long long k = leap_draw(tau * av[j], coarse_byte(o, (uint32_t)j), v, kSelfId, sv.step, c3base,
@@ -947,7 +947,7 @@ __device__ __forceinline__ bool leap_subvolume(const KernelArgs& a, const NetVie
                 if (!(lo0 > 0.0 || lo1 > 0.0 || li0 > 0.0 || li1 > 0.0)) continue;
                 const uint32_t lo = v < u ? v : u, hi = v < u ? u : v;
                 const uint32_t dout = v > u ? 1u : 0u, din = 1u - dout;
-                const U4 o = philox10(lo, hi, sv.step, cb, k0, k1);
+                const U4 o = philox10_u(lo, hi, sv.step, cb, k0, k1);
                 auto hop = [&](double l, uint32_t w) {
                     return leap_draw(l, coarse_byte(o, w), lo, hi, sv.step, c3hop, k0, k1, w);
                 };
@@ -981,7 +981,7 @@ __device__ __forceinline__ bool leap_subvolume(const KernelArgs& a, const NetVie
                 if (s >= n.S) break;
                 if (!act[s]) continue;
                 const uint32_t wd = 2u * (uint32_t)s + dout;
-                const U4 o = philox10(lo, hi, sv.step, c3hop | (wd >> 4), k0, k1);
+                const U4 o = philox10_u(lo, hi, sv.step, c3hop | (wd >> 4), k0, k1);
                 const long long k =
                     leap_draw(tau * (dx[s] * wq), coarse_byte(o, wd), lo, hi, sv.step, c3hop, k0, k1, wd);
                 nx[s] -= k;
@@ -1002,7 +1002,7 @@ __device__ __forceinline__ bool leap_subvolume(const KernelArgs& a, const NetVie
                 const double du = n.d[cu * n.S + s];
                 if (!hop_active(du, xu, nc)) continue;
                 const uint32_t wd = 2u * (uint32_t)s + din;
-                const U4 o = philox10(lo, hi, sv.step, c3hop | (wd >> 4), k0, k1);
+                const U4 o = philox10_u(lo, hi, sv.step, c3hop | (wd >> 4), k0, k1);
                 nx[s] += leap_draw(tau * ((du * (double)xu) * wq), coarse_byte(o, wd), lo, hi, sv.step, c3hop, k0,
                                    k1, wd);
             }
@@ -1083,6 +1083,15 @@ constexpr uint32_t kQueue = 256;
 constexpr float kPtrsMaybeF = 9.9999f;
 constexpr uint32_t kQueueReact = 0x80000000u;  // reaction: flag | lane << 16 | j << 8 | byte
                                                // hop: entry << 12 | w << 8 | byte (kMaxTileEdges)
+// Draws that are made at once instead of queued: from kInlineDraws open ones
+// per species among 64 entries, or of one reaction in a tile, on, one fine block
+// and one squeeze per direction for all 64 lanes cost less than each queued
+// draw's own block, entry and counts (bistable 64^3 grid at its equilibrium
+// 38 -> 30 us a leap with thresholds of 32 or 48, 30.1 with 16).  Means of kInlineMaxF or more and draws
+// the squeeze leaves open are queued all the same.  Networks of more than 3
+// species have no registers left for it.
+constexpr uint32_t kInlineDraws = 32;
+constexpr float kInlineMaxF = 9.99f;
 constexpr float kNoHop = -0x1p+100f;           // rate of a hop that is critical or absent: never open
 
 // One wavefront's staging.  The queue takes all draws of 64 entries.
@@ -1180,7 +1189,7 @@ __device__ __forceinline__ void drain_draw(const KernelArgs& a, const NetView& n
         c3 = ctr_word3(sv.real, sv.attempt, kHop, kFineBlock + (w >> 2));
         big = big || lf > kPtrsMaybeF;
     }
-    const uint32_t word = draw_word(hb, philox10(v0 + i, c1, sv.step, c3, a.seed_lo, a.seed_hi), w);
+    const uint32_t word = draw_word(hb, philox10_u(v0 + i, c1, sv.step, c3, a.seed_lo, a.seed_hi), w);
     long long k = lf < kSqueezeMaxF ? poisson_squeeze(lf, __uint2float_rn(word) * 0x1p-32f) : -1;
     if (k < 0) {
         if (lam < kPoissonInvMax) k = inversion_search(lam, word);
@@ -1307,7 +1316,7 @@ __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetVi
                     any = any || on || rate[2 * s] > 0.0f;
                 }
                 if (wave_ballot(any && valid) == 0ull) continue;
-                const U4 o = philox10(v0 + i, u, sv.step, c3hop, k0, k1);
+                const U4 o = philox10_u(v0 + i, u, sv.step, c3hop, k0, k1);
                 bool open[2 * MS];
                 uint32_t total = 0u;
 #pragma unroll
@@ -1317,6 +1326,36 @@ __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetVi
                 }
                 if (qn + total > kCap) break;  // drawn below, then this entry again
                 opened += total;
+                if constexpr (MS <= 3) {
+                    if (total >= kInlineDraws * MS) {
+                        U4 f{};
+#pragma unroll
+                        for (int s = 0; s < MS; ++s) {
+                            if (s % 2 == 0)
+                                f = philox10_u(v0 + i, u, sv.step, c3hop | (kFineBlock + (uint32_t)s / 2u), k0, k1);
+                            int k[2] = {0, 0};
+#pragma unroll
+                            for (int dir = 0; dir < 2; ++dir) {
+                                const int w = 2 * s + dir;
+                                // (within 8 2^-24 of the double mean, like hop_mean_f)
+                                const float lf = (rate[w] * (dir ? w1 : w0)) * (1.0f / kCoarseScale);
+                                if (!(open[w] && lf < kInlineMaxF)) continue;
+                                const uint32_t word = draw_word(coarse_byte(o, (uint32_t)w), f, (uint32_t)w);
+                                const int kd = poisson_squeeze(lf, __uint2float_rn(word) * 0x1p-32f);
+                                if (kd < 0) continue;
+                                open[w] = false;
+                                k[dir] = kd;
+                            }
+                            fire += (unsigned long long)(uint32_t)(k[0] + k[1]);
+                            const int b = k[1] - k[0];  // never wide: a squeezed draw is at most kSqueezeK
+                            if (b != 0) {
+                                atomicAdd(&L.del[s][i], b);
+                                if (u - v0 < (uint32_t)kTile) atomicAdd(&L.del[s][u - v0], -b);
+                                else atomicAdd(&Y[ri.x_off + (uint64_t)s * N + u], (uint32_t)-b);
+                            }
+                        }
+                    }
+                }
                 const uint32_t code = (e - eb) << 12;
 #pragma unroll
                 for (int w = 0; w < 2 * MS; ++w) {
@@ -1330,7 +1369,9 @@ __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetVi
         if (it == nit) {
             // reactions of subvolume v, propensities and criticality as react_props
             // computes them (same operations, one reaction at a time)
-            const U4 o = philox10(v, kSelfId, sv.step, c3react, k0, k1);
+            const U4 o = philox10_u(v, kSelfId, sv.step, c3react, k0, k1);
+            U4 f{};
+            int fine = -1;  // f: the fine bits of reactions 4 fine .. 4 fine + 3
             for (; j < n.R; ++j) {
                 double aj = n.k[cl * n.R + j];
                 bool low = false;
@@ -1342,11 +1383,33 @@ __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetVi
                     low = low || below_nc(xs, rq, nc);
                 }
                 const uint32_t hb = coarse_byte(o, (uint32_t)j);
-                const bool open = vok && !(n.order[j] > 0 && low) && aj > 0.0 && !coarse_zero(tau * aj, hb);
-                const uint64_t m = wave_ballot(open);
-                const uint32_t cnt = (uint32_t)__popcll(m);
+                bool open = vok && !(n.order[j] > 0 && low) && aj > 0.0 && !coarse_zero(tau * aj, hb);
+                uint64_t m = wave_ballot(open);
+                uint32_t cnt = (uint32_t)__popcll(m);
                 if (qn + cnt > kCap) break;
                 opened += cnt;
+                if constexpr (MS <= 3) {
+                    if (cnt >= kInlineDraws) {
+                        if (fine != (j >> 2)) {
+                            fine = j >> 2;
+                            f = philox10_u(v, kSelfId, sv.step, c3react | (kFineBlock + (uint32_t)fine), k0, k1);
+                        }
+                        const float lf = (float)(tau * aj);
+                        if (open && lf < kInlineMaxF) {
+                            const int k = poisson_squeeze(lf, __uint2float_rn(draw_word(hb, f, (uint32_t)j)) * 0x1p-32f);
+                            open = k < 0;
+                            if (k > 0) {
+                                fire += (unsigned long long)(uint32_t)k;
+                                for (int s = 0; s < n.S; ++s) {
+                                    const int nu = n.nu[s * n.R + j];
+                                    if (nu != 0) add_balance(a, ri, L, Y, v0, s, v, (long long)k * (long long)nu);
+                                }
+                            }
+                        }
+                        m = wave_ballot(open);
+                        cnt = (uint32_t)__popcll(m);
+                    }
+                }
                 if (open) L.q[qn + lanes_below(m)] = kQueueReact | (lane << 16) | ((uint32_t)j << 8) | hb;
                 qn += cnt;
             }
@@ -1511,11 +1574,13 @@ __device__ __forceinline__ StepView step_view(const RealInfo& ri, cptr<RealCtl> 
 // an entry's or a code's bits).  GEN: several compartments, or (EP) an
 // asymmetric topology.
 //
-// The edge-parallel leap of up to 5 species, one compartment, runs at 5 waves
+// The edge-parallel leap of 4 or 5 species, one compartment, runs at 5 waves
 // per SIMD (96 VGPRs): at 6 the sampler spills (1M-subvolume Brusselator mesh
-// 83.6 -> 94.5 us), at 4 fewer waves hide the walk's gathers (88 us).
+// 83.6 -> 94.5 us), at 4 fewer waves hide the walk's gathers (88 us).  Up to 3
+// species draw dense tiles in the walk and run at 4 (at 5 it spills: bistable
+// 64^3 grid 28.4 -> 29.6 us dense, 19.4 -> 20.9 sparse).
 template <int MS, int MR, bool EP, bool GEN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EP && !GEN && MS <= 5 ? 5 : 1)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EP && !GEN && MS <= 5 ? (MS <= 3 ? 4 : 5) : 1)))
 void phase_b_kernel(KernelArgs a0) {
     const uint32_t wv = wave_uniform(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     __shared__ LeapLds<EP ? MS : 1, GEN> s_l[EP ? 4 : 1];  // (up to 4 waves per block)

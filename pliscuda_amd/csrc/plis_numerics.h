@@ -40,20 +40,35 @@ __device__ __forceinline__ uint32_t ctr_word3(uint32_t real, uint32_t attempt, u
 
 struct U4 { uint32_t x, y, z, w; };
 
+// one three-input instruction (the compiler makes two of a ^ b ^ c): 4 per
+// Philox round instead of 6
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+}
+
 __device__ __forceinline__ U4 philox10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
                                        uint32_t k0, uint32_t k1) {
 #pragma unroll
     for (int i = 0; i < 10; ++i) {
         const uint64_t p0 = (uint64_t)0xD2511F53u * c0;   // one v_mad_u64_u32 each
         const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
-        c0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0;
-        c2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
+        c0 = xor3((uint32_t)(p1 >> 32), c1, k0);
+        c2 = xor3((uint32_t)(p0 >> 32), c3, k1);
         c1 = (uint32_t)p1;
         c3 = (uint32_t)p0;
         k0 += 0x9E3779B9u;
         k1 += 0xBB67AE85u;
     }
     return U4{c0, c1, c2, c3};
+}
+
+// With a key that is the same in every lane.  Its round keys are formed by the
+// scalar unit at each call: left to itself the compiler forms all 20 once and
+// holds them, spilled to lanes of vector registers, over the whole kernel.
+__device__ __forceinline__ U4 philox10_u(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
+                                         uint32_t k1) {
+    asm volatile("" : "+s"(k0), "+s"(k1));
+    return philox10(c0, c1, c2, c3, k0, k1);
 }
 
 __device__ __forceinline__ uint32_t pick(const U4& o, uint32_t i) {
@@ -291,8 +306,8 @@ __device__ __attribute__((noinline)) long long poisson_slow(double lam, uint32_t
 // (0, 10) and k <= kSqueezeK, |G_k - F_k| stays below 2^-20 (checked over
 // all such floats on the host with the same operations); rounding the mean
 // moves F_k by at most 2^-21 (|dF_k/dlam| <= 1), rounding u by at most
-// 2^-25, and forming G -+ delta by 2^-25 more.  With delta = 2^-15 >> the
-// sum, u_f <= G_k - delta proves u <= F_k and u_f > G_k + delta proves
+// 2^-25, and forming u -+ delta by 2^-25 more.  With delta = 2^-15 >> the
+// sum, u_f + delta <= G_k proves u <= F_k and u_f - delta > G_k proves
 // u > F_k: the search result is found without double arithmetic, and is
 // the one the double search returns.  u within delta of some G_k (odds
 // about 6e-5 per comparison) or k > kSqueezeK leaves it to the double search.
@@ -326,16 +341,20 @@ __device__ __forceinline__ float fexp_neg(float l) {
 __device__ __forceinline__ int poisson_squeeze(float l, float u) {
     float p = fexp_neg(l);
     float G = p;
-    // (unrolled: the reciprocals are literals; from a table each trip waited
-    // on a scalar load)
+    const float lo = u - kSqueeze, hi = u + kSqueeze;
+    // Unrolled: the reciprocals are literals; from a table each trip waited on a
+    // scalar load.  Lanes that are done keep their G under a select and the
+    // wavefront leaves together: sixteen nested exits held a mask each.
+    int k = 0;
 #pragma unroll
-    for (int k = 0; k <= kSqueezeK; ++k) {
-        if (u <= G - kSqueeze) return k;
-        if (!(u > G + kSqueeze) || k == kSqueezeK) return -1;
-        p = (p * l) * kRecipF[k < kSqueezeK ? k + 1 : 0];
-        G = G + p;
+    for (int j = 1; j <= kSqueezeK; ++j) {
+        const bool on = G < lo;
+        if (__builtin_amdgcn_ballot_w64(on) == 0ull) break;
+        p = (p * l) * kRecipF[j];
+        G = on ? G + p : G;
+        k = on ? j : k;
     }
-    return -1;
+    return G >= hi ? k : -1;
 }
 
 // Poisson(lam) from the packed word u0 (inversion) or the draw's PTRS stream.
