@@ -346,6 +346,13 @@ static ResLists res_lists(const NetHeader& h, const std::vector<int32_t>& I) {
     return l;
 }
 
+// Contexts of at most this many tiles give each tile of the leap a block of
+// four wavefronts (up to four on a SIMD).  us a step, one wavefront a tile / four:
+// 343 tiles bistable 24.6 / 20.1, A-B-C with drift 28.5 / 23.4, Brusselator mesh
+// 41.1 / 32.4; 1,000 tiles 25.4 / 22.6, 29.3 / 26.2, 43.6 / 36.6; 1,521 tiles
+// 27.2 / 28.0, 32.5 / 34.6, 48.5 / 48.1.
+constexpr uint32_t kSplitTiles = 1024;
+
 static KernelArgs make_args(plis_ctx* c) {
     KernelArgs a{};
     a.net_i = c->d_net_i;
@@ -412,7 +419,8 @@ static void launch_kernel(plis_ctx* c, int which, const KernelArgs& a) {
     c->ctl_fresh = false;
     const LaunchEnv e{c->stream,     c->split_ev,   c->blocks, c->wpb,        c->nreal,
                       c->decide_chunks, (uint32_t)c->cus, c->finish_bpc, c->learned_bpc, c->nh.C > 1,
-                      c->d_frw != nullptr, c->mlp_act == 1, c->learned_on != 0, c->edge_parallel};
+                      c->d_frw != nullptr, c->mlp_act == 1, c->learned_on != 0, c->edge_parallel,
+                      c->ntiles <= kSplitTiles};
     switch (c->variant) {
         case 0: launch_variant<1, 4>(e, which, a); break;
         case 1: launch_variant<3, 4>(e, which, a); break;
@@ -562,14 +570,17 @@ static bool resident_fit(plis_ctx* c, const NetHeader& h, const std::vector<doub
     // One CU makes a step of N subvolumes in about 5 us + N (2 + 0.84 S deg +
     // 2.8 R) ns (measured: A-B-C 7.6 us at 64, 15 at 512, 26 at 1,000, 41 at
     // 1,728; diffusion of one species 21 at 1,728; Brusselator mesh 25 at 512,
-    // 50 at 1,000).  The launch-per-pass step takes about 30 us (47 for the
-    // Brusselator) at these sizes, and 730 us or more in its general
-    // instantiation (cascade of 32 species, 62 reactions: 17 us here at 60
-    // subvolumes, 165 at 1,000).  The line lies where the two meet.
+    // 50 at 1,000).  The launch-per-pass step takes 18 us with one species, 22
+    // with the three of A-B-C and 30 with the Brusselator's five at these sizes
+    // (both sides measured: bistable 18.7 / 19.1 us at 729; A-B-C 19.3 / 21.9
+    // at 729, 25.4 / 21.9 at 1,000; diffusion 14.1 / 18.0 at 1,000, 20.1 / 18.9
+    // at 1,728; Brusselator 23.5 / 29.8 at 512), and 730 us or more in its
+    // general instantiation (cascade of 32 species, 62 reactions: 17 us here at
+    // 60 subvolumes, 165 at 1,000).  The line lies where the two meet.
     double est = 0.0;
     for (const auto& ri : c->info)
         est = std::max(est, 1e-3 * (ri.N * (2.0 + 2.8 * h.R) + 0.84 * h.S * (double)ri.n_in));
-    if (est > (c->variant > 3 ? 600.0 : 20.0 + 3.0 * h.S)) return false;
+    if (est > (c->variant > 3 ? 600.0 : 10.5 + 4.0 * h.S)) return false;
     // wavefronts: one per item of the widest phase, 4 to 16
     const uint64_t nt = (maxN + 63) / 64;
     const uint64_t items = std::max<uint64_t>(nt * std::max(h.S + 1, h.R), (nf + 63) / 64 * ((h.S + 7) / 8) + nt * ((h.R + 3) / 4));

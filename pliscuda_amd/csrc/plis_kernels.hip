@@ -109,10 +109,9 @@ __device__ __forceinline__ void lds_wave_sync() {
 
 
 // XCD-aware persistent tile walk (grid is a multiple of 8 blocks).
-__device__ __forceinline__ uint32_t tile_at(uint32_t it, uint32_t ntiles, uint32_t wpb) {
+__device__ __forceinline__ uint32_t tile_at(uint32_t it, uint32_t ntiles, uint32_t wpb, uint32_t wv) {
     const uint32_t G = gridDim.x;
     const uint32_t b = blockIdx.x;
-    const uint32_t wv = wave_uniform(threadIdx.x >> 6);
     const uint32_t xcd = b & 7u;
     const uint32_t nbx = (G - xcd + 7u) >> 3;
     const uint32_t lb = b >> 3;
@@ -120,6 +119,9 @@ __device__ __forceinline__ uint32_t tile_at(uint32_t it, uint32_t ntiles, uint32
     const uint32_t ce = (uint32_t)(((uint64_t)ntiles * (xcd + 1u)) >> 3);
     const uint32_t t = cb + lb * wpb + wv + it * nbx * wpb;
     return t < ce ? t : 0xFFFFFFFFu;
+}
+__device__ __forceinline__ uint32_t tile_at(uint32_t it, uint32_t ntiles, uint32_t wpb) {
+    return tile_at(it, ntiles, wpb, wave_uniform(threadIdx.x >> 6));
 }
 
 __device__ __forceinline__ uint32_t* count_buf(const KernelArgs& a, uint32_t i) {
@@ -500,6 +502,48 @@ __device__ __forceinline__ void tau_subvolume(const KernelArgs& a, const NetView
     double du[MS];
 #pragma unroll
     for (int s = 0; s < MS; ++s) du[s] = n.d[s < n.S ? s : 0];
+    if constexpr (MS <= 3) {
+        // three in-edges' counts in flight together, the next three's ids and
+        // weights behind them (an interior subvolume of a lattice has six): at
+        // a few waves per SIMD each trip is one memory round (A-B-C on 24,679
+        // subvolumes 8.5 -> 7.8 us against one edge a trip).  One past the
+        // row's end adds +0.
+        constexpr uint32_t kB = 3;
+        uint64_t cw[kB];
+#pragma unroll
+        for (uint32_t i = 0; i < kB; ++i) cw[i] = ib + i < ie ? icw[ib + i] : (uint64_t)v | kOneW;
+        for (uint32_t q = ib; q < ie; q += kB) {
+            uint32_t xu[kB][MS];
+            uint32_t u[kB];
+            double wq[kB];
+#pragma unroll
+            for (uint32_t i = 0; i < kB; ++i) {
+                u[i] = (uint32_t)cw[i];
+                wq[i] = (double)__uint_as_float((uint32_t)(cw[i] >> 32));
+#pragma unroll
+                for (int s = 0; s < MS; ++s) xu[i][s] = X[ri.x_off + (uint64_t)(s < n.S ? s : n.S - 1) * N + u[i]];
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < kB; ++i)
+                cw[i] = q + kB + i < ie ? icw[q + kB + i] : (uint64_t)v | kOneW;
+            int cu[kB];
+#pragma unroll
+            for (uint32_t i = 0; i < kB; ++i) cu[i] = n.C > 1 ? a.comp[ri.comp_off + u[i]] : 0;
+#pragma unroll
+            for (uint32_t i = 0; i < kB; ++i) {
+                if (n.C > 1) {
+#pragma unroll
+                    for (int s = 0; s < MS; ++s) du[s] = n.d[cu[i] * n.S + (s < n.S ? s : 0)];
+                }
+#pragma unroll
+                for (int s = 0; s < MS; ++s) xu[i][s] = q + i < ie ? xu[i][s] : 0u;
+                tau_in_edge<MS>(n.S, du, xu[i], wq[i], a.n_critical, t);
+            }
+        }
+        tp_out = tau_bound<MS>(a, n, t);
+        a0c_out = t.a0c;
+        return;
+    }
     // software pipeline: in-edge q's counts were requested in iteration q-1,
     // in-edge q+1's id and weight in iteration q-1 too, so each iteration
     // waits on nothing issued in it
@@ -1103,6 +1147,22 @@ struct LeapLds {
     int32_t del[MS][kTile];  // the tile's balances
     uint32_t q[kCap];
     int32_t c[GEN ? kTile : 1];
+    // what each wavefront of a split tile found: {firings, open draws, a mean
+    // of 10 or more}
+    unsigned long long part_fire;
+    uint32_t part_opened, part_big;
+};
+
+// A wavefront's share of a tile: wavefront `part` of `parts` (1, or the block's
+// 4) takes every parts-th group of 64 entries, reaction and species.
+template <uint32_t PARTS>
+struct TileShare {
+    static constexpr uint32_t parts = PARTS;
+    uint32_t part;
+    __device__ __forceinline__ void sync() const {
+        if (parts > 1u) __syncthreads();
+        else lds_wave_sync();
+    }
 };
 
 __device__ __forceinline__ uint64_t wave_ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
@@ -1213,13 +1273,14 @@ __device__ __forceinline__ void drain_draw(const KernelArgs& a, const NetView& n
 // The draws of one tile, and the critical event if it is the tile's, into the
 // target buffer Y.  Control flow stays
 // wave-uniform around every queue append: the loops run the same trip count
-// on every lane, lanes without work carry flags.  Returns whether the tile
-// counts as beyond its queue.  GEN: several compartments or an asymmetric
+// on every lane, lanes without work carry flags.  q_: the wavefront's queue.
+// Returns whether some mean was 10 or more, in opened_out the open draws.  GEN: several compartments or an asymmetric
 // topology.
-template <int MS, int MR, bool GEN>
+template <int MS, int MR, bool GEN, uint32_t PARTS>
 __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetView& n, const RealInfo& ri,
                                                 const uint32_t* X, uint32_t* Y, uint32_t v0, const StepView& sv,
-                                                LeapLds<MS, GEN>& L, unsigned long long& fire) {
+                                                LeapLds<MS, GEN>& L, uint32_t* q_, const TileShare<PARTS>& sh,
+                                                unsigned long long& fire, uint32_t& opened_out) {
     static_assert(MS <= 8 && MR <= 16, "one coarse block per pair and per subvolume; hop codes hold w in 4 bits");
     constexpr uint32_t kCap = LeapLds<MS, GEN>::kCap;
     const uint32_t lane = threadIdx.x & 63u;
@@ -1239,6 +1300,7 @@ __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetVi
         const double d = n.d[s < n.S ? s : 0];
         dt[s] = (float)d * scale;
         dpos[s] = s < n.S && d > 0.0;
+        if (sh.parts > 1u && ((uint32_t)s & 3u) != sh.part) continue;
         const uint32_t x = (vok && s < n.S) ? X[ri.x_off + (uint64_t)s * N + v] : 0u;
         L.x[s][lane] = x;
         L.del[s][lane] = 0;
@@ -1252,7 +1314,7 @@ __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetVi
     if constexpr (GEN) L.c[lane] = cl;
     const uint32_t eb = wave_uniform(a.frp[ri.rp_off + v0]);
     const uint32_t ee = wave_uniform(a.frp[ri.rp_off + min(v0 + (uint32_t)kTile, N)]);
-    lds_wave_sync();
+    sh.sync();
     const uint64_t* cwp = a.fcw + ri.fe_off;  // neighbour, row in the tile and weight in one load
     const float* rwp = GEN && a.frw ? a.frw + ri.fe_off : nullptr;
     const uint32_t c3hop = ctr_word3(sv.real, sv.attempt, kHop, 0u);
@@ -1268,16 +1330,17 @@ __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetVi
 #pragma unroll
         for (int s = 0; s < MS; ++s) xo[s] = X[ri.x_off + (uint64_t)(s < n.S ? s : n.S - 1) * N + u];
     };
-    uint32_t it = 0u;
-    int j = 0;
+    const uint32_t step64 = sh.parts * (uint32_t)kTile;
+    uint32_t it = sh.part;
+    int j = (int)(sh.parts - 1u - sh.part);  // (the wavefronts with fewer entries have more reactions)
     for (bool all = false; !all;) {
         if (it < nit) {
             uint32_t e = eb + it * (uint32_t)kTile + lane;
             const uint64_t none = (uint64_t)v0 | kOneW;
-            uint64_t cw = e < ee ? cwp[e] : none, cw_next = e + (uint32_t)kTile < ee ? cwp[e + kTile] : none;
+            uint64_t cw = e < ee ? cwp[e] : none, cw_next = e + step64 < ee ? cwp[e + step64] : none;
             uint32_t xn[MS];
             counts((uint32_t)cw & kFwdIdMask, xn);
-            for (; it < nit; ++it, e += (uint32_t)kTile) {
+            for (; it < nit; it += sh.parts, e += step64) {
                 const bool valid = e < ee;
                 const uint32_t i = (uint32_t)cw >> 26;            // the entry's row in the tile
                 const uint32_t u = (uint32_t)cw & kFwdIdMask;     // u > v0 + i
@@ -1289,9 +1352,9 @@ __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetVi
 #pragma unroll
                 for (int s = 0; s < MS; ++s) xc[s] = xn[s];
                 cw = cw_next;
-                if (e + (uint32_t)kTile < ee) {
+                if (e + step64 < ee) {
                     counts((uint32_t)cw & kFwdIdMask, xn);
-                    if (e + 2u * (uint32_t)kTile < ee) cw_next = cwp[e + 2u * kTile];
+                    if (e + 2u * step64 < ee) cw_next = cwp[e + 2u * step64];
                 }
                 int cu = 0;
                 if (GEN && n.C > 1 && valid)
@@ -1361,18 +1424,18 @@ __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetVi
                 for (int w = 0; w < 2 * MS; ++w) {
                     const uint64_t m = wave_ballot(open[w]);
                     if (m == 0ull) continue;
-                    if (open[w]) L.q[qn + lanes_below(m)] = code | ((uint32_t)w << 8) | coarse_byte(o, (uint32_t)w);
+                    if (open[w]) q_[qn + lanes_below(m)] = code | ((uint32_t)w << 8) | coarse_byte(o, (uint32_t)w);
                     qn += (uint32_t)__popcll(m);
                 }
             }
         }
-        if (it == nit) {
+        if (it >= nit) {
             // reactions of subvolume v, propensities and criticality as react_props
             // computes them (same operations, one reaction at a time)
             const U4 o = philox10_u(v, kSelfId, sv.step, c3react, k0, k1);
             U4 f{};
             int fine = -1;  // f: the fine bits of reactions 4 fine .. 4 fine + 3
-            for (; j < n.R; ++j) {
+            for (; j < n.R; j += (int)sh.parts) {
                 double aj = n.k[cl * n.R + j];
                 bool low = false;
                 const int nr = n.nrs[j];
@@ -1410,18 +1473,18 @@ __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetVi
                         cnt = (uint32_t)__popcll(m);
                     }
                 }
-                if (open) L.q[qn + lanes_below(m)] = kQueueReact | (lane << 16) | ((uint32_t)j << 8) | hb;
+                if (open) q_[qn + lanes_below(m)] = kQueueReact | (lane << 16) | ((uint32_t)j << 8) | hb;
                 qn += cnt;
             }
             all = j >= n.R;
         }
         lds_wave_sync();
         for (uint32_t q = lane; q < qn; q += (uint32_t)kTile)
-            drain_draw<MS, GEN>(a, n, ri, X, Y, v0, sv, L, eb, L.q[q], fire, big);
+            drain_draw<MS, GEN>(a, n, ri, X, Y, v0, sv, L, eb, q_[q], fire, big);
         lds_wave_sync();
         qn = 0u;
     }
-    if (sv.crit && sv.vstar - v0 < (uint32_t)kTile) {
+    if (sv.crit && sh.part == 0u && sv.vstar - v0 < (uint32_t)kTile) {
         if (v == sv.vstar && (sv.ev_kind == 1 || sv.ev_kind == 2)) {
             fire += 1ull;
             if (sv.ev_kind == 1) {
@@ -1434,13 +1497,15 @@ __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetVi
         }
         lds_wave_sync();
     }
+    if (sh.parts > 1u) __syncthreads();
     if (vok) {
 #pragma unroll
         for (int s = 0; s < MS; ++s)
-            if (s < n.S && L.del[s][lane] != 0)
+            if (s < n.S && (sh.parts == 1u || ((uint32_t)s & 3u) == sh.part) && L.del[s][lane] != 0)
                 atomicAdd(&Y[ri.x_off + (uint64_t)s * N + v], (uint32_t)L.del[s][lane]);
     }
-    return opened > kQueue || wave_ballot(big) != 0ull;
+    opened_out = opened;
+    return wave_ballot(big) != 0ull;
 }
 
 // Completes the leap of one tile (finish_counts) where the post-leap leap
@@ -1579,13 +1644,15 @@ __device__ __forceinline__ StepView step_view(const RealInfo& ri, cptr<RealCtl> 
 // 83.6 -> 94.5 us), at 4 fewer waves hide the walk's gathers (88 us).  Up to 3
 // species draw dense tiles in the walk and run at 4 (at 5 it spills: bistable
 // 64^3 grid 28.4 -> 29.6 us dense, 19.4 -> 20.9 sparse).
-template <int MS, int MR, bool EP, bool GEN>
+// SPLIT: a block of 4 wavefronts shares one tile, for contexts of few tiles,
+// where one wavefront per tile leaves most SIMDs idle.
+template <int MS, int MR, bool EP, bool GEN, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EP && !GEN && MS <= 5 ? (MS <= 3 ? 4 : 5) : 1)))
 void phase_b_kernel(KernelArgs a0) {
     const uint32_t wv = wave_uniform(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     __shared__ LeapLds<EP ? MS : 1, GEN> s_l[EP ? 4 : 1];  // (up to 4 waves per block)
     for (uint32_t it = 0;; ++it) {
-        const uint32_t t = tile_at(it, a0.ntiles, a0.waves_per_block);
+        const uint32_t t = tile_at(it, a0.ntiles, SPLIT ? 1u : a0.waves_per_block, SPLIT ? 0u : wv);
         if (t == 0xFFFFFFFFu) break;
         const KernelArgs& a = tile_args();
         const NetView n = net_view<GEN>(a);
@@ -1600,9 +1667,27 @@ void phase_b_kernel(KernelArgs a0) {
         unsigned long long fire = 0;
         uint32_t bad = 0, viol = 0;
         if constexpr (EP) {
-            const bool over = leap_tile_draws<MS, MR, GEN>(a, n, ri, X, Xn, te.v0, sv, s_l[wv], fire);
+            const TileShare<SPLIT ? 4u : 1u> sh{SPLIT ? wv : 0u};
+            uint32_t opened = 0u;
+            uint32_t big = leap_tile_draws<MS, MR, GEN>(a, n, ri, X, Xn, te.v0, sv, s_l[SPLIT ? 0u : wv], s_l[wv].q, sh,
+                                                        fire, opened) ? 1u : 0u;
             reduce_partB(fire, bad, viol);
-            if (lane == 0) a.partB_tile[t] = PartB{fire, over && a.count_redo ? 2u : 0u, 0u};
+            if constexpr (SPLIT) {
+                if (lane == 0) {
+                    s_l[wv].part_fire = fire;
+                    s_l[wv].part_opened = opened;
+                    s_l[wv].part_big = big;
+                }
+                __syncthreads();
+                for (uint32_t w = 1; wv == 0u && w < 4u; ++w) {
+                    fire += s_l[w].part_fire;
+                    opened += s_l[w].part_opened;
+                    big |= s_l[w].part_big;
+                }
+            }
+            if (lane == 0 && (!SPLIT || wv == 0u))
+                a.partB_tile[t] = PartB{fire, (opened > kQueue || big) && a.count_redo ? 2u : 0u, 0u};
+            if constexpr (SPLIT) __syncthreads();  // (before the next tile's staging)
         } else {
             const uint32_t v = te.v0 + lane;
             if (v < ri.N) bad = leap_subvolume<MS, MR>(a, n, ri, X, Xn, v, sv, fire, viol) ? 1u : 0u;

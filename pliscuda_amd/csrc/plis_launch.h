@@ -14,6 +14,7 @@ struct LaunchEnv {
     hipEvent_t* split_ev;  // profiling: events between the leap pass's kernels, or nullptr
     uint32_t blocks, wpb, nreal, decide_chunks, cus, finish_bpc, learned_bpc;
     bool mc, asym, gelu, learned_on, edge_parallel;
+    bool leap_split;  // a tile of the edge-parallel leap per block of 4 wavefronts
 };
 
 // decide_kernel and commit_decide_kernel: most blocks per realization

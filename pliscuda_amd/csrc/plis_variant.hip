@@ -39,8 +39,12 @@ void launch_variant(const LaunchEnv& c, int which, const KernelArgs& a) {
         case 2:
             if constexpr (MS <= 8) {
                 if (c.edge_parallel) {
-                    if (mc || c.asym) hipLaunchKernelGGL((phase_b_kernel<MS, MR, true, true>), grid, block, 0, c.stream, a);
-                    else hipLaunchKernelGGL((phase_b_kernel<MS, MR, true, false>), grid, block, 0, c.stream, a);
+                    const dim3 sgrid((a.ntiles + 7u) & ~7u), sblock(256);
+                    const bool gen = mc || c.asym;
+                    if (c.leap_split && gen) hipLaunchKernelGGL((phase_b_kernel<MS, MR, true, true, true>), sgrid, sblock, 0, c.stream, a);
+                    else if (c.leap_split) hipLaunchKernelGGL((phase_b_kernel<MS, MR, true, false, true>), sgrid, sblock, 0, c.stream, a);
+                    else if (gen) hipLaunchKernelGGL((phase_b_kernel<MS, MR, true, true, false>), grid, block, 0, c.stream, a);
+                    else hipLaunchKernelGGL((phase_b_kernel<MS, MR, true, false, false>), grid, block, 0, c.stream, a);
                     if (c.split_ev) (void)hipEventRecord(*c.split_ev, c.stream);
                     if (c.learned_on) launch_learned<MS, MR>(c, kLearnedFinish, a);
                     else if (!a.judge_on) break;
@@ -49,8 +53,8 @@ void launch_variant(const LaunchEnv& c, int which, const KernelArgs& a) {
                     break;
                 }
             }
-            if (mc) hipLaunchKernelGGL((phase_b_kernel<MS, MR, false, true>), grid, block, 0, c.stream, a);
-            else hipLaunchKernelGGL((phase_b_kernel<MS, MR, false, false>), grid, block, 0, c.stream, a);
+            if (mc) hipLaunchKernelGGL((phase_b_kernel<MS, MR, false, true, false>), grid, block, 0, c.stream, a);
+            else hipLaunchKernelGGL((phase_b_kernel<MS, MR, false, false, false>), grid, block, 0, c.stream, a);
             break;
         case 3:
             hipLaunchKernelGGL(commit_kernel, rgrid, rblock, 0, c.stream, a);

@@ -72,3 +72,27 @@ def test_hub():
     x0 = W.uniform_state(N, 500, 900, 3)
     x0[N - 1] = 400_000_000
     _check(net, topo, x0, 0.5, 10, 4, [2, 2])
+
+
+@pytest.mark.parametrize("sides", [(41, 40, 40), (41, 41, 40), (11, 11, 13), (13, 11, 11)])
+def test_tiles_split_over_wavefronts(sides):
+    """Either side of the sizes at which a tile gets four wavefronts, ragged last tiles."""
+    net = W.abc_network()
+    topo = W.cubic_grid(*sides, periodic=False)
+    x0 = W.poisson_state(3, topo["N"], [40.0, 12.0, 30.0], 8)
+    _check(net, topo, x0, 0.1, 10, 9, [3, 2], crit_events=1)
+
+
+def test_tiles_split_in_a_batch():
+    """Uneven realizations, one tile to many, in one launch."""
+    net = W.brusselator_network(W.SEED_BRUSS)
+    topos = [W.random_mesh(14, 12, 10, 3), W.random_mesh(4, 4, 4, 4), W.random_mesh(8, 8, 6, 5)]
+    xs = [W.poisson_state(5, t["N"], [60, 40, 80, 100, 20], 6 + i) for i, t in enumerate(topos)]
+    ctx = capi.Context(net, topos, xs, seed=3)
+    ctx.run(np.inf, step_limit=25)
+    for r, (t, x0) in enumerate(zip(topos, xs)):
+        x = x0.copy()
+        st = ffi.run(ffi.Model(net, t), x, 0.03, 10, 3, np.inf, step_limit=25, realization=r)
+        assert np.array_equal(ctx.get_state(r), x)
+        assert ctx.stats(r)["firings"] == st.firings and ctx.stats(r)["t"] == st.t
+    ctx.close()
