@@ -301,22 +301,20 @@ __device__ __forceinline__ void decide(RealCtl& c) {
 
 // Destination of a critical hop from v: the edge of v's row at which the
 // weights, summed one edge at a time in CSR order, pass tw.  Run by a whole
-// wavefront, which loads up to 64 edges at once.
-__device__ __forceinline__ uint32_t choose_hop_edge(const KernelArgs& a, const RealInfo& ri, uint32_t v, double tw) {
-    const uint32_t rb = a.rp[ri.rp_off + v], re = a.rp[ri.rp_off + v + 1];
-    const bool weighted = (ri.flags & 2u) != 0;
+// wavefront, which loads up to 64 edges at once; cw: the first ones of the row
+// [rb, re), from hop_row.
+__device__ __forceinline__ uint32_t choose_hop_edge(const KernelArgs& a, const RealInfo& ri, uint32_t v, uint32_t rb,
+                                                    uint32_t re, uint64_t cw, double tw) {
     const uint32_t lane = threadIdx.x & 63u;
     double accw = 0.0;
     uint32_t dst = v;
     bool found = false;
     for (uint32_t q0 = rb; q0 < re && !found; q0 += 64u) {
-        const uint32_t q = q0 + lane;
-        const float wl = q < re ? (weighted ? a.w[ri.e_off + q] : 1.0f) : 0.0f;
-        const uint32_t cl = q < re ? a.col[ri.e_off + q] : v;
+        if (q0 != rb) cw = a.cw[ri.e_off + min(q0 + lane, re - 1u)];
         const uint32_t cnt = min(64u, re - q0);
         for (uint32_t i = 0; i < cnt; ++i) {
-            accw += (double)__shfl(wl, (int)i);
-            dst = (uint32_t)__shfl((int)cl, (int)i);
+            accw += (double)__int_as_float(__builtin_amdgcn_readlane((int)(cw >> 32), (int)i));
+            dst = (uint32_t)__builtin_amdgcn_readlane((int)cw, (int)i);
             if (tw < accw) {
                 found = true;
                 break;
@@ -326,61 +324,103 @@ __device__ __forceinline__ uint32_t choose_hop_edge(const KernelArgs& a, const R
     return dst;
 }
 
+// v's out-edges: the row's bounds and the lane's edge {id, weight} among the
+// first 64.
+struct HopRow {
+    uint32_t rb, re;
+    uint64_t cw;
+};
+__device__ __forceinline__ HopRow hop_row(const KernelArgs& a, const RealInfo& ri, uint32_t v) {
+    HopRow h;
+    h.rb = a.rp[ri.rp_off + v];
+    h.re = a.rp[ri.rp_off + v + 1];
+    h.cw = h.rb < h.re ? a.cw[ri.e_off + min(h.rb + (threadIdx.x & 63u), h.re - 1u)] : (uint64_t)v;
+    return h;
+}
+
+__device__ __forceinline__ double lane_f64(double x, uint32_t l) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, (int)l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), (int)l);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // Critical event at v*: a critical reaction or a critical hop, chosen with
 // probability proportional to its propensity; a hop's edge is chosen in
-// proportion to its weight.  Run by a whole wavefront (every value is
-// wave-uniform).  (The reference picks a uniform slot among 6
+// proportion to its weight.  (The reference picks a uniform slot among 6
 // including self-padding, PLISCuda/src/leap.cu:180-194, ssa.cu:88-106.)
-template <int MS, int MR>
-__device__ void choose_event(const KernelArgs& a, const NetView& n, const RealInfo& ri, RealCtl& c,
-                             const uint32_t* X) {
-    const uint32_t v = c.vstar;
-    const uint32_t N = ri.N;
-    uint32_t x[MS];
-#pragma unroll
-    for (int s = 0; s < MS; ++s) x[s] = s < n.S ? X[ri.x_off + (uint64_t)s * N + v] : 0u;
-    const int cc = n.C > 1 ? a.comp[ri.comp_off + v] : 0;
-    double av[MR];
-    uint32_t crit[(MR + 31) / 32];
-    react_props<MR, MS>(n, x, cc, a.n_critical, av, crit);
+//
+// Run by a whole wavefront: lane s takes species s, lane j reactions j and
+// j + 64, so that every table entry is requested at once, and the sums then go
+// over the lanes in the network's order, as one lane would form them.  (One
+// reaction after the other, each waiting for its own table entries,
+// commit_decide_kernel took 10.7 us on the 1M-subvolume Brusselator mesh, 8.9
+// now, and 8.5 on 32 meshes in one context, 6.9 now.)
+static __device__ void choose_event(const KernelArgs& a, const RealInfo& ri, RealCtl& c, const uint32_t* X) {
+    const uint32_t v = c.vstar, lane = threadIdx.x & 63u;
+    const int S = a.nh.S, R = a.nh.R, nc = a.n_critical;
+    const int cc = a.nh.C > 1 ? a.comp[ri.comp_off + v] : 0;
     const double W = a.wsum[ri.rp_off + v];
+    HopRow row = hop_row(a, ri, v);
+    const int s = min((int)lane, S - 1);  // (kMaxS = 64 species, one a lane)
+    const uint32_t xs = X[ri.x_off + (uint64_t)s * ri.N + v];
+    const double d = a.net_d[a.nh.off_d + cc * S + s];
+    const uint64_t hops = __ballot((int)lane < S && d > 0.0 && !hop_active(d, xs, nc));
+    const double ao = (d * (double)xs) * W;
+    double aj[2];
+    uint64_t crit[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {  // (kMaxR = 128 reactions)
+        const int j = min((int)lane + 64 * h, R > 0 ? R - 1 : 0);
+        const bool on = (int)lane + 64 * h < R;
+        const int nr = on ? a.net_i[a.nh.off_nrs + j] : 0, order = on ? a.net_i[a.nh.off_order + j] : 0;
+        int sp[3], mu[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            sp[i] = on ? a.net_i[a.nh.off_rs + 3 * j + i] : 0;
+            mu[i] = on ? a.net_i[a.nh.off_rr + 3 * j + i] : 1;
+        }
+        aj[h] = on ? a.net_d[a.nh.off_k + cc * R + j] : 0.0;
+        bool low = false;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const uint32_t x = (uint32_t)__shfl((int)xs, i < nr ? sp[i] : 0);
+            if (i >= nr) continue;
+            aj[h] = aj[h] * binom_d(x, mu[i]);
+            low = low || below_nc(x, mu[i], nc);
+        }
+        crit[h] = __ballot(on && order > 0 && low);
+    }
+    asm volatile("" : "+v"(row.cw));  // (loaded by now, not after the choice)
     double a0c = 0.0;
 #pragma unroll
-    for (int j = 0; j < MR; ++j)
-        if (j < n.R && is_crit<MR>(crit, j)) a0c += av[j];
-#pragma unroll
-    for (int s = 0; s < MS; ++s) {
-        if (s >= n.S) break;
-        const double d = n.d[cc * n.S + s];
-        if (d > 0.0 && !hop_active(d, x[s], a.n_critical)) a0c += (d * (double)x[s]) * W;
-    }
+    for (int h = 0; h < 2; ++h)
+        for (uint64_t m = crit[h]; m != 0ull; m &= m - 1ull) a0c += lane_f64(aj[h], (uint32_t)__builtin_ctzll(m));
+    for (uint64_t m = hops; m != 0ull; m &= m - 1ull) a0c += lane_f64(ao, (uint32_t)__builtin_ctzll(m));
     const U4 o = philox10_u(v, kSelfId, c.step, ctr_word3(ri.id, 0u, kCrit, 0u), a.seed_lo, a.seed_hi);
     const double target = uniform01(o.x) * a0c;
     double acc = 0.0;
-    int kind = 0, idx = -1;
-    for (int j = 0; j < n.R; ++j) {
-        if (!is_crit<MR>(crit, j) || !(av[j] > 0.0)) continue;
-        acc += av[j];
-        idx = j;
-        if (target < acc) { kind = 1; break; }
-    }
-    int lastkind = idx >= 0 ? 1 : 0;
-    if (kind == 0) {
-        for (int s = 0; s < n.S; ++s) {
-            const double d = n.d[cc * n.S + s];
-            if (!(d > 0.0) || hop_active(d, x[s], a.n_critical)) continue;
-            const double ao = (d * (double)x[s]) * W;
-            if (!(ao > 0.0)) continue;
-            acc += ao;
-            idx = s;
-            lastkind = 2;
-            if (target < acc) { kind = 2; break; }
+    int kind = 0, idx = -1, lastkind = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        for (uint64_t m = crit[h] & __ballot(aj[h] > 0.0); m != 0ull && kind == 0; m &= m - 1ull) {
+            const uint32_t l = (uint32_t)__builtin_ctzll(m);
+            acc += lane_f64(aj[h], l);
+            idx = (int)l + 64 * h;
+            lastkind = 1;
+            if (target < acc) kind = 1;
         }
+    for (uint64_t m = hops & __ballot(ao > 0.0); m != 0ull && kind == 0; m &= m - 1ull) {
+        const uint32_t l = (uint32_t)__builtin_ctzll(m);
+        acc += lane_f64(ao, l);
+        idx = (int)l;
+        lastkind = 2;
+        if (target < acc) kind = 2;
     }
     if (kind == 0) kind = lastkind;
     c.ev_kind = kind;
     c.ev_idx = idx;
-    c.ev_dst = kind == 2 ? choose_hop_edge(a, ri, v, uniform01(o.y) * W) : v;
+    c.ev_dst = kind == 2 ? choose_hop_edge(a, ri, v, row.rb, row.re, row.cw, uniform01(o.y) * W) : v;
 }
 
 // ---------------------------------------------------------------------------
@@ -668,7 +708,7 @@ __device__ void finalize_A(const KernelArgs& a, const NetView& n, const RealInfo
     decide(c);
     // the event is needed only if tau'' <= tau' (a leap-back halves tau' and
     // can lift the clamp to t_end, but never makes a larger tau'' fire)
-    if (t2 < kInf && t2 <= tp) choose_event<MS, MR>(a, n, ri, c, count_buf(a, c.cur));
+    if (t2 < kInf && t2 <= tp) choose_event(a, ri, c, count_buf(a, c.cur));
     if (lead) a.ctl[r] = c;
 }
 

@@ -132,6 +132,7 @@ __device__ __forceinline__ long long res_draw(const KernelArgs& a, const ResView
 __device__ void res_choose_event(const KernelArgs& a, const NetView& n, const RealInfo& ri, RealCtl& c,
                                  const double* prop, const uint32_t* x) {
     const uint32_t v = c.vstar, N = ri.N;
+    const HopRow row = hop_row(a, ri, v);
     const int cc = n.C > 1 ? a.comp[ri.comp_off + v] : 0;
     const double W = a.wsum[ri.rp_off + v];
     double a0c = 0.0;
@@ -178,7 +179,7 @@ __device__ void res_choose_event(const KernelArgs& a, const NetView& n, const Re
     if (kind == 0) kind = lastkind;
     c.ev_kind = kind;
     c.ev_idx = idx;
-    c.ev_dst = kind == 2 ? choose_hop_edge(a, ri, v, uniform01(o.y) * W) : v;
+    c.ev_dst = kind == 2 ? choose_hop_edge(a, ri, v, row.rb, row.re, row.cw, uniform01(o.y) * W) : v;
 }
 
 // MODE 0: everything in LDS; 1: the topology stays in global memory; 2: the

@@ -96,3 +96,22 @@ def test_tiles_split_in_a_batch():
         assert np.array_equal(ctx.get_state(r), x)
         assert ctx.stats(r)["firings"] == st.firings and ctx.stats(r)["t"] == st.t
     ctx.close()
+
+
+@pytest.mark.parametrize("S", [2, 40, 64])
+def test_critical_event_over_the_lanes(S):
+    """Up to 64 species and 66 reactions at low counts: every step an event, of
+    reactions in both halves and of hops (a judged context keeps the launches)."""
+    sp = [f"X{i}" for i in range(S)]
+    rx = [({sp[i]: 1}, {sp[(i + 1) % S]: 1}) for i in range(S)] + [({sp[0]: 2}, {sp[1]: 1}), ({sp[0]: 1, sp[1]: 1}, {})]
+    net = W.network(sp, rx, [0.1 + 0.01 * i for i in range(S)] + [0.3, 0.2], [0.3 if i % 3 == 0 else 0.0 for i in range(S)])
+    topo = H.asym_topology(75, 4)
+    x0 = W.poisson_state(S, 75, 3.0, 5)
+    ctx = capi.Context(net, [topo], [x0], seed=3)
+    ctx.set_tau_mode(False, theta=1.0)
+    ctx.run(np.inf, step_limit=150)
+    x = x0.copy()
+    st = ffi.run(ffi.Model(net, topo), x, 0.03, 10, 3, np.inf, step_limit=150)
+    assert st.crit_events > 100 and ctx.stats(0)["crit_events"] == st.crit_events
+    assert np.array_equal(ctx.get_state(0), x) and ctx.stats(0)["t"] == st.t
+    ctx.close()
