@@ -43,10 +43,11 @@ def algorithmic_bytes(S, topos, part):
     """Compulsory HBM bytes of one launch: what the kernel must read and
     write once.  part: "tau" (phase_a_kernel: counts, CSR row pointers,
     neighbour ids and weights), "leap" (the whole leap pass: counts in and
-    out plus the topology once), "leap_kernel" (phase_b_kernel of the
+    out plus the topology once), "leap_draws" (phase_b_kernel of the
     edge-parallel pass: counts, the forward CSR -- each undirected edge once
-    -- and the 64-bit balances it produces), "finish" (phase_b_finish_kernel:
-    counts and balances in, new counts out), "step" (one whole step:
+    -- and the 32-bit balances it adds), "leap_kernel" and "finish" (the pass
+    with 64-bit balances in an array of their own, and the kernel that adds
+    them to the counts), "step" (one whole step:
     N (12 S + 10) + 2 topology)."""
     tot = 0
     for t in topos:
@@ -59,6 +60,8 @@ def algorithmic_bytes(S, topos, part):
             tot += 8 * S * N + 4 * (N + 1) + 4 * E + (4 * E if wt else 0)
         elif part == "leap_kernel":
             tot += 4 * S * N + 4 * (N + 1) + 2 * E + (2 * E if wt else 0) + 8 * S * N
+        elif part == "leap_draws":
+            tot += 4 * S * N + 4 * (N + 1) + 2 * E + (2 * E if wt else 0) + 4 * S * N
         elif part == "finish":
             tot += 4 * S * N + 8 * S * N + 4 * S * N
         elif part == "step":
@@ -397,13 +400,11 @@ def main():
     value = res["subvolume_leaps"] / res["seconds"]
     bytes_leap = algorithmic_bytes(S, wl["topos"], "leap")
     bytes_tau = algorithmic_bytes(S, wl["topos"], "tau")
-    split = res["finish_ms"] > 0.0  # edge-parallel leap pass: three kernels
+    split = S <= 8 and wl["net"]["R"] <= 16  # edge-parallel leap pass
     # the roofline is taken on the single kernel with the longest launches
     cand = {"phase_a_kernel": (res["tau_ms"], bytes_tau),
             "phase_b_kernel": (res["leap_kernel_ms"],
-                               algorithmic_bytes(S, wl["topos"], "leap_kernel" if split else "leap"))}
-    if split:
-        cand["phase_b_finish_kernel"] = (res["finish_ms"], algorithmic_bytes(S, wl["topos"], "finish"))
+                               algorithmic_bytes(S, wl["topos"], "leap_draws" if split else "leap"))}
     kname = max(cand, key=lambda k: cand[k][0])
     dom_ms, dom_bytes = cand[kname]
     achieved = dom_bytes / (dom_ms * 1e-3) / 1e9
@@ -442,8 +443,7 @@ def main():
                     "tau_GBs": bytes_tau / (res["tau_ms"] * 1e-3) / 1e9,
                     "leap_GBs": bytes_leap / (res["leap_ms"] * 1e-3) / 1e9,
                     "leap_pass_split_ms_avg": {"phase_b_kernel": res["leap_kernel_ms"],
-                                               "phase_b_redo_kernel": res["redo_ms"],
-                                               "phase_b_finish_kernel": res["finish_ms"]},
+                                               "completion": res["finish_ms"]},
                     "per_kernel_GBs": {k: b / (ms * 1e-3) / 1e9 for k, (ms, b) in cand.items() if ms > 0}},
         "step_roofline": {"B_step": b_step, "achieved": b_step_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                           "frac": b_step_gbs / HBM_PEAK_GBS},

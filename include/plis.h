@@ -136,7 +136,8 @@ int plis_profile(plis_ctx *ctx, uint32_t n, double *out);
 
 /* As plis_profile, with the leap pass split by kernel: out[0..4] as there,
  * out[5] = phase_b_kernel, out[6] = 0 (a pass that no longer exists), out[7] =
- * phase_b_finish_kernel (summed ms).  A context with the per-subvolume leap
+ * the kernel that completes the leap in learned and judged contexts (summed
+ * ms; next to 0 with plain tau, where the tau pass does).  A context with the per-subvolume leap
  * kernel (more than 8 species or 16 reactions) reports it in out[5] and 0 in
  * out[7].  Small realizations, whose steps run inside one kernel otherwise,
  * are stepped with a launch per pass here.  Diagnostics of this

@@ -1,22 +1,22 @@
 // plis_kernels.hip -- gfx950 kernels for the RDME tau-leap + SSA step.
 //
-// One global step of one realization is two persistent kernels:
-//   phase A (tau): per subvolume FP64 mass-action propensities, Cao tau' with
-//     hops treated as first-order channels, the critical set and an
-//     exponential tau'' clock; a wave-shuffle min/argmin per 64-subvolume
-//     tile written as a tile partial; a one-block-per-realization decide
-//     kernel reduces the partials and decides the step (tau, critical event).  Replaces compute_rates
-//     (PLISCuda/src/rates.cu:82-96), compute_taus (tau.cu:197-251) and the
-//     host thrust::min_element + tau[i] round trips (driver.cu:267-277).
-//   phase B (leap): per subvolume Poisson firings of non-critical reactions,
-//     gather-form diffusion (each subvolume regenerates its in-neighbours'
-//     hop counts from the same counter-based Philox draw the sender used, so
-//     there are no atomics on counts), the critical event of the argmin
-//     subvolume, and the negative-population check; a one-block-per-
-//     realization commit kernel accepts the step or leaps back (tau' halved,
-//     new attempt index).  Replaces
-//     leap_step (leap.cu:3-201), ssa_step (ssa.cu:56-110), check_state +
-//     none_of + revert (leap.cu:203-212, driver.cu:292-323).
+// One global step of one realization is three kernels:
+//   the leap (phase_b_kernel): Poisson firings of non-critical reactions and
+//     hops, every linked pair drawn once by the tile of its lower end from a
+//     counter-based Philox draw, integer balances added to a copy of the
+//     counts, and the critical event.  Replaces leap_step (leap.cu:3-201) and
+//     ssa_step (ssa.cu:56-110).
+//   the tau pass on the counts the leap wrote (phase_a_kernel): per subvolume
+//     FP64 mass-action propensities, Cao tau' with hops treated as first-order
+//     channels, the critical set and an exponential tau'' clock, min / argmin
+//     per 64-subvolume tile as a tile partial; and the range check of the new
+//     counts (check_state + none_of, leap.cu:203-212, driver.cu:292-323).
+//     Replaces compute_rates (PLISCuda/src/rates.cu:82-96) and compute_taus
+//     (tau.cu:197-251).
+//   commit_decide_kernel: reduces the partials, commits the step or leaps back
+//     (tau' halved, new attempt index) and decides the next one.  Replaces the
+//     host's thrust::min_element + tau[i] round trips and the revert
+//     (driver.cu:267-277, 292-323).
 //
 // Wavefront-per-tile: lane i of a wave owns subvolume v0+i of its tile;
 // species-major counts make every per-species load and store one coalesced
