@@ -861,13 +861,15 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         plis_destroy(c);
         return rc;
     }
-    if (ep && ((rc = dev_alloc(c, &c->d_gdelta, hx.size())) ||
-               (rc = upload(c, &c->d_wide, std::vector<uint32_t>(c->ntiles, 0u))) || (any_asym && (rc = upload(c, &c->d_frw, hfrw))))) {
+    // (the tiles' flags behind the wide balances: one allocation, cleared together)
+    const size_t wide_words = hx.size() + ((size_t)c->ntiles + 1) / 2;
+    if (ep && ((rc = dev_alloc(c, &c->d_gdelta, wide_words)) || (any_asym && (rc = upload(c, &c->d_frw, hfrw))))) {
         g_create_err = c->err;
         plis_destroy(c);
         return rc;
     }
-    if (ep && (hipMemsetAsync(c->d_gdelta, 0, hx.size() * sizeof(unsigned long long), c->stream) != hipSuccess ||
+    if (ep) c->d_wide = reinterpret_cast<uint32_t*>(c->d_gdelta + hx.size());
+    if (ep && (hipMemsetAsync(c->d_gdelta, 0, wide_words * sizeof(unsigned long long), c->stream) != hipSuccess ||
                hipStreamSynchronize(c->stream) != hipSuccess)) {
         g_create_err = "clearing the balances failed";
         plis_destroy(c);
