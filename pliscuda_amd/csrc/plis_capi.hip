@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/plis.h"
+#include "plis_dispatch.h"
 #include "plis_launch.h"
 #include "plis_mlp.hip"
 #include "plis_resident.h"
@@ -575,31 +576,19 @@ extern "C" void plis_destroy(plis_ctx* c) {
     delete c;
 }
 
-// Whether every realization of the context is small enough for
-// resident_kernel, and its launch shape.
+// Whether the context's realizations step in one block each (resident_pays),
+// and the kernel's launch shape.
 static bool resident_fit(plis_ctx* c, const NetHeader& h, const std::vector<double>& D, const ResLists& l,
                          const std::vector<uint32_t>& frp, bool huge) {
     uint64_t maxN = 0, nf = 0, ne = 0;
+    std::vector<StepSize> sizes;
     for (const auto& ri : c->info) {
+        sizes.push_back({ri.N, ri.n_in, ri.ntiles});
         maxN = std::max<uint64_t>(maxN, ri.N);
         nf = std::max<uint64_t>(nf, frp[ri.rp_off + ri.N]);
         ne = std::max<uint64_t>(ne, ri.n_in);
     }
     if (huge || maxN > kResidentMaxN) return false;
-    // One CU makes a step of N subvolumes in about 5 us + N (2 + 0.84 S deg +
-    // 2.8 R) ns (measured: A-B-C 7.6 us at 64, 15 at 512, 26 at 1,000, 41 at
-    // 1,728; diffusion of one species 21 at 1,728; Brusselator mesh 25 at 512,
-    // 50 at 1,000).  The launch-per-pass step takes 18 us with one species, 22
-    // with the three of A-B-C and 30 with the Brusselator's five at these sizes
-    // (both sides measured: bistable 18.7 / 19.1 us at 729; A-B-C 19.3 / 21.9
-    // at 729, 25.4 / 21.9 at 1,000; diffusion 14.1 / 18.0 at 1,000, 20.1 / 18.9
-    // at 1,728; Brusselator 23.5 / 29.8 at 512), and 730 us or more in its
-    // general instantiation (cascade of 32 species, 62 reactions: 17 us here at
-    // 60 subvolumes, 165 at 1,000).  The line lies where the two meet.
-    double est = 0.0;
-    for (const auto& ri : c->info)
-        est = std::max(est, 1e-3 * (ri.N * (2.0 + 2.8 * h.R) + 0.84 * h.S * (double)ri.n_in));
-    if (est > (c->variant > 3 ? 600.0 : 10.5 + 4.0 * h.S)) return false;
     // wavefronts: one per item of the widest phase, 4 to 16
     const uint64_t nt = (maxN + 63) / 64;
     const uint64_t items = std::max<uint64_t>(nt * std::max(h.S + 1, h.R), (nf + 63) / 64 * ((h.S + 7) / 8) + nt * ((h.R + 3) / 4));
@@ -608,6 +597,8 @@ static bool resident_fit(plis_ctx* c, const NetHeader& h, const std::vector<doub
     if (b.tables > 64 * 1024) return false;
     c->res_mode = b.tables + b.arrays + b.topology <= kResidentLdsMax ? 0 : b.tables + b.arrays <= kResidentLdsMax ? 1 : 2;
     c->res_lds = (uint32_t)(b.tables + (c->res_mode <= 1 ? b.arrays : 0) + (c->res_mode == 0 ? b.topology : 0));
+    const uint64_t slots = resident_blocks_per_cu(c->res_waves, c->res_lds) * (uint64_t)c->cus;
+    if (!resident_pays(h.S, h.R, c->variant > 3, sizes, slots)) return false;
     c->res.ws_slice = c->res_mode == 2 ? (b.arrays + 255) & ~255ull : 0;
     c->res.nspe = (uint32_t)l.spe.size();
     for (int s = 0; s < h.S; ++s)
