@@ -111,7 +111,7 @@ struct plis_ctx {
     bool sourced = false;  // no realization can run out of events (has_source)
     // steps of small realizations inside one block each (resident_kernel)
     bool resident_fits = false;
-    uint32_t res_waves = 0, res_lds = 0;
+    uint32_t res_waves = 0, res_lds = 0, res_iters = 1;  // res_iters: iterations of a launch
     int res_mode = 0;
     ResidentArgs res{};
     bool edge_parallel = false;  // at most 8 species and 16 reactions, tiles < 2^19 forward entries
@@ -599,6 +599,7 @@ static bool resident_fit(plis_ctx* c, const NetHeader& h, const std::vector<doub
     c->res_lds = (uint32_t)(b.tables + (c->res_mode <= 1 ? b.arrays : 0) + (c->res_mode == 0 ? b.topology : 0));
     const uint64_t slots = resident_blocks_per_cu(c->res_waves, c->res_lds) * (uint64_t)c->cus;
     if (!resident_pays(h.S, h.R, c->variant > 3, sizes, slots)) return false;
+    c->res_iters = resident_launch_iters(resident_step_us(h.S, h.R, sizes, slots));
     c->res.ws_slice = c->res_mode == 2 ? (b.arrays + 255) & ~255ull : 0;
     c->res.nspe = (uint32_t)l.spe.size();
     for (int s = 0; s < h.S; ++s)
@@ -615,9 +616,8 @@ static int resident_iters(plis_ctx* c, uint32_t n) {
     a.k = make_args(c);
     a.k.ep = 0u;  // two count buffers
     c->ctl_fresh = false;
-    // (a launch makes at most 4,096 iterations, some tens of milliseconds)
     while (n > 0) {
-        a.iters = std::min(n, 4096u);
+        a.iters = std::min(n, c->res_iters);
         HIPCHK(c, launch_resident(c->stream, c->nreal, c->res_waves, c->res_lds, c->res_mode, a));
         n -= a.iters;
     }
@@ -1059,7 +1059,7 @@ extern "C" int plis_run_until(plis_ctx* c, double t_end, double t_pause, uint64_
             if (int rc = pull_ctl(c)) return rc;
             left = std::max<uint64_t>(1, to_limit());
         }
-        const uint32_t n = res ? 1024u : (uint32_t)std::min<uint64_t>(k, left);
+        const uint32_t n = res ? c->res_iters : (uint32_t)std::min<uint64_t>(k, left);
         if (int rc = res ? resident_iters(c, n) : graph_iters(c, n)) return rc;
         HIPCHK(c, hipMemcpyAsync(c->h_ndone, d_ndone, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));

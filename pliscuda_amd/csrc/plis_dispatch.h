@@ -82,4 +82,12 @@ inline bool resident_pays(int S, int R, bool general, const std::vector<StepSize
     return resident_step_us(S, R, rs, slots) <= 14.0 + 3.0 * S + 1e-3 * (double)tiles * (2.3 + 0.5 * (S + R));
 }
 
+// Iterations of one launch that make `us` an iteration: some 50 ms, so that the
+// host sees the realizations' progress and a wait for the stream stays short
+// (4,096 at the general line of 600 us would take 2.5 s).  At most 1,024, which
+// the smallest boxes make in 8 ms.
+inline uint32_t resident_launch_iters(double us) {
+    return (uint32_t)std::min(1024.0, std::max(1.0, 50e3 / us));
+}
+
 }  // namespace plis

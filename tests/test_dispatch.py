@@ -4,6 +4,7 @@ import os
 import shutil
 import subprocess
 
+import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -25,8 +26,8 @@ int main() {
             r = {N, E, (N + 63) / 64};
         }
         for (unsigned long i = 0; i < count; ++i) rs.push_back(k[i % kinds]);
-        std::printf("%d %.3f\n", (int)resident_pays(S, R, general != 0, rs, 256 * per_cu),
-                    resident_step_us(S, R, rs, 256 * per_cu));
+        const double us = resident_step_us(S, R, rs, 256 * per_cu);
+        std::printf("%d %.3f %u\n", (int)resident_pays(S, R, general != 0, rs, 256 * per_cu), us, resident_launch_iters(us));
     }
 }
 """
@@ -46,7 +47,7 @@ def rule(tmp_path_factory):
         line = " ".join(str(v) for v in (S, R, int(general), count, per_cu, len(sizes))) + " "
         out = subprocess.run([str(d / "rule")], input=line + " ".join(f"{n} {e}" for n, e in sizes), capture_output=True,
                              text=True, check=True).stdout.split()
-        return out[0] == "1", float(out[1])
+        return out[0] == "1", float(out[1]), int(out[2])
 
     return ask
 
@@ -83,7 +84,45 @@ def test_uneven_realizations_are_scheduled_one_after_the_other(rule):
     latest when the first small one has ended, so the step lasts no longer than
     the two together, not two rounds of the large one."""
     large, small = rule(3, 3, False, 1, 1, (700, 3700))[1], rule(3, 3, False, 1, 1, (8, 24))[1]
-    pays, us = rule(3, 3, False, 320, 1, (700, 3700), *[(8, 24)] * 9)
+    pays, us, _ = rule(3, 3, False, 320, 1, (700, 3700), *[(8, 24)] * 9)
     assert pays and us == pytest.approx(large + small, rel=1e-3) and us < 1.5 * large
     assert rule(3, 3, False, 256, 1, (700, 3700))[1] == pytest.approx(large, rel=1e-3)
     assert rule(3, 3, False, 257, 1, (700, 3700))[1] == pytest.approx(2 * large, rel=1e-3)
+
+
+@pytest.mark.parametrize("S,R,general,size,count", [
+    (1, 1, False, (1, 0), 1), (3, 3, False, (64, 288), 1), (3, 3, False, (900, 4900), 256), (32, 62, True, (60, 118), 1),
+    (32, 62, True, (60, 118), 65536), (32, 62, True, (2600, 5198), 1), (64, 128, True, (1200, 2398), 5000)])
+def test_a_launch_of_one_block_kernels_is_short(rule, S, R, general, size, count):
+    """About 50 ms however large the network and however many the realizations, and
+    no shorter than it has to be."""
+    pays, us, iters = rule(S, R, general, count, 1, size)
+    assert pays and 1 <= iters <= 1024
+    assert iters == 1 or iters * us <= 50e3
+    assert iters == 1024 or (iters + 1) * us > 50e3
+
+
+@pytest.mark.gpu
+def test_a_call_of_several_launches():
+    """38 species, 40 reactions on 900 subvolumes: a launch makes some 480 iterations.
+    One call of 700 equals a launch per pass, which evaluates the leap condition."""
+    from pliscuda_amd import capi
+    from pliscuda_amd import workloads as W
+
+    S = 38
+    sp = [f"X{i}" for i in range(S)]
+    rx = [({sp[i]: 1}, {sp[(i + 1) % S]: 1}) for i in range(S)] + [({sp[0]: 1, sp[1]: 1}, {sp[2]: 1}), ({}, {sp[0]: 2})]
+    net = W.network(sp, rx, [0.4] * S + [2e-3, 3.0], [0.5 if i % 3 == 0 else 0.0 for i in range(S)])
+    topo = W.cubic_grid(900, 1, 1, periodic=False)
+    x0 = W.poisson_state(S, 900, 30.0, 7)
+    out = []
+    for theta in (0.0, 1.0):
+        ctx = capi.Context(net, [topo], [x0], seed=4)
+        ctx.set_tau_mode(False, theta=theta)
+        ctx.arm(step_limit=700)
+        ctx.iterate(700)
+        out.append((ctx.get_state(0), ctx.stats(0)))
+        ctx.close()
+    (xa, sa), (xb, sb) = out
+    assert np.array_equal(xa, xb) and all(sa[f] == sb[f] for f in ("t", "steps", "leapbacks", "firings", "crit_events"))
+    assert sa["steps"] + sa["leapbacks"] == 700
