@@ -74,7 +74,7 @@ struct plis_ctx {
     std::vector<RealInfo> info;
     std::vector<RealCtl> ctl_host;
     bool ctl_fresh = false;  // ctl_host equals the device's controls, nothing launched since
-    char* h_stage = nullptr;  // pinned, two halves of stage_half bytes (fetch)
+    char* h_stage = nullptr;  // pinned, two halves of stage_half bytes (upload, fetch), then h_ndone
     size_t stage_half = 0;
     hipEvent_t stage_ev[2] = {};
     // device buffers
@@ -102,7 +102,7 @@ struct plis_ctx {
     uint32_t* d_dcnt = nullptr;   // decide_kernel's per-realization chunk counters
     PartB* d_pb_t = nullptr;
     uint32_t* d_cnt = nullptr;   // [0] realizations done, [2..3] tiles beyond a wavefront's queue (u64)
-    uint32_t* h_ndone = nullptr;  // pinned
+    uint32_t* h_ndone = nullptr;
     double eps = 0.03;
     int32_t nc = 10;
     uint64_t seed = 0;
@@ -151,10 +151,16 @@ static int dev_alloc(plis_ctx* c, T** p, size_t n) {
     return 0;
 }
 
+// (hipMemcpy takes 110 us for 256 KB of pageable memory, 19 through the pinned
+// buffer; from 512 KB on there is no difference)
 template <typename T>
 static int upload(plis_ctx* c, T** p, const std::vector<T>& v) {
+    const size_t bytes = v.size() * sizeof(T);
     if (int rc = dev_alloc(c, p, v.size())) return rc;
-    if (!v.empty()) HIPCHK(c, hipMemcpy(*p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+    if (bytes == 0) return 0;
+    const bool staged = bytes <= 2 * c->stage_half;
+    if (staged) std::memcpy(c->h_stage, v.data(), bytes);
+    HIPCHK(c, hipMemcpy(*p, staged ? (const void*)c->h_stage : v.data(), bytes, hipMemcpyHostToDevice));
     return 0;
 }
 
@@ -199,6 +205,20 @@ static bool canonical_csr(const plis_topology& t, Csr& out, std::string& err) {
     for (uint32_t v = 0; v < N; ++v) {
         const uint32_t b = t.row_ptr[v], e = t.row_ptr[v + 1];
         if (e < b || e > t.n_edges) { err = "row_ptr not monotone or beyond n_edges"; return false; }
+        // a row in its canonical form already is copied as it stands
+        const size_t at = out.col.size();
+        uint32_t q0 = b;
+        for (; q0 < e; ++q0) {
+            const uint32_t u = t.col[q0];
+            const float wq = t.weight ? t.weight[q0] : 1.0f;
+            if (u >= N || u == v || (q0 > b && u <= t.col[q0 - 1]) || !(wq > 0.0f) || !std::isfinite(wq)) break;
+            out.col.push_back(u);
+            out.w.push_back(wq);
+        }
+        out.rp[v] = (uint32_t)at;
+        if (q0 == e) continue;
+        out.col.resize(at);
+        out.w.resize(at);
         tmp.clear();
         for (uint32_t q = b; q < e; ++q) {
             const uint32_t u = t.col[q];
@@ -211,7 +231,6 @@ static bool canonical_csr(const plis_topology& t, Csr& out, std::string& err) {
         std::sort(tmp.begin(), tmp.end(), [](const Nb& x, const Nb& y) {
             return x.id != y.id ? x.id < y.id : x.pos < y.pos;
         });
-        out.rp[v] = (uint32_t)out.col.size();
         for (size_t i = 0; i < tmp.size();) {
             size_t i2 = i;
             double acc = 0.0;
@@ -225,14 +244,14 @@ static bool canonical_csr(const plis_topology& t, Csr& out, std::string& err) {
     return true;
 }
 
+// Rows are ascending, so with v ascending too the edges v -> u meet the entries
+// of row u in their order, one after the other, if every edge has its reverse.
 static bool is_symmetric(const Csr& g, uint32_t N) {
+    std::vector<uint32_t> next(g.rp.begin(), g.rp.end() - 1);  // row u's first entry without its reverse so far
     for (uint32_t v = 0; v < N; ++v)
         for (uint32_t q = g.rp[v]; q < g.rp[v + 1]; ++q) {
-            const uint32_t u = g.col[q];
-            auto b = g.col.begin() + g.rp[u], e = g.col.begin() + g.rp[u + 1];
-            auto it = std::lower_bound(b, e, v);
-            if (it == e || *it != v) return false;
-            if (g.w[it - g.col.begin()] != g.w[q]) return false;
+            const uint32_t u = g.col[q], e = next[u]++;
+            if (e >= g.rp[u + 1] || g.col[e] != v || g.w[e] != g.w[q]) return false;
         }
     return true;
 }
@@ -568,7 +587,6 @@ extern "C" void plis_destroy(plis_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     drop_graphs(c);
     for (void* p : c->allocs) (void)hipFree(p);
-    if (c->h_ndone) (void)hipHostFree(c->h_ndone);
     if (c->h_stage) (void)hipHostFree(c->h_stage);
     for (auto e : c->stage_ev)
         if (e) (void)hipEventDestroy(e);
@@ -670,8 +688,6 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         std::memcpy(&w, &b, 4);
         return w;
     };
-    bool small = true;  // every realization so far may be stepped by resident_kernel
-    std::vector<uint32_t> hfsrc;
     std::vector<float> hfrw;
     auto idw = [](uint32_t u, float w) {
         uint32_t b;
@@ -713,34 +729,44 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         hcol.insert(hcol.end(), g.col.begin(), g.col.end());
         Csr in;
         if (!sym) transpose(g, N, in);
-        small = small && N <= kResidentMaxN;
         // forward CSR: each pair of linked subvolumes once, in the row of its
         // lower end, with the weights of both hops (an asymmetric topology's
         // may differ, or one of them be absent: weight 0)
         ri.fe_off = hfcw.size();
-        if (!sym)  // the first asymmetric realization: the weights back of those before it
+        const bool back = !sym || any_asym;
+        if (back && !any_asym)  // the first asymmetric realization: the weights back of those before it
             for (size_t e = hfrw.size(); e < ri.fe_off; ++e) hfrw.push_back(weight_of(hfcw[e]));
+        // (as many pairs as there may be at most: half the edges, or all of them)
+        const size_t most = sym ? g.col.size() / 2 : g.col.size();
+        hfcw.resize(ri.fe_off + most);
+        if (back) hfrw.resize(ri.fe_off + most);
+        uint64_t* const fe = hfcw.data() + ri.fe_off;
+        float* const fb = back ? hfrw.data() + ri.fe_off : nullptr;
+        uint32_t nfe = 0;
         for (uint32_t v = 0; v < N; ++v) {
-            hfrp.push_back((uint32_t)(hfcw.size() - ri.fe_off));
+            hfrp.push_back(nfe);
             auto put = [&](uint32_t u, float wf, float wr) {
-                hfcw.push_back(idw((u & kFwdIdMask) | ((v % kTile) << 26), wf));
-                if (small) hfsrc.push_back(v);
-                if (!sym || any_asym) hfrw.push_back(wr);
+                fe[nfe] = idw((u & kFwdIdMask) | ((v % kTile) << 26), wf);
+                if (back) fb[nfe] = wr;
+                ++nfe;
             };
-            uint32_t q = g.rp[v], qe = g.rp[v + 1];
+            const uint32_t qe = g.rp[v + 1];
+            uint32_t q = (uint32_t)(std::upper_bound(g.col.begin() + g.rp[v], g.col.begin() + qe, v) - g.col.begin());
             if (sym) {
-                for (; q < qe; ++q)
-                    if (g.col[q] > v) put(g.col[q], g.w[q], g.w[q]);
+                for (; q < qe; ++q) put(g.col[q], g.w[q], g.w[q]);
                 continue;
             }
-            uint32_t p = in.rp[v], pe = in.rp[v + 1];
+            const uint32_t pe = in.rp[v + 1];
+            uint32_t p = (uint32_t)(std::upper_bound(in.col.begin() + in.rp[v], in.col.begin() + pe, v) - in.col.begin());
             while (q < qe || p < pe) {  // merge the out-row and the in-row, both ascending
                 const uint32_t uo = q < qe ? g.col[q] : UINT32_MAX, ui = p < pe ? in.col[p] : UINT32_MAX;
                 const uint32_t u = std::min(uo, ui);
                 const float wf = uo == u ? g.w[q++] : 0.0f, wr = ui == u ? in.w[p++] : 0.0f;
-                if (u > v) put(u, wf, wr);
+                put(u, wf, wr);
             }
         }
+        hfcw.resize(ri.fe_off + nfe);
+        if (back) hfrw.resize(ri.fe_off + nfe);
         hfrp.push_back((uint32_t)(hfcw.size() - ri.fe_off));
         // a subvolume's balances below `narrow` must add up to less than 2^31:
         // it takes part in at most two hops of a species per neighbour, 16
@@ -752,7 +778,12 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         for (uint32_t v = 0; v < N; v += kTile)  // entry offsets of a tile's queue codes
             if (hfrp[rpoff + std::min(v + (uint32_t)kTile, N)] - hfrp[rpoff + v] >= kMaxTileEdges) huge_tile = true;
         hw.insert(hw.end(), g.w.begin(), g.w.end());
-        for (size_t q = 0; q < g.col.size(); ++q) hcw.push_back(idw(g.col[q], g.w[q]));
+        auto interleave = [&](std::vector<uint64_t>& to, const Csr& m) {
+            const size_t at = to.size();
+            to.resize(at + m.col.size());
+            for (size_t q = 0; q < m.col.size(); ++q) to[at + q] = idw(m.col[q], m.w[q]);
+        };
+        interleave(hcw, g);
         // W_v = sum of out-edge weights, summed in CSR order in double
         for (uint32_t v = 0; v < N; ++v) {
             double W = 0.0;
@@ -767,7 +798,7 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
             hirp.insert(hirp.end(), in.rp.begin(), in.rp.end());
             hicol.insert(hicol.end(), in.col.begin(), in.col.end());
             hiw.insert(hiw.end(), in.w.begin(), in.w.end());
-            for (size_t q = 0; q < in.col.size(); ++q) hicw.push_back(idw(in.col[q], in.w[q]));
+            interleave(hicw, in);
             ieoff += in.col.size();
             irpoff += N + 1;
         } else {
@@ -826,6 +857,16 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         g_create_err = "hipStreamCreate failed";
         return PLIS_ERR_HIP;
     }
+    // (an allocation of pinned memory takes the same 14 us at any of these sizes)
+    c->stage_half = std::min<size_t>(1u << 21, std::max<size_t>(1u << 18, ((size_t)c->total_counts * 4 + 4095) & ~(size_t)4095));
+    bool staging = hipHostMalloc((void**)&c->h_stage, 2 * c->stage_half + sizeof(uint32_t)) == hipSuccess;
+    for (auto& e : c->stage_ev) staging = staging && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    if (!staging) {
+        g_create_err = "hipHostMalloc failed";
+        plis_destroy(c);
+        return PLIS_ERR_HIP;
+    }
+    c->h_ndone = reinterpret_cast<uint32_t*>(c->h_stage + 2 * c->stage_half);
     c->ctl_host.resize(n_real);
     for (auto& rc : c->ctl_host) {
         rc = RealCtl{};
@@ -887,18 +928,26 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         return PLIS_ERR_HIP;
     }
     if (c->resident_fits) {
-        std::vector<uint4> fwd(hfcw.size());
-        for (size_t e = 0; e < fwd.size(); ++e) {
-            uint32_t back = (uint32_t)(hfcw[e] >> 32);
-            if (any_asym) std::memcpy(&back, &hfrw[e], 4);
-            fwd[e] = {(uint32_t)hfcw[e] & kFwdIdMask, (uint32_t)(hfcw[e] >> 32), hfsrc[e], back};
-        }
-        int4* rx = nullptr;
-        int2 *sp = nullptr, *spe = nullptr, *jp = nullptr, *jpe = nullptr, *hm = nullptr;
-        uint4* fw = nullptr;
-        if ((rc = upload(c, &rx, lists.rx)) || (rc = upload(c, &sp, lists.sp)) || (rc = upload(c, &spe, lists.spe)) ||
-            (rc = upload(c, &jp, lists.jp)) || (rc = upload(c, &jpe, lists.jpe)) || (rc = upload(c, &hm, lists.hm)) ||
-            (rc = upload(c, &fw, fwd)) ||
+        // one block of device memory for its tables: seven small ones took 0.1 ms
+        std::vector<uint4> host;
+        auto put = [&](const auto& v) {
+            const size_t at = host.size(), bytes = v.size() * sizeof(v[0]);
+            host.resize(at + (bytes + sizeof(uint4) - 1) / sizeof(uint4));
+            if (bytes) std::memcpy(host.data() + at, v.data(), bytes);
+            return at;
+        };
+        const size_t rx = put(lists.rx), sp = put(lists.sp), spe = put(lists.spe), jp = put(lists.jp),
+                     jpe = put(lists.jpe), hm = put(lists.hm), fwd = host.size();
+        host.resize(fwd + hfcw.size());
+        for (const auto& ri : c->info)
+            for (uint32_t v = 0; v < ri.N; ++v)
+                for (uint64_t e = ri.fe_off + hfrp[ri.rp_off + v]; e < ri.fe_off + hfrp[ri.rp_off + v + 1]; ++e) {
+                    uint32_t back = (uint32_t)(hfcw[e] >> 32);
+                    if (any_asym) std::memcpy(&back, &hfrw[e], 4);
+                    host[fwd + e] = {(uint32_t)hfcw[e] & kFwdIdMask, (uint32_t)(hfcw[e] >> 32), v, back};
+                }
+        uint4* dev = nullptr;
+        if ((rc = upload(c, &dev, host)) ||
             (c->res.ws_slice && (rc = dev_alloc(c, &c->res.ws, c->res.ws_slice * c->nreal)))) {
             g_create_err = c->err;
             plis_destroy(c);
@@ -910,20 +959,15 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
             plis_destroy(c);
             return PLIS_ERR_HIP;
         }
-        c->res.rx = rx;
-        c->res.sp = sp;
-        c->res.spe = spe;
-        c->res.jp = jp;
-        c->res.jpe = jpe;
-        c->res.hm = hm;
-        c->res.fwd = fw;
+        c->res.rx = reinterpret_cast<const int4*>(dev + rx);
+        c->res.sp = reinterpret_cast<const int2*>(dev + sp);
+        c->res.spe = reinterpret_cast<const int2*>(dev + spe);
+        c->res.jp = reinterpret_cast<const int2*>(dev + jp);
+        c->res.jpe = reinterpret_cast<const int2*>(dev + jpe);
+        c->res.hm = reinterpret_cast<const int2*>(dev + hm);
+        c->res.fwd = dev + fwd;
     }
     c->edge_parallel = ep;
-    if (hipHostMalloc((void**)&c->h_ndone, sizeof(uint32_t)) != hipSuccess) {
-        g_create_err = "hipHostMalloc failed";
-        plis_destroy(c);
-        return PLIS_ERR_HIP;
-    }
     // 16 blocks of 4 waves per CU unless told otherwise: about one tile per
     // wave, so that tiles start as others end (Brusselator mesh of 1,048,576
     // subvolumes 203 us a step with 4 blocks per CU, 193 with 8, 185 with 16;
@@ -953,12 +997,6 @@ static int pull_ctl(plis_ctx* c) {
 // of one half overlaps the copy out of the other.  (hipMemcpy to pageable
 // memory stages too, but one piece at a time and with its own launch.)
 static int fetch(plis_ctx* c, void* to, const void* from, size_t bytes) {
-    if (!c->h_stage) {
-        const size_t half = std::min<size_t>(1u << 21, ((size_t)c->total_counts * sizeof(uint32_t) + 4095) & ~(size_t)4095);
-        HIPCHK(c, hipHostMalloc((void**)&c->h_stage, 2 * half));
-        c->stage_half = half;
-        for (auto& e : c->stage_ev) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
     char* dst = static_cast<char*>(to);
     const char* src = static_cast<const char*>(from);
     size_t sent = 0, done = 0;
