@@ -164,6 +164,19 @@ static int upload(plis_ctx* c, T** p, const std::vector<T>& v) {
     return 0;
 }
 
+// Gives back what was allocated since there were `mark` allocations.
+static void release_to(plis_ctx* c, size_t mark) {
+    for (; c->allocs.size() > mark; c->allocs.pop_back()) (void)hipFree(c->allocs.back());
+    (void)hipGetLastError();  // (of the allocation that failed)
+}
+
+// Whether the device has 1 GiB left, for kernels' scratch memory, training or
+// another context.
+static bool memory_left() {
+    size_t left = 0, all = 0;
+    return hipMemGetInfo(&left, &all) == hipSuccess && left >= 1ull << 30;
+}
+
 static int fail_create(const std::string& m) {
     g_create_err = m;
     return PLIS_ERR_ARG;
@@ -876,13 +889,13 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         rc.ev_idx = -1;
         rc.tgt = 1u;
     }
-    const bool ep = !huge_tile && c->variant <= 3;
+    bool ep = !huge_tile && c->variant <= 3;
     int rc = 0;
     std::vector<uint32_t> zeros_cnt(4, 0u);
     if ((rc = upload(c, &c->d_net_i, I)) || (rc = upload(c, &c->d_net_d, D)) ||
         (rc = upload(c, &c->d_info, c->info)) || (rc = upload(c, &c->d_ctl, c->ctl_host)) ||
         (rc = upload(c, &c->d_tiles, tiles)) ||
-        (rc = dev_alloc(c, &c->d_x, (ep ? 4 : 2) * hx.size())) || (rc = upload(c, &c->d_rp, hrp)) ||
+        (rc = upload(c, &c->d_rp, hrp)) ||
         (rc = upload(c, &c->d_wsum, hwsum)) ||
         (rc = upload(c, &c->d_col, hcol)) ||
         (rc = upload(c, &c->d_w, any_weighted ? hw : std::vector<float>())) ||
@@ -898,27 +911,33 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         plis_destroy(c);
         return rc;
     }
+    // The edge-parallel leap takes 24 bytes a count and the forward CSR, the
+    // per-subvolume leap 8 and no more.  Where the device does not have the
+    // former to spare the context takes the latter, with the same results.
+    // (the tiles' flags behind the wide balances: one allocation, cleared together)
+    const size_t wide_words = hx.size() + ((size_t)c->ntiles + 1) / 2;
+    if (ep) {
+        const size_t mark = c->allocs.size();
+        ep = !dev_alloc(c, &c->d_x, 4 * hx.size()) && !dev_alloc(c, &c->d_gdelta, wide_words) &&
+             !upload(c, &c->d_frp, hfrp) && !upload(c, &c->d_fcw, hfcw) && (!any_asym || !upload(c, &c->d_frw, hfrw)) &&
+             memory_left();
+        if (!ep) {
+            release_to(c, mark);
+            c->d_gdelta = nullptr;
+            c->d_frp = nullptr;
+            c->d_fcw = nullptr;
+            c->d_frw = nullptr;
+        }
+    }
+    if (!ep && (rc = dev_alloc(c, &c->d_x, 2 * hx.size()))) {
+        g_create_err = c->err;
+        plis_destroy(c);
+        return rc;
+    }
     if (hipMemcpy(c->d_x, hx.data(), hx.size() * sizeof(uint32_t), hipMemcpyHostToDevice) != hipSuccess) {
         g_create_err = "copying the counts failed";
         plis_destroy(c);
         return PLIS_ERR_HIP;
-    }
-    // the forward CSR serves the edge-parallel leap and the resident kernel,
-    // the zeroed balances the former
-    c->sourced = has_source(nh, I, D);
-    const ResLists lists = res_lists(nh, I);
-    c->resident_fits = resident_fit(c, nh, D, lists, hfrp, huge_tile);
-    if ((ep || c->resident_fits) && ((rc = upload(c, &c->d_frp, hfrp)) || (rc = upload(c, &c->d_fcw, hfcw)))) {
-        g_create_err = c->err;
-        plis_destroy(c);
-        return rc;
-    }
-    // (the tiles' flags behind the wide balances: one allocation, cleared together)
-    const size_t wide_words = hx.size() + ((size_t)c->ntiles + 1) / 2;
-    if (ep && ((rc = dev_alloc(c, &c->d_gdelta, wide_words)) || (any_asym && (rc = upload(c, &c->d_frw, hfrw))))) {
-        g_create_err = c->err;
-        plis_destroy(c);
-        return rc;
     }
     if (ep) c->d_wide = reinterpret_cast<uint32_t*>(c->d_gdelta + hx.size());
     if (ep && (hipMemsetAsync(c->d_gdelta, 0, wide_words * sizeof(unsigned long long), c->stream) != hipSuccess ||
@@ -927,6 +946,9 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
         plis_destroy(c);
         return PLIS_ERR_HIP;
     }
+    c->sourced = has_source(nh, I, D);
+    const ResLists lists = res_lists(nh, I);
+    c->resident_fits = resident_fit(c, nh, D, lists, hfrp, huge_tile);
     if (c->resident_fits) {
         // one block of device memory for its tables: seven small ones took 0.1 ms
         std::vector<uint4> host;
@@ -947,25 +969,28 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
                     host[fwd + e] = {(uint32_t)hfcw[e] & kFwdIdMask, (uint32_t)(hfcw[e] >> 32), v, back};
                 }
         uint4* dev = nullptr;
-        if ((rc = upload(c, &dev, host)) ||
-            (c->res.ws_slice && (rc = dev_alloc(c, &c->res.ws, c->res.ws_slice * c->nreal)))) {
-            g_create_err = c->err;
-            plis_destroy(c);
-            return rc;
+        const size_t mark = c->allocs.size();
+        if ((!ep && upload(c, &c->d_frp, hfrp)) || upload(c, &dev, host) ||
+            (c->res.ws_slice && dev_alloc(c, &c->res.ws, c->res.ws_slice * c->nreal))) {
+            release_to(c, mark);  // a launch per pass needs none of it
+            if (!ep) c->d_frp = nullptr;
+            c->res.ws = nullptr;
+            c->resident_fits = false;
+        } else {
+            // (one limit for every context: a smaller one set here would take it from another)
+            if (const hipError_t e = resident_reserve(kResidentLdsMax); e != hipSuccess) {
+                g_create_err = std::string("hipFuncSetAttribute(resident_kernel): ") + hipGetErrorString(e);
+                plis_destroy(c);
+                return PLIS_ERR_HIP;
+            }
+            c->res.rx = reinterpret_cast<const int4*>(dev + rx);
+            c->res.sp = reinterpret_cast<const int2*>(dev + sp);
+            c->res.spe = reinterpret_cast<const int2*>(dev + spe);
+            c->res.jp = reinterpret_cast<const int2*>(dev + jp);
+            c->res.jpe = reinterpret_cast<const int2*>(dev + jpe);
+            c->res.hm = reinterpret_cast<const int2*>(dev + hm);
+            c->res.fwd = dev + fwd;
         }
-        // (one limit for every context: a smaller one set here would take it from another)
-        if (const hipError_t e = resident_reserve(kResidentLdsMax); e != hipSuccess) {
-            g_create_err = std::string("hipFuncSetAttribute(resident_kernel): ") + hipGetErrorString(e);
-            plis_destroy(c);
-            return PLIS_ERR_HIP;
-        }
-        c->res.rx = reinterpret_cast<const int4*>(dev + rx);
-        c->res.sp = reinterpret_cast<const int2*>(dev + sp);
-        c->res.spe = reinterpret_cast<const int2*>(dev + spe);
-        c->res.jp = reinterpret_cast<const int2*>(dev + jp);
-        c->res.jpe = reinterpret_cast<const int2*>(dev + jpe);
-        c->res.hm = reinterpret_cast<const int2*>(dev + hm);
-        c->res.fwd = dev + fwd;
     }
     c->edge_parallel = ep;
     // 16 blocks of 4 waves per CU unless told otherwise: about one tile per
