@@ -1447,6 +1447,9 @@ extern "C" int plis_debug_poison(plis_ctx* c) {
             if (i != c->ctl_host[r].cur)
                 HIPCHK(c, hipMemsetD32Async(count_buf(c, i) + ri.x_off, (int)kPoisonCount, (size_t)c->S * ri.N, c->stream));
     }
+    // the one-block kernel's arrays outside LDS (propensities 1.0000002, balances of 2^62)
+    if (c->res.ws)
+        HIPCHK(c, hipMemsetD32Async(c->res.ws, 0x3FF00000, c->res.ws_slice / 4 * c->nreal, c->stream));
     hipLaunchKernelGGL(poison_parts_kernel, dim3(std::min<uint32_t>((c->ntiles + 255) / 256, 1024u)), dim3(256), 0,
                        c->stream, c->d_pa_t, c->d_pb_t, c->ntiles, c->d_pa_c, c->d_pb_c,
                        c->nreal * kDecideChunks);
