@@ -142,7 +142,7 @@ def gpu_measure(wl, steps, warmup, seed=2024, autotune=True, shape=None):
             "leapbacks": lbs, "crit_events": crit, "subvolume_simtime": simt, "shape": shape, "tuned": (wpb, bpc),
             "tau_ms": prof[1] / n_prof, "decide_ms": prof[2] / n_prof, "leap_ms": prof[3] / n_prof,
             "commit_ms": prof[4] / n_prof, "iter_ms_events": prof[0] / n_prof,
-            "leap_kernel_ms": prof[5] / n_prof, "redo_ms": prof[6] / n_prof, "finish_ms": prof[7] / n_prof}
+            "leap_kernel_ms": prof[5] / n_prof, "finish_ms": prof[7] / n_prof}
 
 
 def learned_measure(wl, steps, warmup, train_steps, batch, seed=2024, kappa=1.0, snapshots=16,
@@ -212,7 +212,7 @@ def learned_measure(wl, steps, warmup, train_steps, batch, seed=2024, kappa=1.0,
                                      zip(s0, s1, [int(t["N"]) for t in wl["topos"]])),
             "activation": "gelu" if act == 1 else "relu",
             "tau_ms": prof[1] / n_prof, "decide_ms": prof[2] / n_prof, "leap_ms": prof[3] / n_prof,
-            "commit_ms": prof[4] / n_prof, "leap_kernel_ms": prof[5] / n_prof, "redo_ms": prof[6] / n_prof,
+            "commit_ms": prof[4] / n_prof, "leap_kernel_ms": prof[5] / n_prof,
             "finish_with_proposals_ms": prof[7] / n_prof, "iteration_ms_events": prof[0] / n_prof,
             "records_seconds": t_rec, "train_seconds": t_train,
             "viol_rate_max": vmax, "kappa": kappa, **info}

@@ -1,7 +1,7 @@
 // plis_capi.hip -- host side of libplis_hip.so: the C ABI declared in
 // include/plis.h.  Builds the canonical device layout of a batch of
-// realizations, launches the two step kernels (optionally replayed as a
-// hipGraph), and keeps every control decision on the device: the host only
+// realizations, launches the kernels of a step (optionally replayed as a
+// hipGraph) or, for small realizations, one kernel that makes many, and keeps every control decision on the device: the host only
 // polls a done-counter once per batch of iterations (the reference makes at
 // least seven blocking host<->device transactions per step,
 // PLISCuda/src/driver.cu:259-376).

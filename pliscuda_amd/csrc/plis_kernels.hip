@@ -1440,7 +1440,7 @@ __device__ __forceinline__ bool leap_tile_draws(const KernelArgs& a, const NetVi
 #pragma unroll
                             for (int dir = 0; dir < 2; ++dir) {
                                 const int w = 2 * s + dir;
-                                // (within 8 2^-24 of the double mean, like hop_mean_f)
+                                // (within 9 2^-24 of the double mean, one rounding more than hop_mean_f)
                                 const float lf = (rate[w] * (dir ? w1 : w0)) * (1.0f / kCoarseScale);
                                 if (!(open[w] && lf < kInlineMaxF)) continue;
                                 const uint32_t word = draw_word(coarse_byte(o, (uint32_t)w), f, (uint32_t)w);

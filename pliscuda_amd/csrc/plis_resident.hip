@@ -1,7 +1,8 @@
 // plis_resident.hip -- all steps of a small realization inside one block.
 //
 // Stepping a small realization with one launch per pass is bound by launches:
-// an empty kernel of the captured step takes 4.4 us, the whole step of a
+// a kernel of the captured step that finds nothing to do takes 4.4 us with what
+// its boundary flushes (1.65 in a graph of empty kernels), the whole step of a
 // 64-subvolume box 26-29 us whatever its size.  resident_kernel gives each
 // realization one block that makes up to `iters` iterations: counts,
 // balances and propensities stay in LDS (in a global workspace for networks

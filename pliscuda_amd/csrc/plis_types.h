@@ -46,7 +46,7 @@ struct RealInfo {
     uint64_t rp_off;     // out row_ptr base (N+1 entries)
     uint64_t irp_off;    // in row_ptr base
     uint64_t comp_off;   // compartment ids base (if C > 1)
-    uint64_t fe_off;     // forward-CSR edge base (entries v -> u with u > v; symmetric only)
+    uint64_t fe_off;     // forward-CSR edge base (entries v -> u with u > v)
     uint32_t N, id;
     uint32_t tile_begin, ntiles;
     uint32_t flags;      // bit0: symmetric (in-CSR aliases out-CSR), bit1: weighted
