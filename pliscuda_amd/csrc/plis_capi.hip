@@ -171,10 +171,11 @@ static void release_to(plis_ctx* c, size_t mark) {
 }
 
 // Whether the device has 1 GiB left, for kernels' scratch memory, training or
-// another context.
-static bool memory_left() {
+// another context, once `taken` bytes are; a context that takes a small part of
+// what is left does not give up its way of stepping for it.
+static bool memory_left(uint64_t taken) {
     size_t left = 0, all = 0;
-    return hipMemGetInfo(&left, &all) == hipSuccess && left >= 1ull << 30;
+    return hipMemGetInfo(&left, &all) == hipSuccess && left >= std::min<uint64_t>(1ull << 30, 64 * taken);
 }
 
 static int fail_create(const std::string& m) {
@@ -918,9 +919,10 @@ extern "C" int plis_create(const plis_network* net, int32_t n_real, const plis_t
     const size_t wide_words = hx.size() + ((size_t)c->ntiles + 1) / 2;
     if (ep) {
         const size_t mark = c->allocs.size();
+        const uint64_t taken = 16 * hx.size() + 8 * (wide_words + hfcw.size()) + 4 * (hfrp.size() + hfrw.size());
         ep = !dev_alloc(c, &c->d_x, 4 * hx.size()) && !dev_alloc(c, &c->d_gdelta, wide_words) &&
              !upload(c, &c->d_frp, hfrp) && !upload(c, &c->d_fcw, hfcw) && (!any_asym || !upload(c, &c->d_frw, hfrw)) &&
-             memory_left();
+             memory_left(taken);
         if (!ep) {
             release_to(c, mark);
             c->d_gdelta = nullptr;
