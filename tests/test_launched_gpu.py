@@ -188,9 +188,9 @@ def test_a_judged_context_completes_its_leap_in_a_kernel_of_its_own(kind):
         ctx.set_tau_mode(False, theta=theta)
         ctx.arm()
         ctx.profile_kernels(2)
-        p = ctx.profile_kernels(10)
-        assert p[5] > 0.0 and p[6] == 0.0
-        ms.append(p[7])
+        ps = [ctx.profile_kernels(5) for _ in range(6)]  # (the least of several: a host that was held up adds to a gap)
+        assert all(p[5] > 0.0 and p[6] == 0.0 for p in ps)
+        ms.append(min(p[7] for p in ps))
         _matches(ctx, net, topo, x0, 0.03, 10, 9)
         ctx.close()
     assert ms[1] > ms[0] >= 0.0
